@@ -24,21 +24,32 @@
 //                             slots, and fp32 acc only for the lead rows (the first `lead` tokens
 //                             of each row, which the exact lead-attention pass reads).
 //
-// Block: a 256 x 256 output tile (activation rows x weight rows) on 8 waves, each owning 32 MFMA
-// tiles (128 fp32 accumulators per lane): 64 rows x 128 weight rows in a 4 x 2 wave grid for the
-// split forms, 32 rows x 256 weight rows (8 x 1) for A_NORM.  K advances 32 at a time through a
-// ring of three LDS stages of 48 KB.  A stage holds 16 weight fragments and 32 activation
-// fragments of 1 KB in MFMA lane order (bf16 {hi, lo} of 16 row blocks; for A_NORM the fp32 x of
-// 16 row blocks in the fp32 tile layout, split after the read), so every fragment read is one
+// Block: a 128 x 256 output tile (activation rows x weight rows) on 4 waves, each owning 32 MFMA
+// tiles (128 fp32 accumulators per lane): 64 rows x 128 weight rows in a 2 x 2 wave grid for the
+// split forms, 32 rows x 256 weight rows (4 x 1) for A_NORM.  K advances 32 at a time through a
+// ring of two LDS stages of 32 KB.  A stage holds 16 weight fragments and 16 activation
+// fragments of 1 KB in MFMA lane order (bf16 {hi, lo} of 8 row blocks; for A_NORM the fp32 x of
+// 8 row blocks in the fp32 tile layout, split after the read), so every fragment read is one
 // conflict-free 16-byte LDS read per lane.  Global data goes straight to LDS
-// (global_load_lds_dwordx4, 16 bytes per lane, one kilobyte per wave instruction), issued two
-// k-steps ahead; nothing is staged in registers, and a step ends with one barrier after an exact
-// vmcnt wait for the next stage's loads.  Blocks are persistent (one per CU, each walking its
-// tiles), and the load ring runs on across tile boundaries, so a tile's epilogue overlaps the
-// next tile's first loads. Every weight fragment feeds two MFMAs (hi and lo rows), as in K5.
-// Blocks are numbered so that an XCD (block i runs on XCD i mod 8) takes a contiguous run of
-// tiles, row tile major: the N tiles of one row tile share its activation rows in one L2.
-// Summation order is fixed (k-steps in order, hi before lo), so results are reproducible.
+// (global_load_lds_dwordx4, 16 bytes per lane, one kilobyte per wave instruction), issued one
+// k-step ahead; nothing is staged in registers, and a step ends with one barrier after an exact
+// vmcnt wait for the next stage's loads.
+//
+// Two such blocks share a CU.  What bounds a block is the alternation inside a k-step: behind the
+// barrier every wave first reads its 16-20 KB of fragments from LDS, then issues its 64 MFMAs,
+// and a finished tile's epilogue issues none.  With two blocks at barriers of their own, one's
+// LDS reads and epilogues run under the other's MFMAs.  Against one block of 256 x 256 on 8 waves
+// with a ring of three (the same fragment reads per MFMA, a quarter fewer copies), us per launch
+// at d = 768, F = 2048 (qkv / out / gate-up / down): 2,059 / 712 / 3,351 / 1,507 -> 1,981 / 667 /
+// 3,244 / 1,375 at 282,695 rows (1,293 TFLOP/s executed by the last), 157 / 50 / 227 / 103 -> 136
+// / 43 / 195 / 86 at 16,669 rows, where the smaller tiles also fill the last round better.
+//
+// Blocks are persistent (two per CU, each walking its tiles), and the load ring runs on across
+// tile boundaries, so a tile's epilogue overlaps the next tile's first loads.  Every weight
+// fragment feeds two MFMAs (hi and lo rows), as in K5.  Blocks are numbered so that an XCD (block
+// i runs on XCD i mod 8) takes a contiguous run of tiles, row tile major: the N tiles of one row
+// tile share its activation rows in one L2.  Summation order is fixed (k-steps in order, hi
+// before lo), so results are reproducible and do not depend on the block shape.
 #include <algorithm>
 
 #include "common.h"
@@ -50,16 +61,13 @@ namespace mdl {
 
 namespace {
 
-constexpr int kBM = 256, kBN = 256;
-constexpr int kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kAFrags = (kBM / 16) * 2;   // {hi, lo} fragments of 16 row blocks
-constexpr int kWFrags = kBN / 16;
-constexpr int kStage = (kAFrags + kWFrags) * 1024;   // bytes of one LDS stage
-constexpr int kRing = 3;                             // LDS stages (loads run 2 k-steps ahead)
-// DMA instructions per thread per stage: two weight fragments and four activation fragments
-// (two for the split forms with the hi part alone)
-template <int AMODE, int AP>
-constexpr int loads_per_stage() { return AMODE != 2 && AP == 1 ? 4 : 6; }
+// A block shape: a BM x BN output tile on WMW x WNW waves, K through a ring of RING LDS stages of
+// KS k-steps (of 32) each; the blocks that fit a CU's LDS and registers together are OCC.
+template <int BM_, int BN_, int WMW_, int WNW_, int KS_, int RING_, int OCC_>
+struct Shape {
+  static constexpr int BM = BM_, BN = BN_, WMW = WMW_, WNW = WNW_, KS = KS_, RING = RING_;
+  static constexpr int OCC = OCC_, NW = WMW_ * WNW_;
+};
 constexpr int kMaxNormK = 2048;                      // A_NORM: gamma lives in LDS
 
 enum AMode { A_ROWS = 0, A_TILES = 1, A_NORM = 2 };
@@ -72,6 +80,7 @@ struct Args {
   const float* gamma;
   float eps;
   const uint16_t* w;   // tiled [N, K]
+  const uint16_t* wl;  // WL forms: low bf16 part of an fp32 weight, tiled like w
   float* out;          // E_STORE
   int64_t ldo;
   float* rstd_out;     // E_STORE with A_NORM (may be NULL)
@@ -106,10 +115,24 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
-template <int AMODE, int EPI, int AP>
-__global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p) {
+template <int AMODE, int EPI, int AP, bool WL, class S>
+__global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_kernel(
+    const Args p) {
   static_assert(AP == 1 || AP == 2, "activation parts: hi, or hi and lo");
-  constexpr int kLoads = loads_per_stage<AMODE, AP>();
+  static_assert(!WL || AP == 2, "the low weight part goes with split activations");
+  constexpr int kBM = S::BM, kBN = S::BN, kWaves = S::NW, kThreads = 64 * S::NW;
+  constexpr int KS = S::KS, kRing = S::RING;
+  // fragments of 1 KB in one k-step of a stage: {hi, lo} (A_NORM: the two kilobytes of fp32) of
+  // each row block, then the weight row blocks, then (WL) their low parts
+  constexpr int kAFrags = (kBM / 16) * 2, kWFrags = kBN / 16 * (WL ? 2 : 1);
+  constexpr int kStep = (kAFrags + kWFrags) * 1024, kStage = KS * kStep;
+  // copies per wave and stage; the split forms with the hi part alone make half the activation's
+  constexpr bool kHiOnly = AMODE != A_NORM && AP == 1;
+  constexpr int kACopies = KS * kAFrags / (kHiOnly ? 2 : 1) / kWaves;
+  constexpr int kWCopies = KS * kWFrags / kWaves;
+  constexpr int kLoads = kACopies + kWCopies;
+  static_assert(kACopies * kWaves * (kHiOnly ? 2 : 1) == KS * kAFrags &&
+                kWCopies * kWaves == KS * kWFrags, "every wave makes the same copies");
   constexpr int kGammaBytes = AMODE == A_NORM ? kMaxNormK * 4 : 0;
   __shared__ __align__(16) uint8_t lds[kRing * kStage + kGammaBytes];
   __shared__ float rstd_s[kBM];
@@ -122,52 +145,58 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
   const int first = t_lo + (blockIdx.x >> 3);
   if (first >= t_hi) return;   // whole block, before any barrier
   const int M = p.M, N = p.N, K = p.K, nk = K >> 5;
-  const int total = (t_hi - first + bpx - 1) / bpx * nk;   // k-steps over this block's tiles
+  const int ns = (nk + KS - 1) / KS;                       // stages per tile
+  const int total = (t_hi - first + bpx - 1) / bpx * ns;   // stages over this block's tiles
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // wave grid WMW x WNW over the tile: wave (wm, wn) owns FM row blocks and FN weight fragments.
   // The A_NORM forms split x * gamma in registers after the LDS read, so there every row block
-  // belongs to one wave (8 x 1) and is converted once; the split forms use 4 x 2 (8 activation
+  // belongs to one wave (4 x 1) and is converted once; the split forms use 2 x 2 (8 activation
   // and 8 weight fragment reads per wave and k-step).
-  constexpr int WMW = AMODE == A_NORM ? 8 : 4, WNW = kWaves / WMW;
+  constexpr int WMW = S::WMW, WNW = S::WNW;
   constexpr int FM = kBM / 16 / WMW, FN = kBN / 16 / WNW;
   const int wm = wave % WMW, wn = wave / WMW;
   const int c = lane & 15, g = lane >> 4;
   const int last_nb = (N + 15) / 16 - 1, last_mb = (M + 15) / 16 - 1;
   const uint32_t lds0 = lds_addr(lds);
 
-  // The loads of k-step s of the tile at (m0, n0) into ring stage b.  Wave w copies weight
-  // fragments 8 j + w (j = 0, 1: row block n0 / 16 + 8 j + w) and activation fragments f = 8 j +
-  // w (j = 0..3): row block f / 2, part f % 2 (hi / lo; for A_NORM the first or second kilobyte of
-  // the fp32 16 x 32 block, lane l's columns 0..3 or 4..7); with the hi part alone (AP 1, split
-  // forms) f = 2 (8 j + w), j = 0, 1.  Fragment f lands in stage slot f either way.  Every copy is
-  // one contiguous kilobyte per wave, except row-major A.  Row blocks past M or N load valid
-  // memory (clamped to the last; tile-layout buffers hold its padding rows); their results are
-  // never stored.
+  // The loads of stage s (k-steps KS s ..) of the tile at (m0, n0) into ring stage b: the waves
+  // take the stage's fragments in turn.  Weight fragment f is row block n0 / 16 + f (WL: f / 2,
+  // part f % 2, hi / lo); activation fragment f is row block f / 2, part f % 2 (hi / lo; for
+  // A_NORM the first or second kilobyte of the fp32 16 x 32 block, lane l's columns 0..3 or
+  // 4..7); with the hi part alone (AP 1, split forms) only the even f exist.  Fragment f lands
+  // in slot f of its k-step either way.  Every copy is one contiguous kilobyte per wave, except
+  // row-major A.  Row blocks past M or N and k-steps past K load valid memory (clamped to the
+  // last; tile-layout buffers hold its padding rows); their results are never used.
   auto issue = [&](int m0, int n0, int s, int b) {
     const uint32_t base = lds0 + b * kStage;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int nb = min(n0 / 16 + 8 * j + wave, last_nb);
-      dma16(p.w + (static_cast<int64_t>(nb) * nk + s) * 512 + 8 * lane,
-            __builtin_amdgcn_readfirstlane(base + (kAFrags + 8 * j + wave) * 1024));
+    for (int j = 0; j < kWCopies; ++j) {
+      const int f = kWaves * j + wave, ks = f / kWFrags, fw = f - ks * kWFrags;
+      const int nb = min(n0 / 16 + (WL ? fw >> 1 : fw), last_nb);
+      const uint16_t* src = WL && (fw & 1) ? p.wl : p.w;
+      const int st = min(KS * s + ks, nk - 1);
+      dma16(src + (static_cast<int64_t>(nb) * nk + st) * 512 + 8 * lane,
+            __builtin_amdgcn_readfirstlane(base + ks * kStep + (kAFrags + fw) * 1024));
     }
-    constexpr bool kHiOnly = AMODE != A_NORM && AP == 1;
 #pragma unroll
-    for (int j = 0; j < (kHiOnly ? 2 : 4); ++j) {
-      const int f = kHiOnly ? 2 * (8 * j + wave) : 8 * j + wave, rb = f >> 1, part = f & 1;
+    for (int j = 0; j < kACopies; ++j) {
+      constexpr int kPer = kHiOnly ? kAFrags / 2 : kAFrags;
+      const int fa = kWaves * j + wave, ks = fa / kPer;
+      const int f = (kHiOnly ? 2 : 1) * (fa - ks * kPer), rb = f >> 1, part = f & 1;
+      const int st = min(KS * s + ks, nk - 1);
       const void* src;
       if constexpr (AMODE == A_NORM) {
-        const int64_t blk = static_cast<int64_t>(min(m0 / 16 + rb, last_mb)) * nk + s;
+        const int64_t blk = static_cast<int64_t>(min(m0 / 16 + rb, last_mb)) * nk + st;
         src = p.x + blk * 512 + 256 * part + 4 * lane;
       } else if constexpr (AMODE == A_TILES) {
         const int64_t blk = static_cast<int64_t>(min(m0 / 16 + rb, last_mb)) * AP * nk;
-        src = p.a + (blk + part * nk + s) * 512 + 8 * lane;
+        src = p.a + (blk + part * nk + st) * 512 + 8 * lane;
       } else {
         const int row = min(m0 + 16 * rb + c, M - 1);
-        src = p.a + static_cast<int64_t>(row) * p.lda + part * K + 32 * s + 8 * g;
+        src = p.a + static_cast<int64_t>(row) * p.lda + part * K + 32 * st + 8 * g;
       }
-      dma16(src, __builtin_amdgcn_readfirstlane(base + f * 1024));
+      dma16(src, __builtin_amdgcn_readfirstlane(base + ks * kStep + f * 1024));
     }
   };
 
@@ -189,8 +218,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
     for (int j = 0; j < FM; ++j) ss[j] = 0.f;
   };
 
-  auto compute = [&](int s, int b) {
-    const uint8_t* base = lds + b * kStage;
+  auto compute = [&](int s, const uint8_t* base) {
     bf16x8_t ah[FM], al[FM];
     if constexpr (AMODE == A_NORM) {
       // x of row 16 (FM wm + j) + c, columns 8 g .. 8 g + 7: the split of x * gamma, as the
@@ -238,16 +266,24 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
     // hi product (measured at config 2 against one fragment at a time: qkv 7%, gate/up 6%
     // faster; two at a time sits between; eight is within 1% of four and takes the E_QKV form
     // to the 256-register limit).
+    constexpr int kWPer = WL ? 2 : 1;   // fragments per weight row block
     if constexpr (AMODE == A_NORM) {
-      constexpr int kGroup = 4;
+      constexpr int kGroup = FN < 4 ? FN : 4;
       static_assert(FN % kGroup == 0, "the norm forms group their weight fragments");
 #pragma unroll
       for (int i = 0; i < FN; i += kGroup) {
         bf16x8_t wf[kGroup];
 #pragma unroll
         for (int u = 0; u < kGroup; ++u)
-          wf[u] = *reinterpret_cast<const bf16x8_t*>(base + (kAFrags + FN * wn + i + u) * 1024 +
-                                                     16 * lane);
+          wf[u] = *reinterpret_cast<const bf16x8_t*>(
+              base + (kAFrags + kWPer * (FN * wn + i + u)) * 1024 + 16 * lane);
+        bf16x8_t wlf[WL ? kGroup : 1];
+        if constexpr (WL) {
+#pragma unroll
+          for (int u = 0; u < kGroup; ++u)
+            wlf[u] = *reinterpret_cast<const bf16x8_t*>(
+                base + (kAFrags + 2 * (FN * wn + i + u) + 1) * 1024 + 16 * lane);
+        }
 #pragma unroll
         for (int u = 0; u < kGroup; ++u)
 #pragma unroll
@@ -262,13 +298,28 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
               acc[i + u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], al[j],
                                                                       acc[i + u][j], 0, 0, 0);
         }
+        if constexpr (WL) {
+#pragma unroll
+          for (int u = 0; u < kGroup; ++u)
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+              acc[i + u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlf[u], ah[j],
+                                                                      acc[i + u][j], 0, 0, 0);
+        }
       }
     } else {
       bf16x8_t wf[FN];
 #pragma unroll
       for (int i = 0; i < FN; ++i)
-        wf[i] = *reinterpret_cast<const bf16x8_t*>(base + (kAFrags + FN * wn + i) * 1024 +
-                                                   16 * lane);
+        wf[i] = *reinterpret_cast<const bf16x8_t*>(
+            base + (kAFrags + kWPer * (FN * wn + i)) * 1024 + 16 * lane);
+      bf16x8_t wlf[WL ? FN : 1];
+      if constexpr (WL) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+          wlf[i] = *reinterpret_cast<const bf16x8_t*>(
+              base + (kAFrags + 2 * (FN * wn + i) + 1) * 1024 + 16 * lane);
+      }
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
@@ -280,6 +331,14 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
 #pragma unroll
           for (int j = 0; j < FM; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], al[j], acc[i][j], 0, 0, 0);
+      }
+      if constexpr (WL) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+          for (int j = 0; j < FM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlf[i], ah[j], acc[i][j], 0, 0,
+                                                                0);
       }
     }
   };
@@ -301,6 +360,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       if constexpr (EPI == E_STORE || EPI == E_QKV) {
         if (p.rstd_out && n0 == 0 && tid < kBM && m0 + tid < M) p.rstd_out[m0 + tid] = rstd_s[tid];
+        static_assert(kBM <= kThreads, "one thread per row of the tile");
       }
     }
     if constexpr (EPI == E_QKV) {
@@ -378,7 +438,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
       // operation (the stores before it, the next tile's copies), so loads issued one pair at a
       // time after the previous pair's stores took a full round trip per pair.
       const int F = p.d_ff;
-      constexpr int kG = 2, NP = FN / 2;
+      constexpr int NP = FN / 2, kG = NP % 4 == 0 ? 2 : 1;
       static_assert(NP % (2 * kG) == 0, "bias groups");
       auto chan = [&](int pb) { return 16 * (n0 / 32 + NP * wn + pb) + 4 * g; };
       auto load_bias = [&](int pb0, float4 (&bg)[kG], float4 (&bu)[kG]) {
@@ -428,7 +488,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
       // The residual's loads of kG weight fragments are issued together, and those of the next
       // kG before this group's stores (see E_SWIGLU: one load and its wait per fragment, after
       // the previous fragment's store, took a full round trip each).
-      constexpr int kG = 2;
+      constexpr int kG = FN % 4 == 0 ? 2 : 1;
       static_assert(FN % (2 * kG) == 0, "residual groups");
       auto col = [&](int i) { return n0 + 16 * (FN * wn + i) + 4 * g; };
       auto row = [&](int j) { return m0 + 16 * (FM * wm + j) + c; };
@@ -483,49 +543,51 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm_kernel(const Args p)
     }
   };
 
-  // Step u (over all k-steps of this block's tiles, tile after tile) computes ring stage u % 3
-  // while steps u + 1 and u + 2 load -- across a tile boundary too, so the next tile's first
-  // stages are in flight during this tile's epilogue.  The stage step u overwrites,
-  // (u + 2) % 3, was last read in step u - 1, before that step's barrier.  Every wave runs the
-  // same steps (all counters are block-uniform), so every barrier is reached by all.
+  // Step u (over all stages of this block's tiles, tile after tile) computes ring stage
+  // u % kRing while the next kRing - 1 stages load -- across a tile boundary too, so the next
+  // tile's first stages are in flight during this tile's epilogue.  The stage that step u's
+  // copies overwrite, (u + kAhead) % kRing, was last read in step u - 1, before that step's
+  // barrier.  Every wave runs the same steps (all counters are block-uniform), so every barrier
+  // is reached by all.
   auto tile_origin = [&](int t, int& m0, int& n0) {
     const int mt = t / p.tiles_n;
     m0 = mt * kBM;
     n0 = (t - mt * p.tiles_n) * kBN;
   };
-  int it = first, is = 0, im0, in0;   // issue cursor: tile, k-step, tile origin
+  int it = first, is = 0, im0, in0;   // issue cursor: tile, stage of the tile, tile origin
   tile_origin(it, im0, in0);
   auto advance_issue = [&]() {
-    if (++is == nk) {
+    if (++is == ns) {
       is = 0;
       it += bpx;
       tile_origin(it, im0, in0);
     }
   };
-  issue(im0, in0, is, 0);
-  advance_issue();
-  if (total > 1) {
-    issue(im0, in0, is, 1);
-    advance_issue();
-    stage_barrier<kLoads>();
-  } else {
-    stage_barrier<0>();
-  }
+  constexpr int kAhead = kRing - 1;   // stages in flight beyond the one being computed
+#pragma unroll
+  for (int r = 0; r < kAhead; ++r)
+    if (r < total) {
+      issue(im0, in0, is, r);
+      advance_issue();
+    }
+  if (total >= kAhead) stage_barrier<(kAhead - 1) * kLoads>();
+  else stage_barrier<0>();
   int ct = first, cs = 0, cm0, cn0;   // compute cursor
   tile_origin(ct, cm0, cn0);
   reset();
   int b = 0;
   for (int u = 0; u < total; ++u) {
-    const int b2 = b == 0 ? 2 : b - 1;   // (u + 2) % 3
-    if (u + 2 < total) {
-      issue(im0, in0, is, b2);
+    if (u + kAhead < total) {
+      issue(im0, in0, is, b == 0 ? kRing - 1 : b - 1);   // stage (u + kAhead) % kRing
       advance_issue();
     }
-    compute(cs, b);
-    if (u + 2 < total) stage_barrier<kLoads>();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      if (KS == 1 || KS * cs + ks < nk) compute(KS * cs + ks, lds + b * kStage + ks * kStep);
+    if (u + kAhead < total) stage_barrier<(kAhead - 1) * kLoads>();
     else stage_barrier<0>();
-    b = b == 2 ? 0 : b + 1;
-    if (++cs == nk) {
+    b = b == kRing - 1 ? 0 : b + 1;
+    if (++cs == ns) {
       epilogue(cm0, cn0);
       reset();
       cs = 0;
@@ -550,21 +612,30 @@ int device_cus() {
   return cached[dev];
 }
 
-template <int AMODE, int EPI, int AP = 2>
-int launch(Args p, hipStream_t st) {
-  const int64_t tm = (static_cast<int64_t>(p.M) + kBM - 1) / kBM;
-  const int64_t tn = (static_cast<int64_t>(p.N) + kBN - 1) / kBN;
+template <int AMODE, int EPI, int AP, bool WL, class S>
+int launch_shape(Args p, hipStream_t st) {
+  const int64_t tm = (static_cast<int64_t>(p.M) + S::BM - 1) / S::BM;
+  const int64_t tn = (static_cast<int64_t>(p.N) + S::BN - 1) / S::BN;
   const int64_t tiles = tm * tn;
   if (tiles > 0x7fffffff - 8) return MDL_ERR_SHAPE;
   const int64_t per_xcd = (tiles + 7) / 8;
-  // one block per CU (the LDS ring allows no second); blocks per XCD capped by its tiles
-  const int64_t bpx = std::min<int64_t>((device_cus() + 7) / 8, per_xcd);
+  // the blocks that fit the chip at a time; blocks per XCD capped by its tiles
+  const int64_t bpx = std::min<int64_t>(S::OCC * ((device_cus() + 7) / 8), per_xcd);
   p.tiles_n = static_cast<int>(tn);
   p.tiles = static_cast<int>(tiles);
   p.per_xcd = static_cast<int>(per_xcd);
-  prefill_gemm_kernel<AMODE, EPI, AP>
-      <<<dim3(static_cast<unsigned>(8 * bpx)), kThreads, 0, st>>>(p);
+  prefill_gemm_kernel<AMODE, EPI, AP, WL, S>
+      <<<dim3(static_cast<unsigned>(8 * bpx)), 64 * S::NW, 0, st>>>(p);
   return launch_status();
+}
+
+using NormTile = Shape<128, 256, 4, 1, 1, 2, 2>;
+using SplitTile = Shape<128, 256, 2, 2, 1, 2, 2>;
+
+template <int AMODE, int EPI, int AP = 2>
+int launch(Args p, hipStream_t st) {
+  if constexpr (AMODE == A_NORM) return launch_shape<AMODE, EPI, AP, false, NormTile>(p, st);
+  else return launch_shape<AMODE, EPI, AP, false, SplitTile>(p, st);
 }
 
 // shared argument checks: k a positive multiple of 32, n of 16, 16-byte aligned operands

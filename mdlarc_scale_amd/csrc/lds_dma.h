@@ -47,4 +47,13 @@ __device__ __forceinline__ void dma16_sbase(const void* base, uint32_t off, uint
                :: "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
+// dma16_sbase without the memory clobber: the compiler may move its own memory accesses across
+// the copy.  For a kernel that spreads its copies over the work on the stage before: the copy's
+// stage is neither read nor written by the kernel between its two barriers (asm volatile with the
+// clobber, which volatile assembly is not moved across).
+__device__ __forceinline__ void dma16_free(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(lds));
+}
+
 }  // namespace mdl

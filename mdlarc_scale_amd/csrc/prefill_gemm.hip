@@ -24,32 +24,39 @@
 //                             slots, and fp32 acc only for the lead rows (the first `lead` tokens
 //                             of each row, which the exact lead-attention pass reads).
 //
-// Block: a 128 x 256 output tile (activation rows x weight rows) on 4 waves, each owning 32 MFMA
-// tiles (128 fp32 accumulators per lane): 64 rows x 128 weight rows in a 2 x 2 wave grid for the
-// split forms, 32 rows x 256 weight rows (4 x 1) for A_NORM.  K advances 32 at a time through a
-// ring of two LDS stages of 32 KB.  A stage holds 16 weight fragments and 16 activation
+// Block: a tile of activation rows x weight rows (see Shape), e.g. 128 x 256 on 4 waves, each
+// owning 32 MFMA tiles (128 fp32 accumulators per lane): 64 rows x 128 weight rows in a 2 x 2 wave
+// grid for the split forms, 32 rows x 256 weight rows (4 x 1) for A_NORM.  K advances through a
+// ring of LDS stages; a k-step of 32 of this tile is 32 KB: 16 weight fragments and 16 activation
 // fragments of 1 KB in MFMA lane order (bf16 {hi, lo} of 8 row blocks; for A_NORM the fp32 x of
 // 8 row blocks in the fp32 tile layout, split after the read), so every fragment read is one
 // conflict-free 16-byte LDS read per lane.  Global data goes straight to LDS
-// (global_load_lds_dwordx4, 16 bytes per lane, one kilobyte per wave instruction), issued one
-// k-step ahead; nothing is staged in registers, and a step ends with one barrier after an exact
+// (global_load_lds_dwordx4, 16 bytes per lane, one kilobyte per wave instruction), issued RING - 1
+// stages ahead; nothing is staged in registers, and a stage ends with one barrier after an exact
 // vmcnt wait for the next stage's loads.
 //
-// Two such blocks share a CU.  What bounds a block is the alternation inside a k-step: behind the
-// barrier every wave first reads its 16-20 KB of fragments from LDS, then issues its 64 MFMAs,
-// and a finished tile's epilogue issues none.  With two blocks at barriers of their own, one's
-// LDS reads and epilogues run under the other's MFMAs.  Against one block of 256 x 256 on 8 waves
-// with a ring of three (the same fragment reads per MFMA, a quarter fewer copies), us per launch
-// at d = 768, F = 2048 (qkv / out / gate-up / down): 2,059 / 712 / 3,351 / 1,507 -> 1,981 / 667 /
-// 3,244 / 1,375 at 282,695 rows (1,293 TFLOP/s executed by the last), 157 / 50 / 227 / 103 -> 136
-// / 43 / 195 / 86 at 16,669 rows, where the smaller tiles also fill the last round better.
+// What bounds it.  A CU takes in one such copy every 25-32 cycles, and a wave issues in order: the
+// copies of a stage handed out in one go, each with a chain of address arithmetic before it, held
+// back the MFMAs behind them until all were accepted, and a block took the sum of its copy time
+// and its MFMA time (down projection at 731 rows of d = 768, F = 2048, 64 x 64 tiles, us: 25 whole,
+// 12 without the MFMAs, 9 without the copies).  So each copy has a scalar pointer that it moves
+// on by itself, and the shapes that run one or two tiles per CU spread a stage's copies over its
+// MFMAs (17 in that test, 13 with four k-steps a stage).
+// At prompt sizes the chip's power is the limit: 282,695 rows' down projection keeps its MFMAs
+// busy 78% of the cycles, at 1.4 GHz.  There two blocks of 128 x 256 per CU, their copies ahead of
+// the MFMAs at an even pace, take the least time: one block's LDS reads and epilogues run under
+// the other's MFMAs.  Against one block of 256 x 256 on 8 waves (the same fragment reads per MFMA,
+// a quarter fewer copies), us per launch (qkv / out / gate-up / down): 2,059 / 712 / 3,351 / 1,507
+// -> 1,974 / 666 / 3,240 / 1,375 at 282,695 rows, 157 / 50 / 227 / 103 -> 132 / 43 / 195 / 86 at
+// 16,669.
 //
-// Blocks are persistent (two per CU, each walking its tiles), and the load ring runs on across
-// tile boundaries, so a tile's epilogue overlaps the next tile's first loads.  Every weight
+// Blocks are persistent (each walking its tiles), and the load ring runs on across tile
+// boundaries, so a tile's epilogue overlaps the next tile's first loads.  Every weight
 // fragment feeds two MFMAs (hi and lo rows), as in K5.  Blocks are numbered so that an XCD (block
 // i runs on XCD i mod 8) takes a contiguous run of tiles, row tile major: the N tiles of one row
 // tile share its activation rows in one L2.  Summation order is fixed (k-steps in order, hi
-// before lo), so results are reproducible and do not depend on the block shape.
+// before lo), so results are reproducible, and it is the same in every shape: a row's results do
+// not depend on how many rows run beside it.
 #include <algorithm>
 
 #include "common.h"
@@ -62,13 +69,17 @@ namespace mdl {
 namespace {
 
 // A block shape: a BM x BN output tile on WMW x WNW waves, K through a ring of RING LDS stages of
-// KS k-steps (of 32) each; the blocks that fit a CU's LDS and registers together are OCC.
-template <int BM_, int BN_, int WMW_, int WNW_, int KS_, int RING_, int OCC_>
+// KS k-steps (of 32) each (K a multiple of 32 KS); the blocks that fit a CU's LDS and registers
+// together are OCC.  SPREAD: the copies of a stage go out between the MFMAs of a step, otherwise
+// ahead of them.  GK: the largest K of the norm forms (gamma lives in LDS).
+template <int BM_, int BN_, int WMW_, int WNW_, int KS_, int RING_, int OCC_, bool SPREAD_,
+          int GK_ = 2048>
 struct Shape {
   static constexpr int BM = BM_, BN = BN_, WMW = WMW_, WNW = WNW_, KS = KS_, RING = RING_;
-  static constexpr int OCC = OCC_, NW = WMW_ * WNW_;
+  static constexpr int OCC = OCC_, NW = WMW_ * WNW_, GK = GK_;
+  static constexpr bool SPREAD = SPREAD_;
 };
-constexpr int kMaxNormK = 2048;                      // A_NORM: gamma lives in LDS
+constexpr int kMaxNormK = 2048;   // the norm forms' largest K
 
 enum AMode { A_ROWS = 0, A_TILES = 1, A_NORM = 2 };
 enum Epi { E_STORE = 0, E_SWIGLU = 1, E_RESIDUAL = 2, E_QKV = 3 };
@@ -115,6 +126,15 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
+// The epilogue's own loads are used here, on every path: a load whose value only a branch uses is
+// still in flight for the compiler where that branch is not taken, and it then waits for it at the
+// first reuse of its registers, in the middle of the next tile's k-loop and on every pass through
+// it, where vmcnt(0) also waits for the copies of the stages ahead.
+__device__ __forceinline__ void landed(float v) { asm volatile("" ::"v"(v)); }
+__device__ __forceinline__ void landed(const float4& v) {
+  asm volatile("" ::"v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
+}
+
 template <int AMODE, int EPI, int AP, bool WL, class S>
 __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_kernel(
     const Args p) {
@@ -133,7 +153,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
   constexpr int kLoads = kACopies + kWCopies;
   static_assert(kACopies * kWaves * (kHiOnly ? 2 : 1) == KS * kAFrags &&
                 kWCopies * kWaves == KS * kWFrags, "every wave makes the same copies");
-  constexpr int kGammaBytes = AMODE == A_NORM ? kMaxNormK * 4 : 0;
+  constexpr int kGammaBytes = AMODE == A_NORM ? S::GK * 4 : 0;
   __shared__ __align__(16) uint8_t lds[kRing * kStage + kGammaBytes];
   __shared__ float rstd_s[kBM];
   // Persistent blocks: XCD x = blockIdx % 8 owns logical tiles [x per_xcd, (x + 1) per_xcd), row
@@ -145,14 +165,14 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
   const int first = t_lo + (blockIdx.x >> 3);
   if (first >= t_hi) return;   // whole block, before any barrier
   const int M = p.M, N = p.N, K = p.K, nk = K >> 5;
-  const int ns = (nk + KS - 1) / KS;                       // stages per tile
+  const int ns = nk / KS;                                  // stages per tile
   const int total = (t_hi - first + bpx - 1) / bpx * ns;   // stages over this block's tiles
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // wave grid WMW x WNW over the tile: wave (wm, wn) owns FM row blocks and FN weight fragments.
   // The A_NORM forms split x * gamma in registers after the LDS read, so there every row block
-  // belongs to one wave (4 x 1) and is converted once; the split forms use 2 x 2 (8 activation
-  // and 8 weight fragment reads per wave and k-step).
+  // belongs to one wave (WNW 1) and is converted once; the split forms of the large shape use
+  // 2 x 2 (8 activation and 8 weight fragment reads per wave and k-step).
   constexpr int WMW = S::WMW, WNW = S::WNW;
   constexpr int FM = kBM / 16 / WMW, FN = kBN / 16 / WNW;
   const int wm = wave % WMW, wn = wave / WMW;
@@ -160,43 +180,67 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
   const int last_nb = (N + 15) / 16 - 1, last_mb = (M + 15) / 16 - 1;
   const uint32_t lds0 = lds_addr(lds);
 
-  // The loads of stage s (k-steps KS s ..) of the tile at (m0, n0) into ring stage b: the waves
-  // take the stage's fragments in turn.  Weight fragment f is row block n0 / 16 + f (WL: f / 2,
-  // part f % 2, hi / lo); activation fragment f is row block f / 2, part f % 2 (hi / lo; for
-  // A_NORM the first or second kilobyte of the fp32 16 x 32 block, lane l's columns 0..3 or
-  // 4..7); with the hi part alone (AP 1, split forms) only the even f exist.  Fragment f lands
-  // in slot f of its k-step either way.  Every copy is one contiguous kilobyte per wave, except
-  // row-major A.  Row blocks past M or N and k-steps past K load valid memory (clamped to the
-  // last; tile-layout buffers hold its padding rows); their results are never used.
-  auto issue = [&](int m0, int n0, int s, int b) {
-    const uint32_t base = lds0 + b * kStage;
+  // The copies of a stage: the waves take its fragments in turn.  Weight fragment f is row block
+  // n0 / 16 + f (WL: f / 2, part f % 2, hi / lo); activation fragment f is row block f / 2, part
+  // f % 2 (hi / lo; for A_NORM the first or second kilobyte of the fp32 16 x 32 block, lane l's
+  // columns 0..3 or 4..7); with the hi part alone (AP 1, split forms) only the even f exist.
+  // Fragment f lands in slot f of its k-step either way.  Every copy is one contiguous kilobyte
+  // per wave, except row-major A.  Row blocks past M or N load valid memory (clamped to the last;
+  // tile-layout buffers hold its padding rows); their results are never used.
+  //
+  // `seek` finds each copy's first address in a tile, a scalar pointer, and `copy` makes it and
+  // moves the pointer on: six scalar instructions.  Found anew each time the address is a chain of
+  // a dozen (two clamps, 64-bit multiplies) in front of every copy.
+  const uint8_t* wsrc[kWCopies];
+  const uint8_t* asrc[AMODE == A_ROWS ? 1 : kACopies];
+  const uint32_t lane16 = 16 * lane;
+  constexpr int kPer = kHiOnly ? kAFrags / 2 : kAFrags;   // activation fragments of a k-step
+  constexpr int kXStep = AMODE == A_NORM ? 2048 : 1024;   // bytes of an activation block's k-step
+  int am0 = 0, as = 0;                                    // A_ROWS: the cursor itself
+  auto seek = [&](int m0, int n0) {
 #pragma unroll
     for (int j = 0; j < kWCopies; ++j) {
       const int f = kWaves * j + wave, ks = f / kWFrags, fw = f - ks * kWFrags;
       const int nb = min(n0 / 16 + (WL ? fw >> 1 : fw), last_nb);
       const uint16_t* src = WL && (fw & 1) ? p.wl : p.w;
-      const int st = min(KS * s + ks, nk - 1);
-      dma16(src + (static_cast<int64_t>(nb) * nk + st) * 512 + 8 * lane,
-            __builtin_amdgcn_readfirstlane(base + ks * kStep + (kAFrags + fw) * 1024));
+      wsrc[j] = reinterpret_cast<const uint8_t*>(src) + (static_cast<int64_t>(nb) * nk + ks) * 1024;
     }
+    if constexpr (AMODE == A_ROWS) {
+      am0 = m0;
+      as = 0;
+    } else {
 #pragma unroll
-    for (int j = 0; j < kACopies; ++j) {
-      constexpr int kPer = kHiOnly ? kAFrags / 2 : kAFrags;
+      for (int j = 0; j < kACopies; ++j) {
+        const int fa = kWaves * j + wave, ks = fa / kPer;
+        const int f = (kHiOnly ? 2 : 1) * (fa - ks * kPer), rb = f >> 1, part = f & 1;
+        const int64_t blk = min(m0 / 16 + rb, last_mb);
+        if constexpr (AMODE == A_NORM)
+          asrc[j] = reinterpret_cast<const uint8_t*>(p.x) + (blk * nk + ks) * 2048 + part * 1024;
+        else
+          asrc[j] = reinterpret_cast<const uint8_t*>(p.a) +
+                    (blk * AP * nk + part * nk + ks) * 1024;
+      }
+    }
+  };
+  auto copy = [&](int q, uint32_t base) {   // copy q < kLoads of the stage at LDS address base
+    if (q < kWCopies) {
+      const int f = kWaves * q + wave, ks = f / kWFrags, fw = f - ks * kWFrags;
+      dma16_free(wsrc[q], lane16,
+                 __builtin_amdgcn_readfirstlane(base + ks * kStep + (kAFrags + fw) * 1024));
+      wsrc[q] += KS * 1024;
+    } else {
+      const int j = q - kWCopies;
       const int fa = kWaves * j + wave, ks = fa / kPer;
       const int f = (kHiOnly ? 2 : 1) * (fa - ks * kPer), rb = f >> 1, part = f & 1;
-      const int st = min(KS * s + ks, nk - 1);
-      const void* src;
-      if constexpr (AMODE == A_NORM) {
-        const int64_t blk = static_cast<int64_t>(min(m0 / 16 + rb, last_mb)) * nk + st;
-        src = p.x + blk * 512 + 256 * part + 4 * lane;
-      } else if constexpr (AMODE == A_TILES) {
-        const int64_t blk = static_cast<int64_t>(min(m0 / 16 + rb, last_mb)) * AP * nk;
-        src = p.a + (blk + part * nk + st) * 512 + 8 * lane;
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(base + ks * kStep + f * 1024);
+      if constexpr (AMODE == A_ROWS) {
+        const int row = min(am0 + 16 * rb + c, M - 1);
+        dma16(p.a + static_cast<int64_t>(row) * p.lda + part * K + 32 * (KS * as + ks) + 8 * g,
+              dst);
       } else {
-        const int row = min(m0 + 16 * rb + c, M - 1);
-        src = p.a + static_cast<int64_t>(row) * p.lda + part * K + 32 * st + 8 * g;
+        dma16_free(asrc[j], lane16, dst);
+        asrc[j] += KS * kXStep;
       }
-      dma16(src, __builtin_amdgcn_readfirstlane(base + ks * kStep + f * 1024));
     }
   };
 
@@ -218,7 +262,21 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
     for (int j = 0; j < FM; ++j) ss[j] = 0.f;
   };
 
-  auto compute = [&](int s, const uint8_t* base) {
+  // k-step s from LDS, with the copies q0 .. q1 - 1 of the stage at `dst` spread over its MFMAs:
+  // the CU takes in a copy every 25-30 cycles, and a wave that has to wait for that issues
+  // nothing else meanwhile
+  constexpr int kParts = AP + (WL ? 1 : 0);
+  auto compute = [&](int s, const uint8_t* base, uint32_t dst, int q0, int q1) {
+    constexpr int kGroup = AMODE == A_NORM ? (FN < 4 ? FN : 4) : 1;
+    constexpr int kGroups = FN / kGroup * kParts;
+    int grp = 0;
+    auto copies = [&]() {   // after the MFMAs of group grp
+#pragma unroll
+      for (int q = q0 + (q1 - q0) * grp / kGroups; q < q0 + (q1 - q0) * (grp + 1) / kGroups; ++q)
+        copy(q, dst);
+      if (S::SPREAD) __builtin_amdgcn_sched_barrier(0x106);   // VALU, SALU, LDS reads may cross
+      ++grp;
+    };
     bf16x8_t ah[FM], al[FM];
     if constexpr (AMODE == A_NORM) {
       // x of row 16 (FM wm + j) + c, columns 8 g .. 8 g + 7: the split of x * gamma, as the
@@ -268,7 +326,6 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
     // to the 256-register limit).
     constexpr int kWPer = WL ? 2 : 1;   // fragments per weight row block
     if constexpr (AMODE == A_NORM) {
-      constexpr int kGroup = FN < 4 ? FN : 4;
       static_assert(FN % kGroup == 0, "the norm forms group their weight fragments");
 #pragma unroll
       for (int i = 0; i < FN; i += kGroup) {
@@ -290,6 +347,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
           for (int j = 0; j < FM; ++j)
             acc[i + u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], ah[j], acc[i + u][j],
                                                                     0, 0, 0);
+        copies();
         if constexpr (AP == 2) {
 #pragma unroll
           for (int u = 0; u < kGroup; ++u)
@@ -297,6 +355,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
             for (int j = 0; j < FM; ++j)
               acc[i + u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], al[j],
                                                                       acc[i + u][j], 0, 0, 0);
+          copies();
         }
         if constexpr (WL) {
 #pragma unroll
@@ -305,6 +364,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
             for (int j = 0; j < FM; ++j)
               acc[i + u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlf[u], ah[j],
                                                                       acc[i + u][j], 0, 0, 0);
+          copies();
         }
       }
     } else {
@@ -321,24 +381,30 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
               base + (kAFrags + 2 * (FN * wn + i) + 1) * 1024 + 16 * lane);
       }
 #pragma unroll
-      for (int i = 0; i < FN; ++i)
+      for (int i = 0; i < FN; ++i) {
 #pragma unroll
         for (int j = 0; j < FM; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], ah[j], acc[i][j], 0, 0, 0);
+        copies();
+      }
       if constexpr (AP == 2) {
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
+        for (int i = 0; i < FN; ++i) {
 #pragma unroll
           for (int j = 0; j < FM; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], al[j], acc[i][j], 0, 0, 0);
+          copies();
+        }
       }
       if constexpr (WL) {
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
+        for (int i = 0; i < FN; ++i) {
 #pragma unroll
           for (int j = 0; j < FM; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlf[i], ah[j], acc[i][j], 0, 0,
                                                                 0);
+          copies();
+        }
       }
     }
   };
@@ -347,9 +413,9 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
   // acc[row 16 (FM wm + j) + c][weight rows 16 (FN wn + i) + 4 g ..]
   auto epilogue = [&](int m0, int n0) {
     if constexpr (AMODE == A_NORM) {
-      // the four lane groups of a row in a fixed order (one wave per row block: WNW = 1); the
-      // barrier waits for LDS only, so the next tile's loads stay in flight (rstd_s was last read
-      // in the previous tile's epilogue, nk >= 1 stage barriers ago)
+      // the four lane groups of a row in a fixed order (one wave per row block); the barrier waits
+      // for LDS only, so the next tile's loads stay in flight (rstd_s was last read in the
+      // previous tile's epilogue, ns >= 1 stage barriers ago)
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
         float v = ss[j];
@@ -358,16 +424,18 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
         if (g == 0) rstd_s[16 * (FM * wm + j) + c] = rsqrtf(v / static_cast<float>(K) + p.eps);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if constexpr (EPI == E_STORE || EPI == E_QKV) {
-        if (p.rstd_out && n0 == 0 && tid < kBM && m0 + tid < M) p.rstd_out[m0 + tid] = rstd_s[tid];
-        static_assert(kBM <= kThreads, "one thread per row of the tile");
-      }
+    }
+    if constexpr (AMODE == A_NORM && (EPI == E_STORE || EPI == E_QKV)) {
+      static_assert(kBM <= kThreads, "one thread per row of the tile");
+      if (p.rstd_out && n0 == 0 && tid < kBM && m0 + tid < M) p.rstd_out[m0 + tid] = rstd_s[tid];
     }
     if constexpr (EPI == E_QKV) {
-      static_assert(AMODE == A_NORM && WNW == 1, "E_QKV follows the norm prologue");
+      static_assert(AMODE == A_NORM, "E_QKV follows the norm prologue");
       // the arithmetic of K2 (rope_cache.hip); n0 and d are multiples of 64, so lane (c, g) of
-      // weight fragment i holds dims 16 (i % 4) + 4 g .. + 3 of its head: RoPE pairs
-      // 8 (i % 4) + 2 g and + 1
+      // the tile's weight fragment f holds dims 16 (f % 4) + 4 g .. + 3 of its head: RoPE pairs
+      // 8 (f % 4) + 2 g and + 1
+      constexpr int kQ = FN < 4 ? FN : 4;   // distinct f % 4 of this wave
+      static_assert(4 % kQ == 0 && FN % kQ == 0, "the wave's fragments cycle through their dims");
       const int d = N / 3;
       const int64_t head_stride = static_cast<int64_t>(p.slots) * kHeadDim;
 #pragma unroll
@@ -391,15 +459,21 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
         const bool lead_row = p.out != nullptr && slot >= ks && slot - ks < p.lead;
         const float rs = rstd_s[r];
         const int64_t* pos3 = p.pos + static_cast<int64_t>(m) * 3;
-        float cs[8], sn[8];
+        float cs[2 * kQ], sn[2 * kQ];
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
-          rope_cos_sin(8 * (t >> 1) + 2 * g + (t & 1), pos3, p.rope_tab, p.ra, cs[t], sn[t]);
+        for (int t = 0; t < 2 * kQ; ++t)
+          rope_cos_sin(8 * ((FN * wn + (t >> 1)) & 3) + 2 * g + (t & 1), pos3, p.rope_tab, p.ra,
+                       cs[t], sn[t]);
+#pragma unroll
+        for (int t = 0; t < 2 * kQ; ++t) {
+          landed(cs[t]);
+          landed(sn[t]);
+        }
         const int64_t cache_row = (b * (d / kHeadDim) * static_cast<int64_t>(p.slots) + slot) *
                                   kHeadDim;
 #pragma unroll
         for (int i = 0; i < FN; ++i) {
-          const int n = n0 + 16 * i + 4 * g;
+          const int n = n0 + 16 * (FN * wn + i) + 4 * g;
           if (n >= N) continue;
           const f32x4_t v = acc[i][j];
           if (lead_row)
@@ -407,7 +481,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
                 make_float4(v[0], v[1], v[2], v[3]);
           const int part = n / d, e = n - part * d;
           const int head = e / kHeadDim, dim = e - head * kHeadDim;
-          const int q4 = i & 3;
+          const int q4 = i % kQ;
           const float a0 = v[0] * rs, a1 = v[1] * rs, a2 = v[2] * rs, a3 = v[3] * rs;
           uint2 o;
           if (part == 2) {
@@ -432,15 +506,15 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
         }
       }
     } else if constexpr (EPI == E_SWIGLU) {
-      // Gate fragment 2 pb, up fragment 2 pb + 1: channels 16 (n0 / 32 + FN wn / 2 + pb) + 4 g.
+      // Gate fragment 2 pb, up fragment 2 pb + 1: channels 16 (n0 / 32 + FN / 2 * wn + pb) + 4 g.
       // The bias loads of kG pairs are issued together, and those of the next kG pairs before
       // this group's stores: the compiler's wait for a load also waits for every older memory
       // operation (the stores before it, the next tile's copies), so loads issued one pair at a
       // time after the previous pair's stores took a full round trip per pair.
       const int F = p.d_ff;
       constexpr int NP = FN / 2, kG = NP % 4 == 0 ? 2 : 1;
-      static_assert(NP % (2 * kG) == 0, "bias groups");
-      auto chan = [&](int pb) { return 16 * (n0 / 32 + NP * wn + pb) + 4 * g; };
+      static_assert(FN % 2 == 0 && (NP == 1 || NP % (2 * kG) == 0), "bias groups");
+      auto chan = [&](int pb) { return 16 * (n0 / 32 + FN / 2 * wn + pb) + 4 * g; };
       auto load_bias = [&](int pb0, float4 (&bg)[kG], float4 (&bu)[kG]) {
 #pragma unroll
         for (int q = 0; q < kG; ++q) {
@@ -454,6 +528,8 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       auto store_h = [&](int pb0, const float4 (&bg)[kG], const float4 (&bu)[kG]) {
 #pragma unroll
         for (int q = 0; q < kG; ++q) {
+          landed(bg[q]);
+          landed(bu[q]);
           const int pb = pb0 + q, ch = chan(pb);
           if (2 * ch >= N) continue;
 #pragma unroll
@@ -479,17 +555,17 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       load_bias(0, ga, ua);
 #pragma unroll
       for (int pb0 = 0; pb0 < NP; pb0 += 2 * kG) {
-        load_bias(pb0 + kG, gb, ub);
+        if (pb0 + kG < NP) load_bias(pb0 + kG, gb, ub);
         store_h(pb0, ga, ua);
         if (pb0 + 2 * kG < NP) load_bias(pb0 + 2 * kG, ga, ua);
-        store_h(pb0 + kG, gb, ub);
+        if (pb0 + kG < NP) store_h(pb0 + kG, gb, ub);
       }
     } else {
       // The residual's loads of kG weight fragments are issued together, and those of the next
       // kG before this group's stores (see E_SWIGLU: one load and its wait per fragment, after
       // the previous fragment's store, took a full round trip each).
       constexpr int kG = FN % 4 == 0 ? 2 : 1;
-      static_assert(FN % (2 * kG) == 0, "residual groups");
+      static_assert(FN == 1 || FN % (2 * kG) == 0, "residual groups");
       auto col = [&](int i) { return n0 + 16 * (FN * wn + i) + 4 * g; };
       auto row = [&](int j) { return m0 + 16 * (FM * wm + j) + c; };
       auto load_x = [&](int i0, float4 (&xv)[kG][FM], float4 (&bv)[kG]) {
@@ -509,6 +585,11 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       auto store_x = [&](int i0, const float4 (&xv)[kG][FM], const float4 (&bv)[kG]) {
 #pragma unroll
         for (int u = 0; u < kG; ++u) {
+          if constexpr (EPI == E_RESIDUAL) {
+            landed(bv[u]);
+#pragma unroll
+            for (int j = 0; j < FM; ++j) landed(xv[u][j]);
+          }
           const int n = col(i0 + u);
           if (n >= N) continue;
 #pragma unroll
@@ -535,10 +616,10 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       load_x(0, xa, ba);
 #pragma unroll
       for (int i0 = 0; i0 < FN; i0 += 2 * kG) {
-        load_x(i0 + kG, xb, bb);
+        if (i0 + kG < FN) load_x(i0 + kG, xb, bb);
         store_x(i0, xa, ba);
         if (i0 + 2 * kG < FN) load_x(i0 + 2 * kG, xa, ba);
-        store_x(i0 + kG, xb, bb);
+        if (i0 + kG < FN) store_x(i0 + kG, xb, bb);
       }
     }
   };
@@ -554,38 +635,51 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
     m0 = mt * kBM;
     n0 = (t - mt * p.tiles_n) * kBN;
   };
-  int it = first, is = 0, im0, in0;   // issue cursor: tile, stage of the tile, tile origin
+  constexpr int kAhead = kRing - 1;   // stages in flight beyond the one being computed
+  int it = first, is = 0, im0, in0;   // issue cursor: tile, stage of the tile
   tile_origin(it, im0, in0);
+  seek(im0, in0);
   auto advance_issue = [&]() {
+    ++as;
     if (++is == ns) {
       is = 0;
       it += bpx;
       tile_origin(it, im0, in0);
+      seek(im0, in0);
     }
   };
-  constexpr int kAhead = kRing - 1;   // stages in flight beyond the one being computed
 #pragma unroll
-  for (int r = 0; r < kAhead; ++r)
-    if (r < total) {
-      issue(im0, in0, is, r);
-      advance_issue();
-    }
-  if (total >= kAhead) stage_barrier<(kAhead - 1) * kLoads>();
-  else stage_barrier<0>();
+  for (int r = 0; r < kAhead; ++r) {
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q) copy(q, lds0 + r * kStage);
+    advance_issue();
+  }
+  stage_barrier<(kAhead - 1) * kLoads>();
   int ct = first, cs = 0, cm0, cn0;   // compute cursor
   tile_origin(ct, cm0, cn0);
   reset();
   int b = 0;
   for (int u = 0; u < total; ++u) {
-    if (u + kAhead < total) {
-      issue(im0, in0, is, b == 0 ? kRing - 1 : b - 1);   // stage (u + kAhead) % kRing
-      advance_issue();
+    // past the block's last stage the copies go on (clamped addresses, stages no one reads), so
+    // that every step makes the same copies and waits for the same number
+    const uint32_t dst = lds0 + (b == 0 ? kRing - 1 : b - 1) * kStage;   // (u + kAhead) % kRing
+    if constexpr (!S::SPREAD) {
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q) {
+        copy(q, dst);
+        // one copy every 80 cycles (14 wait states and six scalar instructions of 4 cycles):
+        // 310 us for the down projection of 65,536 rows; 336-352 at 24-64 cycles, 324 at 104
+        asm volatile("s_nop 13");
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      if (KS == 1 || KS * cs + ks < nk) compute(KS * cs + ks, lds + b * kStage + ks * kStep);
-    if (u + kAhead < total) stage_barrier<(kAhead - 1) * kLoads>();
-    else stage_barrier<0>();
+    for (int ks = 0; ks < KS; ++ks) {
+      constexpr int n = S::SPREAD ? kLoads : 0;
+      compute(KS * cs + ks, lds + b * kStage + ks * kStep, dst, n * ks / KS, n * (ks + 1) / KS);
+    }
+    advance_issue();
+    stage_barrier<(kAhead - 1) * kLoads>();
     b = b == kRing - 1 ? 0 : b + 1;
     if (++cs == ns) {
       epilogue(cm0, cn0);
@@ -595,6 +689,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       tile_origin(ct, cm0, cn0);
     }
   }
+  stage_barrier<0>();   // the last copies land while the LDS is still this block's
 }
 
 // CUs of the current device (hipDeviceAttributeMultiprocessorCount), cached per device
@@ -629,13 +724,107 @@ int launch_shape(Args p, hipStream_t st) {
   return launch_status();
 }
 
-using NormTile = Shape<128, 256, 4, 1, 1, 2, 2>;
-using SplitTile = Shape<128, 256, 2, 2, 1, 2, 2>;
+// The block shapes, smallest tile first.  The more blocks a product gives, the more it pays to
+// hand each a tile that reads less per MFMA.  The norm forms keep a row block in one wave of the
+// small and mid shapes too, except that gamma's room bounds their K (GK).
+template <bool NORM>
+struct Shapes;
+template <>
+struct Shapes<true> {
+  using Small = Shape<64, 64, 4, 1, 2, 3, 2, true, 1920>;
+  using Mid = Shape<128, 128, 4, 1, 1, 3, 2, true, 1920>;
+  using Wide = Shape<128, 256, 8, 1, 1, 4, 1, true, 1920>;
+  using Large = Shape<128, 256, 4, 1, 1, 2, 2, false>;
+};
+template <>
+struct Shapes<false> {
+  using Small = Shape<64, 64, 4, 2, 2, 3, 2, true>;
+  using Mid = Shape<128, 128, 4, 2, 2, 3, 1, true>;
+  using Wide = Shape<128, 256, 4, 2, 1, 4, 1, true>;
+  using Large = Shape<128, 256, 2, 2, 1, 2, 2, false>;
+};
 
-template <int AMODE, int EPI, int AP = 2>
-int launch(Args p, hipStream_t st) {
-  if constexpr (AMODE == A_NORM) return launch_shape<AMODE, EPI, AP, false, NormTile>(p, st);
-  else return launch_shape<AMODE, EPI, AP, false, SplitTile>(p, st);
+enum Route { R_SMALL, R_MID, R_WIDE, R_LARGE };
+
+// What a k-step takes (us) on tiles of this size: `single` with at most one per CU, else `base` +
+// `round` for every filling of the chip (CUs x OCC blocks).  Fitted to the launches of d = 768, F =
+// 2048 and d = 1280, F = 3392 at 64 to 16,669 rows.
+struct StepCost {
+  int bm, bn, occ;
+  float single, base, round;
+};
+
+template <class S>
+constexpr StepCost step_cost(float single, float base, float round) {
+  return {S::BM, S::BN, S::OCC, single, base, round};
+}
+
+// The cheapest of `costs` for an [m, k] x [n, k]^T product
+int cheapest(const StepCost* costs, int count, int m, int n) {
+  int best = 0;
+  float best_cost = 1e30f;
+  for (int i = 0; i < count; ++i) {
+    const StepCost& c = costs[i];
+    const int64_t tiles = ((static_cast<int64_t>(m) + c.bm - 1) / c.bm) *
+                          ((static_cast<int64_t>(n) + c.bn - 1) / c.bn);
+    const int64_t slots = static_cast<int64_t>(device_cus()) * c.occ;
+    const float cost = tiles <= device_cus()
+                           ? c.single
+                           : c.base + c.round * static_cast<float>((tiles + slots - 1) / slots);
+    if (cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// Measured at d = 768, F = 2048, us per launch (qkv / out / gate-up / down), one block of 256 x 256
+// per CU (what every size ran on before these shapes) -> the shape taken here:
+//   256 rows    50 / 37 / 43 / 87      12 / 6 / 12 / 11     small
+//   731 rows    53 / 38 / 45 / 88      17 / 7 / 21 / 16     small / small / mid / small
+//   2,048 rows  54 / 38 / 48 / 88      30 / 10 / 29 / 20    wide / small / wide / small
+//   4,096 rows  57 / 41 / 54 / 90      50 / 16 / 49 / 30    large / mid / large / mid
+//   8,192 rows  106 / 42 / 99 / 92     77 / 28 / 90 / 53    mid / wide / large / wide
+Route pick_route(bool norm, int m, int n, int k) {
+  static constexpr StepCost kNorm[] = {step_cost<Shapes<true>::Small>(0.5f, 0.35f, 0.375f),
+                                       step_cost<Shapes<true>::Mid>(0.97f, 0.25f, 1.07f),
+                                       step_cost<Shapes<true>::Wide>(1.25f, 0.22f, 1.03f),
+                                       step_cost<Shapes<true>::Large>(1.7f, 0.2f, 1.88f)};
+  static constexpr StepCost kSplit[] = {step_cost<Shapes<false>::Small>(0.26f, 0.1f, 0.3f),
+                                        step_cost<Shapes<false>::Mid>(0.5f, 0.05f, 0.52f),
+                                        step_cost<Shapes<false>::Wide>(0.9f, 0.1f, 0.9f),
+                                        step_cost<Shapes<false>::Large>(1.2f, 0.1f, 1.45f)};
+  if (norm) {
+    if (k > Shapes<true>::Wide::GK) return R_LARGE;
+    const int skip = k % 64 ? 1 : 0;   // the small shape takes two k-steps at a time
+    return static_cast<Route>(skip + cheapest(kNorm + skip, 4 - skip, m, n));
+  }
+  const int skip = k % 64 ? 2 : 0;     // the small and the mid shape do
+  return static_cast<Route>(skip + cheapest(kSplit + skip, 4 - skip, m, n));
+}
+
+template <int AMODE, int EPI>
+int launch(const Args& p, hipStream_t st) {
+  using T = Shapes<AMODE == A_NORM>;
+  switch (pick_route(AMODE == A_NORM, p.M, p.N, p.K)) {
+    case R_SMALL: return launch_shape<AMODE, EPI, 2, false, typename T::Small>(p, st);
+    case R_MID: return launch_shape<AMODE, EPI, 2, false, typename T::Mid>(p, st);
+    case R_WIDE: return launch_shape<AMODE, EPI, 2, false, typename T::Wide>(p, st);
+    default: return launch_shape<AMODE, EPI, 2, false, typename T::Large>(p, st);
+  }
+}
+
+// the split forms by A layout and parts: row-major activations, and the forms with the hi part
+// alone, are not on the prompt path and run on the large shape
+template <int EPI>
+int launch_split(const Args& p, int a_layout, int a_parts, hipStream_t st) {
+  using Large = Shapes<false>::Large;
+  if (a_layout == MDL_LAYOUT_ROWS)
+    return a_parts == 1 ? launch_shape<A_ROWS, EPI, 1, false, Large>(p, st)
+                        : launch_shape<A_ROWS, EPI, 2, false, Large>(p, st);
+  return a_parts == 1 ? launch_shape<A_TILES, EPI, 1, false, Large>(p, st)
+                      : launch<A_TILES, EPI>(p, st);
 }
 
 // shared argument checks: k a positive multiple of 32, n of 16, 16-byte aligned operands
@@ -656,14 +845,6 @@ int check_a(const uint16_t* a, int64_t lda, int a_layout, int a_parts, int k) {
   return MDL_OK;
 }
 
-// the split forms by A layout and parts
-template <int EPI>
-int launch_split(const Args& p, int a_layout, int a_parts, hipStream_t st) {
-  if (a_layout == MDL_LAYOUT_TILES)
-    return a_parts == 1 ? launch<A_TILES, EPI, 1>(p, st) : launch<A_TILES, EPI, 2>(p, st);
-  return a_parts == 1 ? launch<A_ROWS, EPI, 1>(p, st) : launch<A_ROWS, EPI, 2>(p, st);
-}
-
 }  // namespace
 }  // namespace mdl
 
@@ -681,8 +862,7 @@ extern "C" int mdl_prefill_gemm_split(const uint16_t* a, int64_t lda, int a_layo
   if (m == 0) return MDL_OK;
   Args p{};
   p.a = a; p.lda = lda; p.w = w; p.out = out; p.ldo = ldo; p.M = m; p.N = n; p.K = k;
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  return launch_split<E_STORE>(p, a_layout, a_parts, st);
+  return launch_split<E_STORE>(p, a_layout, a_parts, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mdl_prefill_gemm_norm(const float* x, const float* gamma, float eps,
@@ -720,7 +900,8 @@ extern "C" int mdl_prefill_gemm_norm_swiglu(const float* x, const float* gamma, 
   p.x = x; p.gamma = gamma; p.eps = eps; p.w = w_gu; p.bias_a = bias_gate; p.bias_b = bias_up;
   p.h = h_out; p.d_ff = d_ff; p.h_parts = h_parts; p.M = m; p.N = 2 * d_ff; p.K = k;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  return a_parts == 1 ? launch<A_NORM, E_SWIGLU, 1>(p, st) : launch<A_NORM, E_SWIGLU, 2>(p, st);
+  return a_parts == 1 ? launch_shape<A_NORM, E_SWIGLU, 1, false, Shapes<true>::Large>(p, st)
+                      : launch<A_NORM, E_SWIGLU>(p, st);
 }
 
 extern "C" int mdl_prefill_gemm_split_residual(const uint16_t* a, int64_t lda, int a_layout,
@@ -736,8 +917,7 @@ extern "C" int mdl_prefill_gemm_split_residual(const uint16_t* a, int64_t lda, i
   if (m == 0) return MDL_OK;
   Args p{};
   p.a = a; p.lda = lda; p.w = w; p.x_res = x; p.bias_a = bias; p.M = m; p.N = n; p.K = k;
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  return launch_split<E_RESIDUAL>(p, a_layout, a_parts, st);
+  return launch_split<E_RESIDUAL>(p, a_layout, a_parts, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mdl_prefill_gemm_norm_qkv(

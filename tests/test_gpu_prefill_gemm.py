@@ -321,3 +321,64 @@ def test_split_gemm_at_config2_size_against_hipblaslt():
     aa = a[rows].double()
     sub = (aa[:, :k] + aa[:, k:]) @ w.double().t()
     assert float((out[rows].double() - sub).abs().max() / sub.abs().max()) < 2e-6
+
+
+# rows at the tiles' edges, and where d = 768, F = 2048 products change their block shape: the norm
+# forms run small / mid / wide / large, the split forms likewise, over these row counts
+ROUTE_ROWS = [1, 63, 65, 257, 731, 1025, 2047, 3000, 4097, 6030, 8193]
+
+
+@pytest.mark.parametrize("k", [768, 1952, 1984])   # odd multiples of 32, past gamma's 1,920
+def test_rows_do_not_depend_on_the_row_count(k):
+    """Every block shape sums in the same order, so the first m rows of a product are the same bits
+    whatever m is: each form at row counts that take each shape, against the rows of one large
+    product (which the tests above pin to fp64)."""
+    f, total = 2048, 20_000
+    g = torch.Generator(DEV).manual_seed(k)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    wgu = K().tile_matrix((0.05 * rnd(2 * f, k)).to(torch.bfloat16))
+    wo = K().tile_matrix((0.05 * rnd(768, k)).to(torch.bfloat16))
+    x, gam, bias = rnd(total, k), 1 + 0.1 * rnd(k), rnd(f)
+    a, res = torch.cat(split(rnd(total, k)), 1).contiguous(), rnd(total, 768)
+
+    def forms(m):
+        xt, at = K().tile_f32(x[:m]), K().tile_matrix(a[:m].contiguous())
+        store, rs = torch.empty(m, 2 * f, device=DEV), torch.empty(m, device=DEV)
+        K().prefill_gemm_norm(xt, gam, 1e-5, wgu, store, rs, k)
+        h = torch.empty(K().split_numel(m, f, True), dtype=torch.bfloat16, device=DEV)
+        K().prefill_gemm_norm_swiglu(xt, gam, 1e-5, wgu, bias, bias, h, m, f, k)
+        out = torch.empty(m, 768, device=DEV)
+        K().prefill_gemm_split(at, wo, out, k, a_tiled=True)
+        xr = K().tile_f32(res[:m])
+        K().prefill_gemm_split_residual(at, wo, xr, bias, m, 768, k, a_tiled=True)
+        return store, rs, K().untile_matrix(h, m, 2 * f), out, K().untile_f32(xr, m, 768)
+
+    whole = forms(total)
+    for m in ROUTE_ROWS:
+        for name, got, want in zip(("store", "rstd", "swiglu", "split", "residual"), forms(m),
+                                   whole):
+            assert torch.equal(got, want[:m]), f"{name} at {m} rows"
+
+
+@pytest.mark.parametrize("m", ROUTE_ROWS)
+def test_norm_qkv_at_each_block_shape(m):
+    """The qkv epilogue of each shape against the E_STORE form and K2, bit for bit."""
+    H, d = 12, 768
+    g = torch.Generator(DEV).manual_seed(m)
+    x = torch.randn(m, d, generator=g, device=DEV)
+    gam = 1 + 0.1 * torch.randn(d, generator=g, device=DEV)
+    w = K().tile_matrix((0.05 * torch.randn(3 * d, d, generator=g, device=DEV)).to(torch.bfloat16))
+    pos = torch.randint(0, 35, (m, 3), generator=g, device=DEV)
+    tab, geom = _rope()
+    xt = K().tile_f32(x)
+    qkv, rs1, rs2 = torch.empty(m, 3 * d, device=DEV), *torch.empty(2, m, device=DEV).unbind()
+    K().prefill_gemm_norm(xt, gam, 1e-5, w, qkv, rs1, d)
+    bf = lambda *s: torch.full(s, 7.0, dtype=torch.bfloat16, device=DEV)  # noqa: E731
+    q1, kc1, vc1 = bf(m, d), bf(1, H, m + 3, 64), bf(1, H, m + 3, 64)
+    K().qkv_rope_cache(qkv, rs1, pos, tab, geom, 1, m, H, 0.125, q1, kc1, vc1, slot0=0)
+    q2, kc2, vc2 = bf(m, d), bf(1, H, m + 3, 64), bf(1, H, m + 3, 64)
+    lead = torch.full((m, 3 * d), float("nan"), device=DEV)
+    K().prefill_gemm_norm_qkv(xt, gam, 1e-5, w, m, H, rs2, lead, K().LEAD_QUERIES, None, pos, tab,
+                              geom, 0.125, q2, kc2, vc2, seq=m)
+    for got, want in ((rs2, rs1), (q2, q1), (kc2, kc1), (vc2, vc1), (lead[:64], qkv[:64])):
+        assert torch.equal(got, want)

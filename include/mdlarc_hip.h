@@ -378,6 +378,23 @@ int mdl_prefill_gemm_split_residual(const uint16_t* a, int64_t lda, int a_layout
                                     const uint16_t* w, float* x, const float* bias, int m, int n,
                                     int k, void* stream);
 /*
+ * The same for an fp32 weight, passed as its high and low bf16 parts w = bf16(W), w_lo =
+ * bf16(W - w), both tiled (as mdl_gemm_norm takes them): each k-step adds a_hi . w_lo after the hi
+ * and lo products, so the weight is seen to ~2^-17 like the activation.  a is the tiled split
+ * activation, h_out the tiled split [m, 2 d_ff]; the other arguments and limits as above.  Up to
+ * 640 rows run on K5 (mdl_gemm_norm and its kind), with that kernel's order of the sums.
+ */
+int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, float eps, const uint16_t* w,
+                               const uint16_t* w_lo, float* out, int64_t ldo, float* rstd_out,
+                               int m, int n, int k, void* stream);
+int mdl_prefill_gemm_norm_swiglu_f32w(const float* x, const float* gamma, float eps,
+                                      const uint16_t* w_gu, const uint16_t* w_gu_lo,
+                                      const float* bias_gate, const float* bias_up,
+                                      uint16_t* h_out, int m, int d_ff, int k, void* stream);
+int mdl_prefill_gemm_split_residual_f32w(const uint16_t* a, const uint16_t* w,
+                                         const uint16_t* w_lo, float* x, const float* bias, int m,
+                                         int n, int k, void* stream);
+/*
  * K6 with K2 (mdl_qkv_rope_cache) in its epilogue: ln1 + qkv_proj + RoPE + cache write of a
  * prompt in one launch.  w: qkv_proj tiled [3 d, d] (d = n_heads * 64, at most 2048); x as for
  * mdl_prefill_gemm_norm.  Writes, from the projection's fp32 accumulators and rstd, exactly what

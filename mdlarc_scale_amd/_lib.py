@@ -72,6 +72,11 @@ SIGNATURES: dict[str, tuple[object, list]] = {
                                              c_int, c_int, P]),
     "mdl_prefill_gemm_split_residual": (c_int, [P, c_int64, c_int, c_int, P, P, P, c_int, c_int,
                                                 c_int, P]),
+    "mdl_prefill_gemm_norm_f32w": (c_int, [P, P, c_float, P, P, P, c_int64, P, c_int, c_int,
+                                           c_int, P]),
+    "mdl_prefill_gemm_norm_swiglu_f32w": (c_int, [P, P, c_float, P, P, P, P, P, c_int, c_int,
+                                                  c_int, P]),
+    "mdl_prefill_gemm_split_residual_f32w": (c_int, [P, P, P, P, P, c_int, c_int, c_int, P]),
     "mdl_prefill_gemm_norm_qkv": (c_int, [P, P, c_float, P, c_int, c_int, P, P, c_int64, c_int, P,
                                           P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
                                           P, P, P, c_int, c_int, c_int, P, P, P]),

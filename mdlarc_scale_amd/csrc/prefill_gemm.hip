@@ -724,53 +724,69 @@ int launch_shape(Args p, hipStream_t st) {
   return launch_status();
 }
 
-// The block shapes, smallest tile first.  The more blocks a product gives, the more it pays to
-// hand each a tile that reads less per MFMA.  The norm forms keep a row block in one wave of the
-// small and mid shapes too, except that gamma's room bounds their K (GK).
-template <bool NORM>
-struct Shapes;
-template <>
-struct Shapes<true> {
-  using Small = Shape<64, 64, 4, 1, 2, 3, 2, true, 1920>;
-  using Mid = Shape<128, 128, 4, 1, 1, 3, 2, true, 1920>;
-  using Wide = Shape<128, 256, 8, 1, 1, 4, 1, true, 1920>;
-  using Large = Shape<128, 256, 4, 1, 1, 2, 2, false>;
+// The block shapes, smallest tile first: the more blocks a product gives, the more it pays to hand
+// each a tile that reads less per MFMA.  Every norm form keeps a row block in one wave; gamma's
+// room bounds the K of all but the last (GK).
+struct NormShapes {
+  using S0 = Shape<64, 64, 4, 1, 2, 3, 2, true, 1920>;
+  using S1 = Shape<128, 128, 4, 1, 1, 3, 2, true, 1920>;
+  using S2 = Shape<128, 256, 8, 1, 1, 4, 1, true, 1920>;
+  using S3 = Shape<128, 256, 4, 1, 1, 2, 2, true>;
+  using S4 = Shape<128, 256, 4, 1, 1, 2, 2, false>;
 };
-template <>
-struct Shapes<false> {
-  using Small = Shape<64, 64, 4, 2, 2, 3, 2, true>;
-  using Mid = Shape<128, 128, 4, 2, 2, 3, 1, true>;
-  using Wide = Shape<128, 256, 4, 2, 1, 4, 1, true>;
-  using Large = Shape<128, 256, 2, 2, 1, 2, 2, false>;
+struct SplitShapes {
+  using S0 = Shape<64, 64, 4, 2, 2, 3, 2, true>;
+  using S1 = Shape<128, 128, 4, 2, 2, 3, 1, true>;
+  using S2 = Shape<128, 256, 4, 2, 1, 4, 1, true>;
+  using S3 = Shape<128, 256, 2, 2, 1, 2, 2, false>;
+  using S4 = S3;
+};
+// fp32 weights: twice the weight fragments, so half the weight rows a tile
+struct NormShapesF32 {
+  using S0 = Shape<64, 64, 4, 1, 2, 2, 2, true, 1920>;
+  using S1 = Shape<64, 128, 4, 1, 1, 3, 2, true, 1920>;
+  using S2 = Shape<128, 128, 4, 1, 1, 2, 2, true>;
+  using S3 = Shape<256, 128, 8, 1, 1, 3, 1, true>;
+  using S4 = S3;
+};
+struct SplitShapesF32 {
+  using S0 = Shape<64, 64, 4, 2, 2, 2, 2, true>;
+  using S1 = Shape<128, 64, 2, 2, 1, 3, 2, true>;
+  using S2 = Shape<128, 128, 2, 2, 1, 2, 2, false>;
+  using S3 = S2;
+  using S4 = S2;
 };
 
-enum Route { R_SMALL, R_MID, R_WIDE, R_LARGE };
-
-// What a k-step takes (us) on tiles of this size: `single` with at most one per CU, else `base` +
-// `round` for every filling of the chip (CUs x OCC blocks).  Fitted to the launches of d = 768, F =
-// 2048 and d = 1280, F = 3392 at 64 to 16,669 rows.
+// What a k-step takes (us) on tiles of a shape: `single` with at most one per CU, else `base` +
+// `round` for every filling of the chip (CUs x OCC blocks), for up to `limit` of these.  Fitted to
+// launches of d = 768, F = 2048 and d = 1280, F = 3392 at 64 to 282,695 rows.
 struct StepCost {
-  int bm, bn, occ;
+  int bm, bn, ks, gk, occ;
   float single, base, round;
+  int limit;
 };
+constexpr int kAnyRounds = 0x7fffffff;
 
 template <class S>
-constexpr StepCost step_cost(float single, float base, float round) {
-  return {S::BM, S::BN, S::OCC, single, base, round};
+constexpr StepCost step_cost(float single, float base, float round, int limit = kAnyRounds) {
+  return {S::BM, S::BN, S::KS, S::GK, S::OCC, single, base, round, limit};
 }
 
-// The cheapest of `costs` for an [m, k] x [n, k]^T product
-int cheapest(const StepCost* costs, int count, int m, int n) {
-  int best = 0;
+// The index of the cheapest shape for an [m, k] x [n, k]^T product; the last one takes every size
+template <int COUNT>
+int cheapest(const StepCost (&costs)[COUNT], bool norm, int m, int n, int k) {
+  int best = COUNT - 1;
   float best_cost = 1e30f;
-  for (int i = 0; i < count; ++i) {
+  for (int i = 0; i < COUNT; ++i) {
     const StepCost& c = costs[i];
+    if (k % (32 * c.ks) || (norm && k > c.gk)) continue;
     const int64_t tiles = ((static_cast<int64_t>(m) + c.bm - 1) / c.bm) *
                           ((static_cast<int64_t>(n) + c.bn - 1) / c.bn);
     const int64_t slots = static_cast<int64_t>(device_cus()) * c.occ;
-    const float cost = tiles <= device_cus()
-                           ? c.single
-                           : c.base + c.round * static_cast<float>((tiles + slots - 1) / slots);
+    const int64_t rounds = (tiles + slots - 1) / slots;
+    if (rounds > c.limit) continue;
+    const float cost =
+        tiles <= device_cus() ? c.single : c.base + c.round * static_cast<float>(rounds);
     if (cost < best_cost) {
       best = i;
       best_cost = cost;
@@ -781,50 +797,80 @@ int cheapest(const StepCost* costs, int count, int m, int n) {
 
 // Measured at d = 768, F = 2048, us per launch (qkv / out / gate-up / down), one block of 256 x 256
 // per CU (what every size ran on before these shapes) -> the shape taken here:
-//   256 rows    50 / 37 / 43 / 87      12 / 6 / 12 / 11     small
-//   731 rows    53 / 38 / 45 / 88      17 / 7 / 21 / 16     small / small / mid / small
-//   2,048 rows  54 / 38 / 48 / 88      30 / 10 / 29 / 20    wide / small / wide / small
-//   4,096 rows  57 / 41 / 54 / 90      50 / 16 / 49 / 30    large / mid / large / mid
-//   8,192 rows  106 / 42 / 99 / 92     77 / 28 / 90 / 53    mid / wide / large / wide
-Route pick_route(bool norm, int m, int n, int k) {
-  static constexpr StepCost kNorm[] = {step_cost<Shapes<true>::Small>(0.5f, 0.35f, 0.375f),
-                                       step_cost<Shapes<true>::Mid>(0.97f, 0.25f, 1.07f),
-                                       step_cost<Shapes<true>::Wide>(1.25f, 0.22f, 1.03f),
-                                       step_cost<Shapes<true>::Large>(1.7f, 0.2f, 1.88f)};
-  static constexpr StepCost kSplit[] = {step_cost<Shapes<false>::Small>(0.26f, 0.1f, 0.3f),
-                                        step_cost<Shapes<false>::Mid>(0.5f, 0.05f, 0.52f),
-                                        step_cost<Shapes<false>::Wide>(0.9f, 0.1f, 0.9f),
-                                        step_cost<Shapes<false>::Large>(1.2f, 0.1f, 1.45f)};
-  if (norm) {
-    if (k > Shapes<true>::Wide::GK) return R_LARGE;
-    const int skip = k % 64 ? 1 : 0;   // the small shape takes two k-steps at a time
-    return static_cast<Route>(skip + cheapest(kNorm + skip, 4 - skip, m, n));
-  }
-  const int skip = k % 64 ? 2 : 0;     // the small and the mid shape do
-  return static_cast<Route>(skip + cheapest(kSplit + skip, 4 - skip, m, n));
+//   256 rows    50 / 37 / 43 / 87      12 / 6 / 12 / 11     S0
+//   731 rows    53 / 38 / 45 / 88      17 / 7 / 21 / 13     S0
+//   2,300 rows  55 / 38 / 48 / 88      30 / 10 / 40 / 22    S2 / S0 / S3 / S0
+//   4,096 rows  57 / 41 / 54 / 90      50 / 16 / 51 / 31    S3 / S1 / S3 / S1
+//   8,192 rows  106 / 42 / 99 / 92     77 / 28 / 92 / 55    S1 / S2 / S3 / S2
+//   16,669      157 / 50 / 227 / 103   126 / 45 / 185 / 90  S3
+// Past five rounds the power limit sets in, and the paced copies of the norm forms' S4 win: 701
+// against 729 us for the gate / up projection of 65,536 rows.
+int pick_shape(bool norm, int m, int n, int k) {
+  static constexpr StepCost kNorm[] = {
+      step_cost<NormShapes::S0>(0.5f, 0.35f, 0.375f), step_cost<NormShapes::S1>(0.97f, 0.25f, 1.12f),
+      step_cost<NormShapes::S2>(1.25f, 0.22f, 1.03f),
+      step_cost<NormShapes::S3>(1.6f, 0.15f, 1.7f, 5), step_cost<NormShapes::S4>(1.7f, 0.5f, 1.7f)};
+  static constexpr StepCost kSplit[] = {
+      step_cost<SplitShapes::S0>(0.26f, 0.1f, 0.3f), step_cost<SplitShapes::S1>(0.5f, 0.05f, 0.52f),
+      step_cost<SplitShapes::S2>(0.9f, 0.1f, 0.9f), step_cost<SplitShapes::S3>(1.2f, 0.1f, 1.45f)};
+  return norm ? cheapest(kNorm, true, m, n, k) : cheapest(kSplit, false, m, n, k);
 }
 
-template <int AMODE, int EPI>
-int launch(const Args& p, hipStream_t st) {
-  using T = Shapes<AMODE == A_NORM>;
-  switch (pick_route(AMODE == A_NORM, p.M, p.N, p.K)) {
-    case R_SMALL: return launch_shape<AMODE, EPI, 2, false, typename T::Small>(p, st);
-    case R_MID: return launch_shape<AMODE, EPI, 2, false, typename T::Mid>(p, st);
-    case R_WIDE: return launch_shape<AMODE, EPI, 2, false, typename T::Wide>(p, st);
-    default: return launch_shape<AMODE, EPI, 2, false, typename T::Large>(p, st);
+// The same for fp32 weights, against K5 (norm / out / gate-up / down, us; d = 768, F = 2048):
+//   731 rows     17 / 8 / 24 / 19         17 / 8 / 23 / 22
+//   2,300 rows   55 / 22 / 86 / 41        34 / 12 / 52 / 26
+//   11,242 rows  243 / 101 / 413 / 213    117 / 45 / 185 / 102
+// At 256 rows K5 takes 9 / 5 / 9 / 8 against 11 / 8 / 12 / 16: see kK5Rows.
+int pick_shape_f32(bool norm, int m, int n, int k) {
+  static constexpr StepCost kNorm[] = {step_cost<NormShapesF32::S0>(0.47f, 0.2f, 0.52f),
+                                       step_cost<NormShapesF32::S1>(0.72f, 0.3f, 0.65f),
+                                       step_cost<NormShapesF32::S2>(1.1f, 0.2f, 1.25f, 12),
+                                       step_cost<NormShapesF32::S3>(1.5f, 1.5f, 1.42f)};
+  static constexpr StepCost kSplit[] = {step_cost<SplitShapesF32::S0>(0.35f, 0.1f, 0.37f),
+                                        step_cost<SplitShapesF32::S1>(0.5f, 0.1f, 0.63f),
+                                        step_cost<SplitShapesF32::S2>(1.05f, 0.05f, 1.27f)};
+  return norm ? cheapest(kNorm, true, m, n, k) : cheapest(kSplit, false, m, n, k);
+}
+
+template <int AMODE, int EPI, bool WL, class T>
+int launch_of(int shape, const Args& p, hipStream_t st) {
+  switch (shape) {
+    case 0: return launch_shape<AMODE, EPI, 2, WL, typename T::S0>(p, st);
+    case 1: return launch_shape<AMODE, EPI, 2, WL, typename T::S1>(p, st);
+    case 2: return launch_shape<AMODE, EPI, 2, WL, typename T::S2>(p, st);
+    case 3: return launch_shape<AMODE, EPI, 2, WL, typename T::S3>(p, st);
+    default: return launch_shape<AMODE, EPI, 2, WL, typename T::S4>(p, st);
   }
 }
+
+template <int EPI>
+int launch_norm(const Args& p, hipStream_t st) {
+  return launch_of<A_NORM, EPI, false, NormShapes>(pick_shape(true, p.M, p.N, p.K), p, st);
+}
+
+template <int EPI>
+int launch_f32w(const Args& p, hipStream_t st) {
+  if constexpr (EPI == E_RESIDUAL)
+    return launch_of<A_TILES, EPI, true, SplitShapesF32>(pick_shape_f32(false, p.M, p.N, p.K), p,
+                                                         st);
+  else
+    return launch_of<A_NORM, EPI, true, NormShapesF32>(pick_shape_f32(true, p.M, p.N, p.K), p, st);
+}
+
+// fp32 weights: up to this many rows the projections run on K5, whose waves split K and need no
+// ring to fill (d = 768: 31 us a layer against 45 at 256 rows, 67 against 70 at 731)
+constexpr int kK5Rows = 640;
 
 // the split forms by A layout and parts: row-major activations, and the forms with the hi part
 // alone, are not on the prompt path and run on the large shape
 template <int EPI>
 int launch_split(const Args& p, int a_layout, int a_parts, hipStream_t st) {
-  using Large = Shapes<false>::Large;
+  using Large = SplitShapes::S4;
   if (a_layout == MDL_LAYOUT_ROWS)
     return a_parts == 1 ? launch_shape<A_ROWS, EPI, 1, false, Large>(p, st)
                         : launch_shape<A_ROWS, EPI, 2, false, Large>(p, st);
-  return a_parts == 1 ? launch_shape<A_TILES, EPI, 1, false, Large>(p, st)
-                      : launch<A_TILES, EPI>(p, st);
+  if (a_parts == 1) return launch_shape<A_TILES, EPI, 1, false, Large>(p, st);
+  return launch_of<A_TILES, EPI, false, SplitShapes>(pick_shape(false, p.M, p.N, p.K), p, st);
 }
 
 // shared argument checks: k a positive multiple of 32, n of 16, 16-byte aligned operands
@@ -878,7 +924,7 @@ extern "C" int mdl_prefill_gemm_norm(const float* x, const float* gamma, float e
   Args p{};
   p.x = x; p.gamma = gamma; p.eps = eps; p.w = w; p.out = out; p.ldo = ldo;
   p.rstd_out = rstd_out; p.M = m; p.N = n; p.K = k;
-  return launch<A_NORM, E_STORE>(p, static_cast<hipStream_t>(stream));
+  return launch_norm<E_STORE>(p, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mdl_prefill_gemm_norm_swiglu(const float* x, const float* gamma, float eps,
@@ -900,8 +946,8 @@ extern "C" int mdl_prefill_gemm_norm_swiglu(const float* x, const float* gamma, 
   p.x = x; p.gamma = gamma; p.eps = eps; p.w = w_gu; p.bias_a = bias_gate; p.bias_b = bias_up;
   p.h = h_out; p.d_ff = d_ff; p.h_parts = h_parts; p.M = m; p.N = 2 * d_ff; p.K = k;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  return a_parts == 1 ? launch_shape<A_NORM, E_SWIGLU, 1, false, Shapes<true>::Large>(p, st)
-                      : launch<A_NORM, E_SWIGLU>(p, st);
+  return a_parts == 1 ? launch_shape<A_NORM, E_SWIGLU, 1, false, NormShapes::S4>(p, st)
+                      : launch_norm<E_SWIGLU>(p, st);
 }
 
 extern "C" int mdl_prefill_gemm_split_residual(const uint16_t* a, int64_t lda, int a_layout,
@@ -954,5 +1000,64 @@ extern "C" int mdl_prefill_gemm_norm_qkv(
   p.tok_row = token_row; p.tok_slot = token_slot; p.kv_start = kv_start;
   p.slots = cache_slots; p.seq = seq; p.batch = batch; p.lead = lead;
   p.M = m; p.N = 3 * d; p.K = d;
-  return launch<A_NORM, E_QKV>(p, static_cast<hipStream_t>(stream));
+  return launch_norm<E_QKV>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, float eps,
+                                          const uint16_t* w, const uint16_t* w_lo, float* out,
+                                          int64_t ldo, float* rstd_out, int m, int n, int k,
+                                          void* stream) {
+  int rc = check_common(w, m, n, k);
+  if (rc != MDL_OK) return rc;
+  if (!w_lo || !x || !gamma || !out) return MDL_ERR_NULL;
+  if (ldo < n || k > kMaxNormK) return MDL_ERR_SHAPE;
+  if (!aligned16(w_lo) || !aligned16(x) || !aligned16(gamma) || !aligned16(out) || ldo % 4 != 0)
+    return MDL_ERR_ALIGN;
+  if (m == 0) return MDL_OK;
+  if (m <= kK5Rows)
+    return mdl_gemm_norm(x, gamma, eps, w, w_lo, out, ldo, rstd_out, m, n, k, 0, stream);
+  Args p{};
+  p.x = x; p.gamma = gamma; p.eps = eps; p.w = w; p.wl = w_lo; p.out = out; p.ldo = ldo;
+  p.rstd_out = rstd_out; p.M = m; p.N = n; p.K = k;
+  return launch_f32w<E_STORE>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdl_prefill_gemm_norm_swiglu_f32w(const float* x, const float* gamma, float eps,
+                                                 const uint16_t* w_gu, const uint16_t* w_gu_lo,
+                                                 const float* bias_gate, const float* bias_up,
+                                                 uint16_t* h_out, int m, int d_ff, int k,
+                                                 void* stream) {
+  if (d_ff <= 0 || d_ff % 16 != 0 || d_ff > (1 << 28)) return MDL_ERR_SHAPE;
+  int rc = check_common(w_gu, m, 2 * d_ff, k);
+  if (rc != MDL_OK) return rc;
+  if (!w_gu_lo || !x || !gamma || !h_out) return MDL_ERR_NULL;
+  if (k > kMaxNormK) return MDL_ERR_SHAPE;
+  if (!aligned16(w_gu_lo) || !aligned16(x) || !aligned16(gamma) || !aligned8(h_out) ||
+      (bias_gate && !aligned16(bias_gate)) || (bias_up && !aligned16(bias_up)))
+    return MDL_ERR_ALIGN;
+  if (m == 0) return MDL_OK;
+  if (m <= kK5Rows)
+    return mdl_gemm_norm_swiglu(x, gamma, eps, w_gu, w_gu_lo, bias_gate, bias_up, h_out, m, d_ff,
+                                k, 0, stream);
+  Args p{};
+  p.x = x; p.gamma = gamma; p.eps = eps; p.w = w_gu; p.wl = w_gu_lo; p.bias_a = bias_gate;
+  p.bias_b = bias_up; p.h = h_out; p.d_ff = d_ff; p.h_parts = 2; p.M = m; p.N = 2 * d_ff; p.K = k;
+  return launch_f32w<E_SWIGLU>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdl_prefill_gemm_split_residual_f32w(const uint16_t* a, const uint16_t* w,
+                                                    const uint16_t* w_lo, float* x,
+                                                    const float* bias, int m, int n, int k,
+                                                    void* stream) {
+  int rc = check_common(w, m, n, k);
+  if (rc == MDL_OK) rc = check_a(a, 0, MDL_LAYOUT_TILES, 2, k);
+  if (rc != MDL_OK) return rc;
+  if (!w_lo || !x) return MDL_ERR_NULL;
+  if (n % 32 != 0) return MDL_ERR_SHAPE;   // x in the fp32 tile layout: whole 32-column blocks
+  if (!aligned16(w_lo) || !aligned16(x) || (bias && !aligned16(bias))) return MDL_ERR_ALIGN;
+  if (m == 0) return MDL_OK;
+  if (m <= kK5Rows) return mdl_gemm_split_residual(a, w, w_lo, x, bias, m, n, k, 0, stream);
+  Args p{};
+  p.a = a; p.w = w; p.wl = w_lo; p.x_res = x; p.bias_a = bias; p.M = m; p.N = n; p.K = k;
+  return launch_f32w<E_RESIDUAL>(p, static_cast<hipStream_t>(stream));
 }

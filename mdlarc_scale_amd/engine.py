@@ -58,7 +58,8 @@ Two forms, chosen by the model's parameter dtype as the reference chooses its ca
     attn = K4f(q, cache)                                         <- attn_prefill_f32 / decode_f32
     then the three K5 launches of the bf16 decode form, each with its w_lo.
 
-  The prompt's projections run on K5 too (K6 has no room in LDS for a second weight stage).
+  A prompt's projections are the same launches on K6 (its forms for fp32 weights; d_model over 2048
+  stays on K5).
 """
 
 from __future__ import annotations
@@ -221,6 +222,7 @@ class Scratch:
     tiled: bool = False
     fused: bool = False
     f32: bool = False
+    fused_f32: bool = False      # fp32 form of a prompt on K6
 
     @staticmethod
     def alloc(rows: int, d: int, d_ff: int, device: torch.device,
@@ -249,7 +251,9 @@ class Scratch:
         """Scratch of a prompt pass: the fp32 form, or the bf16 form on K6 when the model's
         shapes fit it (hipBLASLt otherwise)."""
         if f32:
-            return Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device, f32=True)
+            sc = Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device, f32=True)
+            sc.fused_f32 = prompt_gemms_fused(cfg.d_model, cfg.d_ff)
+            return sc
         return Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device,
                              fused=prompt_gemms_fused(cfg.d_model, cfg.d_ff))
 
@@ -395,10 +399,9 @@ class HipEngine:
         for li in range(cfg.n_layers):
             kc, vc = kv_layers(li)
             if sc.f32:
-                # fp32 form: projection on K5 with the low weight part, K2 into the fp32 cache,
-                # K4f (the attention is exact, so no lead pass)
-                K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
-                            w_lo=W.qkv_lo[li])
+                # fp32 form: projection with the low weight part, K2 into the fp32 cache, K4f (the
+                # attention is exact, so no lead pass)
+                self._qkv_f32(W, li, sc)
                 K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
                                  sc.q, kc, vc, slot0=0)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, None, B * S,
@@ -450,8 +453,7 @@ class HipEngine:
         for li in range(cfg.n_layers):
             kc, vc = kv_layers(li)
             if sc.f32:   # fp32 form (see run_prompt)
-                K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
-                            w_lo=W.qkv_lo[li])
+                self._qkv_f32(W, li, sc)
                 K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
                                         pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, pk.q_offset,
@@ -475,6 +477,17 @@ class HipEngine:
                                 out_tiled=fused)
             self._mlp(W, li, sc)
 
+    @staticmethod
+    def _qkv_f32(W: PackedWeights, li: int, sc: Scratch) -> None:
+        """ln1 + qkv_proj of a prompt in the fp32 form: the fp32 projection rows and rstd."""
+        k = W.ln1[li].numel()
+        if sc.fused_f32:
+            K.prefill_gemm_norm_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li], W.qkv_lo[li], sc.qkv,
+                                     sc.rstd, k)
+        else:
+            K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, k,
+                        w_lo=W.qkv_lo[li])
+
     def _mlp(self, W: PackedWeights, li: int, sc: Scratch) -> None:
         """out_proj + residual, ln2, SwiGLU MLP + residual, next norm (shared by both phases)."""
         cfg = self.cfg
@@ -491,6 +504,14 @@ class HipEngine:
                                        h_parts=parts)
             K.prefill_gemm_split_residual(sc.h, W.down_t[li], sc.x, W.b_down[li], m, d, F,
                                           a_tiled=True, a_parts=parts)
+            return
+        if sc.fused_f32:
+            K.prefill_gemm_split_residual_f32w(sc.attn, W.out_t[li], W.out_lo[li], sc.x, None,
+                                               sc.rows, d, d)
+            K.prefill_gemm_norm_swiglu_f32w(sc.x, W.ln2[li], W.eps, W.gu_t[li], W.gu_lo[li],
+                                            W.b_gate[li], W.b_up[li], sc.h, sc.rows, F, d)
+            K.prefill_gemm_split_residual_f32w(sc.h, W.down_t[li], W.down_lo[li], sc.x,
+                                               W.b_down[li], sc.rows, d, F)
             return
         if sc.tiled:
             # decode: three K5 launches, the residual adds in the epilogues and ln2 in the

@@ -485,6 +485,53 @@ def prefill_gemm_norm(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch
                                                 _stream()), "mdl_prefill_gemm_norm")
 
 
+def prefill_gemm_norm_f32w(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor,
+                           w_lo: torch.Tensor, out: torch.Tensor, rstd_out: torch.Tensor | None,
+                           k: int) -> None:
+    """prefill_gemm_norm of an fp32 weight given as its high and low bf16 parts (both tiled)."""
+    _need(out, "out", F32)
+    m, n = out.shape
+    _need(x, "x", F32, tile_rows(m) * k)
+    _need(gamma, "gamma", F32, k)
+    _need(w, "w", BF16, tile_rows(n) * k)
+    _need(w_lo, "w_lo", BF16, tile_rows(n) * k)
+    _need(rstd_out, "rstd_out", F32, m, optional=True)
+    _lib.check(_lib.lib().mdl_prefill_gemm_norm_f32w(
+        _p(x), _p(gamma), eps, _p(w), _p(w_lo), _p(out), out.stride(0), _p(rstd_out), m, n, k,
+        _stream()), "mdl_prefill_gemm_norm_f32w")
+
+
+def prefill_gemm_norm_swiglu_f32w(x: torch.Tensor, gamma: torch.Tensor, eps: float,
+                                  w_gu: torch.Tensor, w_gu_lo: torch.Tensor,
+                                  bias_gate: torch.Tensor | None, bias_up: torch.Tensor | None,
+                                  h_out: torch.Tensor, m: int, d_ff: int, k: int) -> None:
+    """prefill_gemm_norm_swiglu (split h) of an fp32 weight given as its high and low parts."""
+    _need(x, "x", F32, tile_rows(m) * k)
+    _need(gamma, "gamma", F32, k)
+    _need(w_gu, "w_gu", BF16, 2 * d_ff * k)
+    _need(w_gu_lo, "w_gu_lo", BF16, 2 * d_ff * k)
+    _need(bias_gate, "bias_gate", F32, d_ff, optional=True)
+    _need(bias_up, "bias_up", F32, d_ff, optional=True)
+    _need(h_out, "h_out", BF16, split_numel(m, d_ff, True))
+    _lib.check(_lib.lib().mdl_prefill_gemm_norm_swiglu_f32w(
+        _p(x), _p(gamma), eps, _p(w_gu), _p(w_gu_lo), _p(bias_gate), _p(bias_up), _p(h_out), m,
+        d_ff, k, _stream()), "mdl_prefill_gemm_norm_swiglu_f32w")
+
+
+def prefill_gemm_split_residual_f32w(a: torch.Tensor, w: torch.Tensor, w_lo: torch.Tensor,
+                                     x: torch.Tensor, bias: torch.Tensor | None, m: int, n: int,
+                                     k: int) -> None:
+    """prefill_gemm_split_residual (tiled a) of an fp32 weight given as its high and low parts."""
+    _need(a, "a", BF16, tile_rows(m) * 2 * k)
+    _need(x, "x", F32, tile_rows(m) * n)
+    _need(w, "w", BF16, tile_rows(n) * k)
+    _need(w_lo, "w_lo", BF16, tile_rows(n) * k)
+    _need(bias, "bias", F32, n, optional=True)
+    _lib.check(_lib.lib().mdl_prefill_gemm_split_residual_f32w(
+        _p(a), _p(w), _p(w_lo), _p(x), _p(bias), m, n, k, _stream()),
+        "mdl_prefill_gemm_split_residual_f32w")
+
+
 def prefill_gemm_norm_swiglu(x: torch.Tensor, gamma: torch.Tensor, eps: float,
                              w_gu: torch.Tensor, bias_gate: torch.Tensor | None,
                              bias_up: torch.Tensor | None, h_out: torch.Tensor, m: int,

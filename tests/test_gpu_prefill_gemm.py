@@ -382,3 +382,49 @@ def test_norm_qkv_at_each_block_shape(m):
                               geom, 0.125, q2, kc2, vc2, seq=m)
     for got, want in ((rs2, rs1), (q2, q1), (kc2, kc1), (vc2, vc1), (lead[:64], qkv[:64])):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("k", [256, 768, 1952, 2048])
+def test_fp32_weight_forms(k):
+    """The fp32-weight forms: a large product against fp64 of the products they form, a_hi w +
+    a_lo w + a_hi w_lo (fp32 sums: 2e-6, as above), and every row count past K5's 640 rows, at the
+    edges of the tiles and in each block shape, the same bits as those rows of the large product."""
+    f, n, total = 704, 768, 20_000
+    g = torch.Generator(DEV).manual_seed(k)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    wg, wo = 0.05 * rnd(2 * f, k), 0.05 * rnd(n, k)
+    (wg_h, wg_l), (wo_h, wo_l) = split(wg), split(wo)
+    tiles = [K().tile_matrix(t) for t in (wg_h, wg_l, wo_h, wo_l)]
+    x, gam, bias, res = rnd(total, k), 1 + 0.1 * rnd(k), rnd(f), rnd(total, n)
+    hi, lo = split(rnd(total, k))
+    a = torch.cat([hi, lo], 1).contiguous()
+
+    def forms(m):
+        xt, at = K().tile_f32(x[:m]), K().tile_matrix(a[:m].contiguous())
+        store, rs = torch.empty(m, 2 * f, device=DEV), torch.empty(m, device=DEV)
+        K().prefill_gemm_norm_f32w(xt, gam, 1e-5, tiles[0], tiles[1], store, rs, k)
+        h = torch.empty(K().split_numel(m, f, True), dtype=torch.bfloat16, device=DEV)
+        K().prefill_gemm_norm_swiglu_f32w(xt, gam, 1e-5, tiles[0], tiles[1], bias, None, h, m, f,
+                                          k)
+        xr = K().tile_f32(res[:m])
+        K().prefill_gemm_split_residual_f32w(at, tiles[2], tiles[3], xr, None, m, n, k)
+        return store, rs, K().untile_matrix(h, m, 2 * f), K().untile_f32(xr, m, n)
+
+    whole = forms(total)
+    th, tl = split(x * gam)
+    d = torch.Tensor.double
+    acc = (d(th) + d(tl)) @ d(wg_h).T + d(th) @ d(wg_l).T
+    assert rel(whole[0], acc) < 2e-6
+    ref = d(res) + (d(hi) + d(lo)) @ d(wo_h).T + d(hi) @ d(wo_l).T
+    assert rel(whole[3], ref) < 2e-6
+    blocks = (acc / torch.sqrt((d(x) ** 2).mean(1, keepdim=True) + 1e-5)).view(total, -1, 2, 16)
+    gate = blocks[:, :, 0].reshape(total, f) + d(bias)
+    ref = torch.nn.functional.silu(gate) * blocks[:, :, 1].reshape(total, f)
+    h = d(whole[2])
+    assert rel(h[:, :f] + h[:, f:], ref) < 2e-5          # as the bf16 form's: the split of h
+    for m in (641, 703, 1025, 1500, 3000, 4097, 8193):
+        for name, got, want in zip(("store", "rstd", "swiglu", "residual"), forms(m), whole):
+            assert torch.equal(got, want[:m]), f"{name} at {m} rows"
+    m = 640                                              # on K5: another order of the sums
+    store = forms(m)[0]
+    assert rel(store, acc[:m]) < 2e-6

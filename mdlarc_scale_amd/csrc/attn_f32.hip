@@ -7,12 +7,12 @@
 // scores and probabilities stay fp32, and only the output is stored as the split (hi|lo bf16)
 // input of the out projection, which carries it to ~2^-17.
 //
-// Work item: 16 consecutive query positions of one (batch row, head).  One wave per item, four
-// independent waves per block; no LDS and no barrier.  Lane l = (c, g), c = l % 16, g = l / 16.
+// A wave computes 16 consecutive query positions of one (batch row, head) against 16 keys at a
+// time.  Lane l = (c, g), c = l % 16, g = l / 16:
 //
 //   S^T = K . Q^T   16 keys x 16 queries, 16 MFMAs of k = 4.  MFMA kb pairs lane group g's
 //                   A element K[key c][16 g + kb] with its B element q[query c][16 g + kb], so a
-//                   lane loads dims 16 g .. 16 g + 15 of one key row and of one query row: four
+//                   lane holds dims 16 g .. 16 g + 15 of one key row and of one query row: four
 //                   float4 each.  The accumulator of lane (c, g) holds S^T[keys 4 g .. 4 g + 3]
 //                   [query c].
 //   softmax         per query column c over the four lane groups (base 2: q carries the softmax
@@ -20,7 +20,7 @@
 //   O^T = V^T . P^T 64 dims x 16 queries as 4 dim blocks x 4 key steps.  Key step r pairs lane
 //                   group g's B element P^T[key 4 g + r][query c] -- accumulator element r of
 //                   the score MFMA, no data movement -- with A element V[key 4 g + r][4 c + db] of
-//                   dim block db, so a lane loads one float4 (dims 4 c .. 4 c + 3) per key step.
+//                   dim block db, so a lane holds one float4 (dims 4 c .. 4 c + 3) per key step.
 //                   Row i of dim block db's accumulator is dim 4 i + db, so lane (c, g) ends
 //                   with dims 16 g .. 16 g + 15 of query c (element r of block db = dim
 //                   16 g + 4 r + db).
@@ -30,21 +30,32 @@
 // per batch row at cache slot t).  Key j is visible to the query at position i iff
 // kv_start[b] <= j < n_keys, (causal) j <= i, and (j >= mask_len or mask[b * mask_len + j] != 0);
 // a query with no visible key outputs 0 (what torch's CPU SDPA returns for an all -inf row).
-// At decode a work item is one split_len-slot chunk of one (row, head): one wave streaming its
-// keys a 16-key tile at a time is latency-bound, so the chunks are what fills the GPU.  With
-// several chunks each writes its running state (m, l, unnormalised o) to the workspace, and
+//
+// Prefill (attn_f32_prefill_kernel): a block of four waves takes 64 queries, and key tiles of 32
+// go through a ring of two LDS stages (K and V, 8 KB each) filled by direct global -> LDS copies,
+// the next tile's while this one is worked on; one barrier per tile.  The 16-byte chunks of a
+// 256-byte row are XOR-swizzled with the row's low four bits, so both reads (16 rows of one chunk;
+// four whole rows) touch every bank once.  What bounds it is the fp32 matrix rate (154 TFLOP/s in
+// a large product on this card).  A wave that loaded its own 16 queries' keys from L2 waited for
+// every tile and moved four times the bytes: 16 rows of up to 811 tokens and 12 heads @F32A@.
+//
+// Decode (attn_f32_decode_kernel): a work item is one split_len-slot chunk of one (row, head), a
+// wave of its own without LDS or barriers; the chunks are what fills the GPU.  With several chunks
+// each writes its running state (m, l, unnormalised o) to the workspace, and
 // attn_f32_combine_kernel merges them.
 #include "common.h"
+#include "lds_dma.h"
 #include "mfma.h"
 
 namespace mdl {
 
 namespace {
 
-constexpr int kQT = 16;          // queries per work item
-constexpr int kWavesF = 4;       // independent waves per block
-
-enum Mode { M_PADDED = 0, M_PACKED = 1, M_DECODE = 2 };
+constexpr int kQT = 16;          // queries of a wave
+constexpr int kWavesF = 4;       // waves per block
+constexpr int kQB = kQT * kWavesF;   // prefill: queries of a block
+constexpr int kKT = 32;              // prefill: keys of a tile
+constexpr int kTileF = kKT * kHeadDim * 4;   // bytes of a K or V tile
 
 struct F32Args {
   const float* q;                // [rows, H, 64], pre-scaled (softmax scale * log2(e))
@@ -53,87 +64,225 @@ struct F32Args {
   const uint8_t* mask;           // [batch, mask_len] or NULL
   int mask_len;
   const int32_t* kv_start;       // [batch] or NULL (0)
-  const int32_t* q_offset;       // M_PACKED: [batch]
-  const int32_t* seq_dev;        // M_DECODE: slot of the query (NULL: seq_pos)
+  const int32_t* q_offset;       // packed prefill: [batch]
+  const int32_t* seq_dev;        // decode: slot of the query (NULL: seq_pos)
   int seq_pos;
   int batch, heads, slots, seq;  // seq: prefill query / key count
   int causal;
-  int q_tiles;                   // work items per (row, head) (M_DECODE: the chunks)
-  int64_t items;
+  int q_tiles;                   // work items per (row, head): query blocks, or decode chunks
+  int64_t items;                 // decode: chunks; prefill: (row, head) pairs
   uint16_t* out;                 // split bf16 [rows, 2 d]
   int out_layout;
-  int split_len;                 // M_DECODE: slots per chunk
-  float* ws;                     // M_DECODE with more than one chunk: kPartF floats per chunk
+  int split_len;                 // decode: slots per chunk
+  float* ws;                     // decode with more than one chunk: kPartF floats per chunk
 };
 
 constexpr int kPartF = 2 + kHeadDim;   // m, l, o[64] of one decode chunk
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int MODE>
-__global__ __launch_bounds__(64 * kWavesF) void attn_f32_kernel(const F32Args p) {
+__device__ __forceinline__ void load16(const float* p, float* v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 t = *reinterpret_cast<const float4*>(p + 4 * i);
+    v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+  }
+}
+
+// o / l of query c as the split output of row qrow: lane (c, g) holds dims 16 g + 4 r + db as
+// element r of block db
+__device__ __forceinline__ void store_out(const F32Args& p, int64_t qrow, int h, int g, float l,
+                                          const f32x4 (&o)[4]) {
+  const int d = p.heads * kHeadDim;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  float res[16];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int db = 0; db < 4; ++db) res[4 * r + db] = o[db][r] * inv;
+  uint4 hi0, lo0, hi1, lo1;
+  split8(res, hi0, lo0);
+  split8(res + 8, hi1, lo1);
+  const int col = h * kHeadDim + 16 * g;
+  if (p.out_layout == MDL_LAYOUT_TILES) {
+    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, col, 2 * d)) = hi0;
+    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, col + 8, 2 * d)) = hi1;
+    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, d + col, 2 * d)) = lo0;
+    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, d + col + 8, 2 * d)) = lo1;
+  } else {
+    uint16_t* orow = p.out + qrow * 2 * d;
+    *reinterpret_cast<uint4*>(orow + col) = hi0;
+    *reinterpret_cast<uint4*>(orow + col + 8) = hi1;
+    *reinterpret_cast<uint4*>(orow + d + col) = lo0;
+    *reinterpret_cast<uint4*>(orow + d + col + 8) = lo1;
+  }
+}
+
+// Blocks: (row, head) pair i % 8 + 8 j on XCD i % 8, its latest (longest) query block first.
+__global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const F32Args p) {
+  const int slot = blockIdx.x >> 3;
+  const int pair = slot / p.q_tiles;
+  const int bh = (blockIdx.x & 7) + 8 * pair;
+  if (bh >= p.items) return;   // pairs padded to a multiple of 8: whole blocks exit
+  const int qt = p.q_tiles - 1 - (slot - pair * p.q_tiles);
+  const int b = bh / p.heads, h = bh - b * p.heads;
+  const int S = p.seq;
+  const int kstart = p.kv_start ? min(max(p.kv_start[b], 0), S) : 0;
+  // packed rows: queries from kstart on, query i at row q_offset[b] + i - kstart
+  const int q0 = (p.q_offset ? kstart : 0) + kQB * qt;
+  if (q0 >= S) return;         // the whole block lies past the row
+  const int64_t qbase = p.q_offset ? static_cast<int64_t>(p.q_offset[b]) - kstart
+                                   : static_cast<int64_t>(b) * S;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wq0 = q0 + kQT * wave;
+  const int qi = wq0 + c;
+  const int64_t qrow = qbase + min(qi, S - 1);
+
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][kTileF];   // [stage][K, V]
+  const int64_t head = (static_cast<int64_t>(b) * p.heads + h) * p.slots * kHeadDim;
+  const float* K = p.kc + head;
+  const float* V = p.vc + head;
+  const uint8_t* mrow = p.mask ? p.mask + static_cast<int64_t>(b) * p.mask_len : nullptr;
+  // a row without a valid key attends to nothing
+  const int kend = kstart >= S ? kstart : (p.causal ? min(S, q0 + kQB) : S);
+
+  float qv[16];
+  load16(p.q + (qrow * p.heads + h) * kHeadDim + 16 * g, qv);
+
+  // Tile kt -> stage st: wave w copies key rows 16 j + 4 w .. + 3 of K and V (j = 0, 1), one
+  // kilobyte each; lane l takes physical chunk l % 16 of its row, i.e. logical chunk
+  // (l % 16) ^ (row % 16).  Rows past S copy the last key (their weights are 0).
+  const uint32_t lds0 = lds_addr(lds);
+  auto issue = [&](int kt, int st) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = 16 * j + 4 * wave + (lane >> 4);
+      const uint32_t off = min(row, S - 1 - kt) * (kHeadDim * 4) + 16 * (c ^ (row & 15));
+      const uint32_t dst = lds0 + 2 * st * kTileF + (16 * j + 4 * wave) * 256;
+      const int64_t tile = static_cast<int64_t>(kt) * kHeadDim;
+      dma16_sbase(K + tile, off, __builtin_amdgcn_readfirstlane(dst));
+      dma16_sbase(V + tile, off, __builtin_amdgcn_readfirstlane(dst + kTileF));
+    }
+  };
+  // lanes 0 .. 31: this lane's key of tile kt is valid (inside the row and not masked)
+  auto key_ok = [&](int kt) -> int {
+    const int j = kt + (lane & 31);
+    if (j >= S) return 0;
+    return mrow && j < p.mask_len ? mrow[j] : 1;
+  };
+
+  float m = -INFINITY, l = 0.f;   // l: this lane group's part of the sum
+  f32x4 o[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  int ok_next = 0;
+  if (kstart < kend) {
+    ok_next = key_ok(kstart);
+    issue(kstart, 0);
+  }
+  // every wave of the block runs the same tiles, so the barriers match
+  for (int kt = kstart, st = 0; kt < kend; kt += kKT, st ^= 1) {
+    // tile kt has landed for every wave, and every wave is done with the other stage (the builtin
+    // wait, so that the compiler counts its own loads, q and the mask bytes, as landed too)
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
+    asm volatile("s_barrier" ::: "memory");
+    const uint32_t valid = static_cast<uint32_t>(__ballot(ok_next != 0));
+    if (kt + kKT < kend) {
+      ok_next = key_ok(kt + kKT);
+      issue(kt + kKT, st ^ 1);
+    }
+    if (p.causal && kt > wq0 + kQT - 1) continue;   // the whole tile is in this wave's future
+    const uint8_t* Kt = lds[st][0];
+    const uint8_t* Vt = lds[st][1];
+    f32x4 s[2];
+    float kv[2][16];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      s[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 t = *reinterpret_cast<const float4*>(Kt + (16 * nb + c) * 256 +
+                                                          16 * ((4 * g + i) ^ c));
+        kv[nb][4 * i] = t.x; kv[nb][4 * i + 1] = t.y;
+        kv[nb][4 * i + 2] = t.z; kv[nb][4 * i + 3] = t.w;
+      }
+    }
+#pragma unroll
+    for (int kb = 0; kb < 16; ++kb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+        s[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[nb][kb], qv[kb], s[nb], 0, 0, 0);
+    if (valid != ~0u || (p.causal && kt + kKT - 1 > wq0)) {
+      uint32_t vis = valid;
+      if (p.causal) {
+        const int x = qi - kt;   // offset of the last key query qi may see
+        vis &= x >= 31 ? ~0u : (x < 0 ? 0u : (2u << x) - 1u);
+      }
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!((vis >> (16 * nb + 4 * g + r)) & 1u)) s[nb][r] = -INFINITY;
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[nb][r]);
+    const float m_new = fmaxf(m, max_over_groups(tmax));
+    const float base = m_new == -INFINITY ? 0.f : m_new;   // no visible key yet: weights 0
+    const float alpha = __builtin_amdgcn_exp2f(m - base);
+    m = m_new;
+    float psum = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[nb][r] = __builtin_amdgcn_exp2f(s[nb][r] - base);
+        psum += s[nb][r];
+      }
+    l = fmaf(l, alpha, psum);
+#pragma unroll
+    for (int db = 0; db < 4; ++db) o[db] *= alpha;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * nb + 4 * g + r;
+        const float4 v = *reinterpret_cast<const float4*>(Vt + row * 256 + 16 * (c ^ (row & 15)));
+        const float ve[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+          o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[db], 0, 0, 0);
+      }
+  }
+  if (qi >= S) return;
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  store_out(p, qrow, h, g, l, o);
+}
+
+__global__ __launch_bounds__(64 * kWavesF) void attn_f32_decode_kernel(const F32Args p) {
   const int64_t item = static_cast<int64_t>(blockIdx.x) * kWavesF + (threadIdx.x >> 6);
   if (item >= p.items) return;   // whole wave; the kernel has no barrier
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int64_t bh = item / p.q_tiles;
-  // the longest query tiles of a row first (causal prefill: the last tiles see the most keys);
-  // at decode, the chunk index
-  const int qt = p.q_tiles - 1 - static_cast<int>(item - bh * p.q_tiles);
+  const int chunk = p.q_tiles - 1 - static_cast<int>(item - bh * p.q_tiles);
   const int b = static_cast<int>(bh / p.heads), h = static_cast<int>(bh - b * p.heads);
-  const int d = p.heads * kHeadDim;
+  const int t = p.seq_dev ? *p.seq_dev : p.seq_pos;
+  const int n_keys = min(t + 1, p.slots);
+  int klo = p.kv_start ? min(max(p.kv_start[b], 0), n_keys) : 0;
+  klo = min(klo + chunk * p.split_len, n_keys);
+  const int khi = min(klo + p.split_len, n_keys);   // slots of this chunk: [klo, khi)
 
-  // key range [klo, n_keys) and this lane's query position / output row
-  int n_keys, klo = 0;
-  if constexpr (MODE == M_DECODE) {
-    const int t = p.seq_dev ? *p.seq_dev : p.seq_pos;
-    n_keys = min(t + 1, p.slots);
-  } else {
-    n_keys = p.seq;
-  }
-  if (p.kv_start) klo = min(max(p.kv_start[b], 0), n_keys);
-  int khi = n_keys;   // keys this item visits: [klo, khi)
-  if constexpr (MODE == M_DECODE) {
-    klo = min(klo + qt * p.split_len, n_keys);
-    khi = min(klo + p.split_len, n_keys);
-  }
-  int qpos, qfirst;   // this lane's query position; the tile's first position
-  int64_t qrow;
-  bool qvalid;
-  if constexpr (MODE == M_DECODE) {
-    qfirst = qpos = n_keys - 1;
-    qvalid = c == 0;
-    qrow = b;
-  } else if constexpr (MODE == M_PACKED) {
-    qfirst = klo + kQT * qt;
-    qpos = qfirst + c;
-    qvalid = qpos < p.seq;
-    qrow = static_cast<int64_t>(p.q_offset[b]) + (qvalid ? qpos : qfirst) - klo;
-  } else {
-    qfirst = kQT * qt;
-    qpos = qfirst + c;
-    qvalid = qpos < p.seq;
-    qrow = static_cast<int64_t>(b) * p.seq + (qvalid ? qpos : qfirst);
-  }
-  if (qfirst >= p.seq && MODE != M_DECODE) return;   // the whole tile lies past the row
-  // keys the tile's last query can see
-  if (p.causal && MODE != M_DECODE) khi = min(n_keys, min(qfirst + kQT, p.seq));
-
-  // q: dims 16 g .. 16 g + 15 of query c
-  float qv[16];
-  {
-    const float* qp = p.q + (qrow * p.heads + h) * kHeadDim + 16 * g;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 v = *reinterpret_cast<const float4*>(qp + 4 * i);
-      qv[4 * i] = v.x; qv[4 * i + 1] = v.y; qv[4 * i + 2] = v.z; qv[4 * i + 3] = v.w;
-    }
-  }
-  const int64_t head_base = (static_cast<int64_t>(b) * p.heads + h) * p.slots * kHeadDim;
-  const float* K = p.kc + head_base;
-  const float* V = p.vc + head_base;
+  float qv[16];   // dims 16 g .. 16 g + 15 of the query, the same in every column
+  load16(p.q + (static_cast<int64_t>(b) * p.heads + h) * kHeadDim + 16 * g, qv);
+  const int64_t head = (static_cast<int64_t>(b) * p.heads + h) * p.slots * kHeadDim;
+  const float* K = p.kc + head;
+  const float* V = p.vc + head;
   const uint8_t* mrow = p.mask ? p.mask + static_cast<int64_t>(b) * p.mask_len : nullptr;
-  const int qlim = (p.causal || MODE == M_DECODE) ? qpos : n_keys - 1;   // last key for query c
-
   float m_run = -INFINITY, l_run = 0.f;
   f32x4 o[4];
 #pragma unroll
@@ -164,7 +313,7 @@ __global__ __launch_bounds__(64 * kWavesF) void attn_f32_kernel(const F32Args p)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int j = k0 + 4 * g + r;
-      bool ok = qvalid && j < khi && j <= qlim;
+      bool ok = c == 0 && j < khi;
       if (ok && mrow && j < p.mask_len) ok = mrow[j] != 0;
       sv[r] = ok ? s[r] : -INFINITY;
       tmax = fmaxf(tmax, sv[r]);
@@ -199,10 +348,9 @@ __global__ __launch_bounds__(64 * kWavesF) void attn_f32_kernel(const F32Args p)
     }
   }
 
-  if (!qvalid) return;
-  if (MODE == M_DECODE && p.ws) {
-    // this chunk's state: m and l (the same in every lane of query column 0), o unnormalised;
-    // lane (0, g) holds dims 16 g + 4 r + db as element r of block db
+  if (c != 0) return;
+  if (p.ws) {
+    // this chunk's state: m and l (the same in every lane of query column 0), o unnormalised
     float* part = p.ws + item * kPartF;
     if (g == 0) {
       part[0] = m_run;
@@ -214,30 +362,8 @@ __global__ __launch_bounds__(64 * kWavesF) void attn_f32_kernel(const F32Args p)
       for (int db = 0; db < 4; ++db) part[2 + 16 * g + 4 * r + db] = o[db][r];
     return;
   }
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  float res[16];   // dims 16 g + e of query c: element r of block db is dim 16 g + 4 r + db
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int db = 0; db < 4; ++db) res[4 * r + db] = o[db][r] * inv;
-  uint4 hi0, lo0, hi1, lo1;
-  split8(res, hi0, lo0);
-  split8(res + 8, hi1, lo1);
-  const int col = h * kHeadDim + 16 * g;
-  if (p.out_layout == MDL_LAYOUT_TILES) {
-    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, col, 2 * d)) = hi0;
-    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, col + 8, 2 * d)) = hi1;
-    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, d + col, 2 * d)) = lo0;
-    *reinterpret_cast<uint4*>(p.out + tile_off(qrow, d + col + 8, 2 * d)) = lo1;
-  } else {
-    uint16_t* orow = p.out + qrow * 2 * d;
-    *reinterpret_cast<uint4*>(orow + col) = hi0;
-    *reinterpret_cast<uint4*>(orow + col + 8) = hi1;
-    *reinterpret_cast<uint4*>(orow + d + col) = lo0;
-    *reinterpret_cast<uint4*>(orow + d + col + 8) = lo1;
-  }
+  store_out(p, b, h, g, l_run, o);
 }
-
 // The decode chunks of one (row, head) merged, lane = channel: the states rescaled to their
 // largest m (base 2), o / l, stored as the split output of mdl_attn_decode_f32.
 __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __restrict__ ws,
@@ -270,16 +396,6 @@ __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __re
     out[static_cast<int64_t>(b) * 2 * d + col] = hi;
     out[static_cast<int64_t>(b) * 2 * d + d + col] = lo;
   }
-}
-
-template <int MODE>
-int launch_f32(F32Args p, hipStream_t st) {
-  if (p.items == 0) return MDL_OK;
-  const int64_t blocks = (p.items + kWavesF - 1) / kWavesF;
-  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
-  hipLaunchKernelGGL(attn_f32_kernel<MODE>, dim3(static_cast<unsigned>(blocks)),
-                     dim3(64 * kWavesF), 0, st, p);
-  return launch_status();
 }
 
 int check_f32(const float* q, const float* k_cache, const float* v_cache, int batch,
@@ -317,11 +433,15 @@ extern "C" int mdl_attn_prefill_f32(const float* q, const float* k_cache, const 
   p.kv_start = kv_start; p.q_offset = q_offset;
   p.batch = batch; p.heads = n_heads; p.slots = cache_slots; p.seq = seq;
   p.causal = causal != 0;
-  p.q_tiles = (seq + kQT - 1) / kQT;
-  p.items = static_cast<int64_t>(batch) * n_heads * p.q_tiles;
+  p.q_tiles = (seq + kQB - 1) / kQB;
+  p.items = static_cast<int64_t>(batch) * n_heads;
   p.out = out; p.out_layout = out_layout;
-  auto st = static_cast<hipStream_t>(stream);
-  return q_offset ? launch_f32<M_PACKED>(p, st) : launch_f32<M_PADDED>(p, st);
+  if (p.items == 0) return MDL_OK;
+  const int64_t blocks = (p.items + 7) / 8 * 8 * p.q_tiles;
+  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
+  hipLaunchKernelGGL(attn_f32_prefill_kernel, dim3(static_cast<unsigned>(blocks)),
+                     dim3(64 * kWavesF), 0, static_cast<hipStream_t>(stream), p);
+  return launch_status();
 }
 
 extern "C" int mdl_attn_decode_f32(const float* q, const float* k_cache, const float* v_cache,
@@ -358,8 +478,13 @@ extern "C" int mdl_attn_decode_f32(const float* q, const float* k_cache, const f
   p.items = n_bh * n_split;
   p.out = out; p.out_layout = out_layout;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  const int rc2 = launch_f32<M_DECODE>(p, st);
-  if (rc2 != MDL_OK || n_split == 1 || n_bh == 0) return rc2;
+  if (p.items == 0) return MDL_OK;
+  const int64_t blocks = (p.items + kWavesF - 1) / kWavesF;
+  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
+  hipLaunchKernelGGL(attn_f32_decode_kernel, dim3(static_cast<unsigned>(blocks)),
+                     dim3(64 * kWavesF), 0, st, p);
+  const int rc2 = launch_status();
+  if (rc2 != MDL_OK || n_split == 1) return rc2;
   if ((n_bh + 3) / 4 > 0x7fffffff) return MDL_ERR_SHAPE;
   hipLaunchKernelGGL(attn_f32_combine_kernel, dim3(static_cast<unsigned>((n_bh + 3) / 4)),
                      dim3(256), 0, st, workspace, static_cast<int>(n_bh), n_heads, n_split, out,

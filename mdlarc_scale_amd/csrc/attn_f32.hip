@@ -37,7 +37,8 @@
 // 256-byte row are XOR-swizzled with the row's low four bits, so both reads (16 rows of one chunk;
 // four whole rows) touch every bank once.  What bounds it is the fp32 matrix rate (154 TFLOP/s in
 // a large product on this card).  A wave that loaded its own 16 queries' keys from L2 waited for
-// every tile and moved four times the bytes: 16 rows of up to 811 tokens and 12 heads @F32A@.
+// every tile and moved four times the bytes: 16 rows of up to 811 tokens and 12 heads
+// 271 -> 178 us (92 us of MFMAs), 8 of up to 1,001 and 4 heads 126 -> 61.
 //
 // Decode (attn_f32_decode_kernel): a work item is one split_len-slot chunk of one (row, head), a
 // wave of its own without LDS or barriers; the chunks are what fills the GPU.  With several chunks
@@ -118,13 +119,14 @@ __device__ __forceinline__ void store_out(const F32Args& p, int64_t qrow, int h,
   }
 }
 
-// Blocks: (row, head) pair i % 8 + 8 j on XCD i % 8, its latest (longest) query block first.
+// Blocks: (row, head) pair i % 8 + 8 j on XCD i % 8, the latest (longest) query block of every pair
+// first, so that the short ones fill the end of the launch (pair by pair, the last pair's longest
+// blocks ran on alone: 213 -> 178 us).
 __global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const F32Args p) {
-  const int slot = blockIdx.x >> 3;
-  const int pair = slot / p.q_tiles;
-  const int bh = (blockIdx.x & 7) + 8 * pair;
+  const int slot = blockIdx.x >> 3, pairs = gridDim.x / (8 * p.q_tiles);   // pairs of an XCD
+  const int qt = p.q_tiles - 1 - slot / pairs;
+  const int bh = (blockIdx.x & 7) + 8 * (slot % pairs);
   if (bh >= p.items) return;   // pairs padded to a multiple of 8: whole blocks exit
-  const int qt = p.q_tiles - 1 - (slot - pair * p.q_tiles);
   const int b = bh / p.heads, h = bh - b * p.heads;
   const int S = p.seq;
   const int kstart = p.kv_start ? min(max(p.kv_start[b], 0), S) : 0;

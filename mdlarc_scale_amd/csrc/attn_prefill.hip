@@ -383,15 +383,15 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
 // Those queries see only keys among the same kLead tokens (causal), so one block holds them all
 // in LDS.  Later queries average over more than kLead keys and keep K4a's output.
 //
-// Block = one (b, h), 256 threads: thread t owns query t/4 and dims 16 (t%4) .. +15.  It first
-// rotates those dims of its own token's q (kept in registers) and k (to LDS) -- RoPE pairs
-// 8 (t%4) .. +7 -- and scales its v dims (to LDS).  Then, with K and V rows read as float4, one
-// pass over the visible keys keeps the online softmax in fp32: the running maximum, and the sum
-// and P V rescaled by exp(m_old - m_new) whenever a score passes it (measured against a pass
-// for the maximum and a second for the sums: 142 -> 103 us at config 2's shape, together with
-// the four-way dot product and the positions loaded once).  Each dot product is four partial
-// sums, added, then summed over the query's 4 threads with 2 xor shuffles.  A wave's loop stops
-// at the wave's last query (keys after it are in every query's future).
+// Block = one (b, h), four waves; wave w owns the 16 queries 16 w .. and lane (c, g) of it
+// (c = lane % 16, g = lane / 16) query 16 w + c and dims 16 g .. + 15: it rotates those dims of
+// its token's q (kept in registers) and k (to LDS) -- RoPE pairs 8 g .. + 7 -- and scales its v
+// dims (to LDS).  Then S^T = K Q^T and O^T = V^T P^T on fp32 MFMA (v_mfma_f32_16x16x4_f32) with the
+// operand layouts of K4f (attn_f32.hip): the probabilities never leave registers, and with all
+// scores of a query at hand its softmax takes one maximum and one sum.  A wave needs the key
+// blocks up to its own only.  One thread a query and a loop over its keys, a dot product with two
+// shuffles and an exponential for each, was a chain of 64 such steps: 12 (row,
+// head) pairs 29 -> 10 us, 3,072 of them 121 -> 66 us.
 constexpr int kLead = 64;
 constexpr int kLeadLd = kHeadDim + 4;   // LDS row stride (floats): 16-byte aligned rows
 
@@ -412,29 +412,33 @@ __global__ __launch_bounds__(256) void attn_lead_kernel(
   __shared__ __attribute__((aligned(16))) float ks[kLead * kLeadLd];
   __shared__ __attribute__((aligned(16))) float vs[kLead * kLeadLd];
   __shared__ uint8_t ok[kLead];
-  const int t = threadIdx.x;
-  const int r = t >> 2, part = t & 3;
-  float q[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int r = 16 * wave + c;
+  float q[16], kr[16], va[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) q[e] = kr[e] = va[e] = 0.f;   // rows past n: finite, and masked
+  uint8_t valid = 0;
   if (r < n) {
     const int64_t row = row0 + r;
     const float rs = rstd[row];
-    const float* src = qkv + row * ld + h * kHeadDim + 16 * part;
-    float qa[16], ka[16], va[16];
+    const float* src = qkv + row * ld + h * kHeadDim + 16 * g;
+    float qa[16], ka[16];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      *reinterpret_cast<float4*>(qa + 4 * c) = *reinterpret_cast<const float4*>(src + 4 * c);
-      *reinterpret_cast<float4*>(ka + 4 * c) = *reinterpret_cast<const float4*>(src + d + 4 * c);
-      *reinterpret_cast<float4*>(va + 4 * c) =
-          *reinterpret_cast<const float4*>(src + 2 * d + 4 * c);
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<float4*>(qa + 4 * i) = *reinterpret_cast<const float4*>(src + 4 * i);
+      *reinterpret_cast<float4*>(ka + 4 * i) = *reinterpret_cast<const float4*>(src + d + 4 * i);
+      *reinterpret_cast<float4*>(va + 4 * i) =
+          *reinterpret_cast<const float4*>(src + 2 * d + 4 * i);
     }
-    float kr[16];
+    valid = !kmask || kmask[static_cast<int64_t>(b) * S + kstart + r] != 0;
     // the token's three positions once, then the sixteen table entries as independent loads
     const int64_t* p3 = pos + row * 3;
     const int64_t P0 = p3[0], P1 = p3[1], P2 = p3[2];
     float csv[8], snv[8];
 #pragma unroll
     for (int pp = 0; pp < 8; ++pp)
-      rope_cos_sin3(part * 8 + pp, P0, P1, P2, tab, ra, csv[pp], snv[pp]);
+      rope_cos_sin3(g * 8 + pp, P0, P1, P2, tab, ra, csv[pp], snv[pp]);
 #pragma unroll
     for (int pp = 0; pp < 8; ++pp) {
       const float cs = csv[pp], sn = snv[pp];
@@ -447,77 +451,85 @@ __global__ __launch_bounds__(256) void attn_lead_kernel(
       va[2 * pp] *= rs;
       va[2 * pp + 1] *= rs;
     }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      *reinterpret_cast<float4*>(ks + r * kLeadLd + 16 * part + 4 * c) =
-          *reinterpret_cast<const float4*>(kr + 4 * c);
-      *reinterpret_cast<float4*>(vs + r * kLeadLd + 16 * part + 4 * c) =
-          *reinterpret_cast<const float4*>(va + 4 * c);
-    }
-    if (part == 0) ok[r] = !kmask || kmask[static_cast<int64_t>(b) * S + kstart + r] != 0;
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    *reinterpret_cast<float4*>(ks + r * kLeadLd + 16 * g + 4 * i) =
+        *reinterpret_cast<const float4*>(kr + 4 * i);
+    *reinterpret_cast<float4*>(vs + r * kLeadLd + 16 * g + 4 * i) =
+        *reinterpret_cast<const float4*>(va + 4 * i);
+  }
+  if (g == 0) ok[r] = valid;
   __syncthreads();
-  if (r >= n) return;   // no barrier follows; the rest of the 4-thread group returns with it
-  // queries of this wave: 16 (t / 64) .. +15; no key after the wave's last query is visible
-  const int jend = min(16 * (t >> 6) + 15, n - 1);
+  if (16 * wave >= n) return;   // whole wave; no barrier follows
 
-  auto dot = [&](int j) {
-    const float4* kr = reinterpret_cast<const float4*>(ks + j * kLeadLd + 16 * part);
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kBlocks = kLead / 16;
+  f32x4_t sc[kBlocks];
+  float mx = -INFINITY;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float4 k4 = kr[c];
-      a[c] = fmaf(q[4 * c], k4.x, a[c]);
-      a[c] = fmaf(q[4 * c + 1], k4.y, a[c]);
-      a[c] = fmaf(q[4 * c + 2], k4.z, a[c]);
-      a[c] = fmaf(q[4 * c + 3], k4.w, a[c]);
+  for (int nb = 0; nb < kBlocks; ++nb) {
+    sc[nb] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    if (nb > wave) continue;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 k4 =
+          *reinterpret_cast<const float4*>(ks + (16 * nb + c) * kLeadLd + 16 * g + 4 * i);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, q[4 * i], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, q[4 * i + 1], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, q[4 * i + 2], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, q[4 * i + 3], acc, 0, 0, 0);
     }
-    float s = (a[0] + a[1]) + (a[2] + a[3]);
-    s += __shfl_xor(s, 1, kWave);
-    return s + __shfl_xor(s, 2, kWave);
-  };
-  // one pass, online: the running maximum m, the sum l and the output o are rescaled by
-  // exp(m_old - m_new) when a visible score passes m
-  float mx = -INFINITY, l = 0.f, o[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) o[e] = 0.f;
-  for (int j = 0; j <= jend; ++j) {
-    const float s = dot(j);
-    if (j <= r && ok[j]) {
-      if (s > mx) {
-        const float alpha = expf(mx - s);   // 0 at the first visible key
-        l *= alpha;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[e] *= alpha;
-        mx = s;
-      }
-      const float pj = expf(s - mx);
-      l += pj;
-      const float4* vr = reinterpret_cast<const float4*>(vs + j * kLeadLd + 16 * part);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float4 v4 = vr[c];
-        o[4 * c] = fmaf(pj, v4.x, o[4 * c]);
-        o[4 * c + 1] = fmaf(pj, v4.y, o[4 * c + 1]);
-        o[4 * c + 2] = fmaf(pj, v4.z, o[4 * c + 2]);
-        o[4 * c + 3] = fmaf(pj, v4.w, o[4 * c + 3]);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int j = 16 * nb + 4 * g + i;
+      if (j <= r && ok[j]) sc[nb][i] = acc[i];
+      mx = fmaxf(mx, sc[nb][i]);
     }
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;   // no visible key: 0, as in K4a
-  const int64_t orow = row0 + r;
-  const int col0 = h * kHeadDim + 16 * part;
+  mx = max_over_groups(mx);
+  const float base = mx == -INFINITY ? 0.f : mx;   // no visible key: weights 0, as in K4a
+  float l = 0.f;
+  f32x4_t o[4];
 #pragma unroll
-  for (int e = 0; e < 16; e += 2) {
-    uint32_t hi, lo;
-    split_bf2(o[e] * inv, o[e + 1] * inv, hi, lo);
-    uint16_t* oh = out_tiled ? out + tile_off(orow, col0 + e, static_cast<int>(2 * d))
-                             : out + orow * 2 * d + col0 + e;
-    uint16_t* ol = out_tiled ? out + tile_off(orow, static_cast<int>(d) + col0 + e,
-                                              static_cast<int>(2 * d))
-                             : oh + d;
-    *reinterpret_cast<uint32_t*>(oh) = hi;
-    *reinterpret_cast<uint32_t*>(ol) = lo;
+  for (int db = 0; db < 4; ++db) o[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int nb = 0; nb < kBlocks; ++nb) {
+    if (nb > wave) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float pj = expf(sc[nb][i] - base);
+      l += pj;
+      const float4 v4 =
+          *reinterpret_cast<const float4*>(vs + (16 * nb + 4 * g + i) * kLeadLd + 4 * c);
+      o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, pj, o[0], 0, 0, 0);
+      o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, pj, o[1], 0, 0, 0);
+      o[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, pj, o[2], 0, 0, 0);
+      o[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, pj, o[3], 0, 0, 0);
+    }
+  }
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  if (r >= n) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // element i of dim block db is dim 16 g + 4 i + db of query r
+  float res[16];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int db = 0; db < 4; ++db) res[4 * i + db] = o[db][i] * inv;
+  const int64_t orow = row0 + r;
+  const int col0 = h * kHeadDim + 16 * g, d2 = static_cast<int>(2 * d);
+#pragma unroll
+  for (int e = 0; e < 16; e += 4) {
+    uint2 hi, lo;
+    split4(res + e, hi, lo);
+    uint16_t* oh = out_tiled ? out + tile_off(orow, col0 + e, d2) : out + orow * d2 + col0 + e;
+    uint16_t* ol = out_tiled ? out + tile_off(orow, static_cast<int>(d) + col0 + e, d2) : oh + d;
+    *reinterpret_cast<uint32_t*>(oh) = hi.x;   // the entry asks for 4-byte alignment only
+    *reinterpret_cast<uint32_t*>(oh + 2) = hi.y;
+    *reinterpret_cast<uint32_t*>(ol) = lo.x;
+    *reinterpret_cast<uint32_t*>(ol + 2) = lo.y;
   }
 }
 

@@ -297,17 +297,9 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* _
   const int bh = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (bh >= n_bh) return;
-  const float* p = ws + static_cast<int64_t>(bh) * n_split * kPart;
-  float M = -INFINITY;
-  for (int s = 0; s < n_split; ++s) M = fmaxf(M, p[s * kPart]);
-  float L = 0.f, O = 0.f;
-  for (int s = 0; s < n_split; ++s) {
-    const float ms = p[s * kPart];
-    const float sc = (ms == -INFINITY) ? 0.f : exp2f(ms - M);
-    L += p[s * kPart + 1] * sc;
-    O += p[s * kPart + 2 + lane] * sc;
-  }
-  store_split(out, bh, n_heads, lane, L > 0.f ? O / L : 0.f, out_tiled);
+  const float v =
+      merge_parts<kPart>(ws + static_cast<int64_t>(bh) * n_split * kPart, n_split, lane);
+  store_split(out, bh, n_heads, lane, v, out_tiled);
 }
 
 constexpr int kSlotsPerIter = 128;   // split_len granularity

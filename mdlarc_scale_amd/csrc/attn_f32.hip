@@ -41,9 +41,14 @@
 // 271 -> 178 us (92 us of MFMAs), 8 of up to 1,001 and 4 heads 126 -> 61.
 //
 // Decode (attn_f32_decode_kernel): a work item is one split_len-slot chunk of one (row, head), a
-// wave of its own without LDS or barriers; the chunks are what fills the GPU.  With several chunks
-// each writes its running state (m, l, unnormalised o) to the workspace, and
-// attn_f32_combine_kernel merges them.
+// wave of its own without LDS or barriers; the chunks are what fills the GPU.  The query fills all
+// 16 columns, and 32 slots are loaded and worked on at a time.  Lane (c, g) holds dims 16 i + 4 g
+// .. + 3 (i = 0..3) of its key row and of the query here (the same order in both, so the products
+// pair up), which makes each load 64 contiguous bytes of 16 rows.  With several chunks each writes
+// its running state (m, l, unnormalised o) to the workspace, and attn_f32_combine_kernel merges
+// them.  What bounds it is the latency of a chunk's few dependent loads, then HBM: 16 rows of 12
+// heads over some 750 slots (74 MB) with the merge 26 -> 20 us, 8 rows of 4 heads 19 -> 12 (16-slot
+// steps at 128-slot chunks before; a lane's mask bytes were read one by one after the products).
 #include "common.h"
 #include "lds_dma.h"
 #include "mfma.h"
@@ -279,80 +284,97 @@ __global__ __launch_bounds__(64 * kWavesF) void attn_f32_decode_kernel(const F32
   klo = min(klo + chunk * p.split_len, n_keys);
   const int khi = min(klo + p.split_len, n_keys);   // slots of this chunk: [klo, khi)
 
-  float qv[16];   // dims 16 g .. 16 g + 15 of the query, the same in every column
-  load16(p.q + (static_cast<int64_t>(b) * p.heads + h) * kHeadDim + 16 * g, qv);
+  float qv[16];   // element 4 i + e: dim 16 i + 4 g + e of the query
+  const float* qp = p.q + (static_cast<int64_t>(b) * p.heads + h) * kHeadDim + 4 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<float4*>(qv + 4 * i) = *reinterpret_cast<const float4*>(qp + 16 * i);
   const int64_t head = (static_cast<int64_t>(b) * p.heads + h) * p.slots * kHeadDim;
   const float* K = p.kc + head;
   const float* V = p.vc + head;
   const uint8_t* mrow = p.mask ? p.mask + static_cast<int64_t>(b) * p.mask_len : nullptr;
-  float m_run = -INFINITY, l_run = 0.f;
+
+  float m_run = -INFINITY, l_run = 0.f;   // l_run: this lane group's part of the sum
   f32x4 o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int k0 = klo; k0 < khi; k0 += kQT) {
-    // S^T: K rows k0 + c (clamped into [0, n_keys); the clamped rows are masked below)
-    const float* kp = K + static_cast<int64_t>(min(k0 + c, n_keys - 1)) * kHeadDim + 16 * g;
-    float kv[16];
+  for (int k0 = klo; k0 < khi; k0 += 2 * kQT) {
+    // the 32 slots' visibility, one lane each, read with the keys
+    const int kj = k0 + (lane & 31);
+    bool ok = kj < khi;
+    if (mrow && kj < p.mask_len) ok = ok && mrow[kj] != 0;
+    // rows past the chunk load its last slot; their weights are 0
+    float4 kv[2][4], vv[2][4];   // V rows k0 + 16 nb + 4 g + r, dims 4 c .. 4 c + 3
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 v = *reinterpret_cast<const float4*>(kp + 4 * i);
-      kv[4 * i] = v.x; kv[4 * i + 1] = v.y; kv[4 * i + 2] = v.z; kv[4 * i + 3] = v.w;
+    for (int nb = 0; nb < 2; ++nb) {
+      const float* kp =
+          K + static_cast<int64_t>(min(k0 + 16 * nb + c, khi - 1)) * kHeadDim + 4 * g;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kv[nb][i] = ld_f4<true>(kp + 16 * i);
     }
-    float4 vv[4];   // V rows k0 + 4 g + r, dims 4 c .. 4 c + 3
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      vv[r] = *reinterpret_cast<const float4*>(
-          V + static_cast<int64_t>(min(k0 + 4 * g + r, n_keys - 1)) * kHeadDim + 4 * c);
-    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-    for (int kb = 0; kb < 16; ++kb)
-      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[kb], qv[kb], s, 0, 0, 0);
-
-    // visibility of keys k0 + 4 g + r to query c
-    float sv[4];
+      for (int r = 0; r < 4; ++r)
+        vv[nb][r] = ld_f4<true>(
+            V + static_cast<int64_t>(min(k0 + 16 * nb + 4 * g + r, khi - 1)) * kHeadDim + 4 * c);
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+          const float4 k4 = kv[nb][i];
+          const float a = e == 0 ? k4.x : e == 1 ? k4.y : e == 2 ? k4.z : k4.w;
+          s[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qv[4 * i + e], s[nb], 0, 0, 0);
+        }
+    const uint32_t vis = static_cast<uint32_t>(__ballot(ok));
+    if (vis != ~0u) {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!((vis >> (16 * nb + 4 * g + r)) & 1u)) s[nb][r] = -INFINITY;
+    }
     float tmax = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = k0 + 4 * g + r;
-      bool ok = c == 0 && j < khi;
-      if (ok && mrow && j < p.mask_len) ok = mrow[j] != 0;
-      sv[r] = ok ? s[r] : -INFINITY;
-      tmax = fmaxf(tmax, sv[r]);
-    }
-    tmax = max_over_groups(tmax);
-    const float m_new = fmaxf(m_run, tmax);
-    float pr[4], psum = 0.f, alpha = 1.f;
-    if (m_new == -INFINITY) {
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) pr[r] = 0.f;
-    } else {
-      alpha = exp2f(m_run - m_new);    // m_run = -inf: 0 (o and l are 0 then)
+      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[nb][r]);
+    const float m_old = m_run;
+    m_run = fmaxf(m_run, max_over_groups(tmax));
+    const float base = m_run == -INFINITY ? 0.f : m_run;   // no visible slot yet: weights 0
+    const float alpha = exp2f(m_old - base);
+    float psum = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pr[r] = exp2f(sv[r] - m_new);  // -inf: 0
-        psum += pr[r];
+        s[nb][r] = exp2f(s[nb][r] - base);
+        psum += s[nb][r];
       }
-    }
-    psum += __shfl_xor(psum, 16, kWave);
-    psum += __shfl_xor(psum, 32, kWave);
     l_run = fmaf(l_run, alpha, psum);
-    m_run = m_new;
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[db] *= alpha;
     // O^T += V^T . P^T, key step r: lane group g contributes key 4 g + r
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float ve[4] = {vv[r].x, vv[r].y, vv[r].z, vv[r].w};
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], pr[r], o[db], 0, 0, 0);
-    }
+      for (int r = 0; r < 4; ++r) {
+        const float ve[4] = {vv[nb][r].x, vv[nb][r].y, vv[nb][r].z, vv[nb][r].w};
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+          o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[db], 0, 0, 0);
+      }
   }
+  l_run += __shfl_xor(l_run, 16, kWave);
+  l_run += __shfl_xor(l_run, 32, kWave);
 
-  if (c != 0) return;
+  if (c != 0) return;   // every column holds the same
   if (p.ws) {
-    // this chunk's state: m and l (the same in every lane of query column 0), o unnormalised
+    // this chunk's state: m and l, o unnormalised
     float* part = p.ws + item * kPartF;
     if (g == 0) {
       part[0] = m_run;
@@ -366,6 +388,7 @@ __global__ __launch_bounds__(64 * kWavesF) void attn_f32_decode_kernel(const F32
   }
   store_out(p, b, h, g, l_run, o);
 }
+
 // The decode chunks of one (row, head) merged, lane = channel: the states rescaled to their
 // largest m (base 2), o / l, stored as the split output of mdl_attn_decode_f32.
 __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __restrict__ ws,
@@ -376,17 +399,8 @@ __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __re
   const int bh = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (bh >= n_bh) return;
-  const float* part = ws + static_cast<int64_t>(bh) * n_split * kPartF;
-  float M = -INFINITY;
-  for (int s = 0; s < n_split; ++s) M = fmaxf(M, part[s * kPartF]);
-  float L = 0.f, O = 0.f;
-  for (int s = 0; s < n_split; ++s) {
-    const float ms = part[s * kPartF];
-    const float sc = ms == -INFINITY ? 0.f : exp2f(ms - M);
-    L = fmaf(part[s * kPartF + 1], sc, L);
-    O = fmaf(part[s * kPartF + 2 + lane], sc, O);
-  }
-  const float v = L > 0.f ? O / L : 0.f;
+  const float v = merge_parts<kPartF>(ws + static_cast<int64_t>(bh) * n_split * kPartF, n_split,
+                                      lane);
   const int b = bh / n_heads, h = bh - b * n_heads;
   const int d = n_heads * kHeadDim, col = h * kHeadDim + lane;
   const uint16_t hi = static_cast<uint16_t>(f2bf(v));

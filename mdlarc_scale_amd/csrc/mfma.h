@@ -68,4 +68,36 @@ __device__ __forceinline__ float max_over_groups(float v) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+// Channel `lane` of the merge of one (row, head)'s split states (m, l, o[64] unnormalised, PART
+// floats apart; base 2): o / l at their largest m, 0 if no split saw a key.  A lane reads one
+// split's m and l, so a wave has all of them (64 at a time) after one round trip, and the o
+// values, whose addresses depend on nothing read, come eight at a time
+// (a chain of one dependent load per split took 6 us at 7 splits of 12 pairs, this 2.9).
+template <int PART>
+__device__ __forceinline__ float merge_parts(const float* __restrict__ part, int n_split,
+                                             int lane) {
+  float M = -INFINITY;
+  for (int s = lane; s < n_split; s += kWave) M = fmaxf(M, part[s * PART]);
+  M = wave_max(M);
+  float L = 0.f, O = 0.f;
+  for (int s0 = 0; s0 < n_split; s0 += kWave) {
+    const int s = min(s0 + lane, n_split - 1);
+    const float ms = part[s * PART];
+    const float sc = s0 + lane < n_split && ms != -INFINITY ? exp2f(ms - M) : 0.f;
+    L = fmaf(part[s * PART + 1], sc, L);
+    const int n = min(kWave, n_split - s0);
+    for (int q0 = 0; q0 < n; q0 += 8) {
+      float o[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        o[q] = part[(s0 + min(q0 + q, n - 1)) * PART + 2 + lane];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)   // lanes past the last split hold a weight of 0
+        O = fmaf(o[q], __shfl(sc, min(q0 + q, kWave - 1), kWave), O);
+    }
+  }
+  L = wave_sum(L);
+  return L > 0.f ? O / L : 0.f;
+}
+
 }  // namespace mdl

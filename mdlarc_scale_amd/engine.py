@@ -319,6 +319,19 @@ def pack_prompt(kv_start: np.ndarray, last_row: np.ndarray, batch: int, seq: int
 
 DECODE_MIN_BLOCKS = 2048   # 8 four-wave blocks per CU on 256 CUs
 
+# The fp32 form's work item is one wave and a SIMD holds four: as many chunks as keep all waves
+# resident at once, three to a SIMD, of at least 64 slots (two of the kernel's steps).  192 pairs of
+# 931 slots take 20.0 us at 64, 21.8 at 32, 23.8 at 128 and 30.7 at 256; 768 pairs of 1,800 take
+# 88.6 at 512, 96 at 384, 104 at 192 and 112 at 1,024.
+DECODE_WAVES_F32 = 3072
+
+
+def choose_split_len_f32(n_bh: int, slots: int) -> int:
+    """Slots per work item of the fp32 decode attention (a multiple of 64), as choose_split_len."""
+    n_split = max(1, DECODE_WAVES_F32 // max(n_bh, 1))
+    per = -(-slots // n_split)
+    return max(64, -(-per // 64) * 64)
+
 
 def choose_split_len(n_bh: int, slots: int) -> int:
     """Slots per decode-attention work item (a multiple of 128).  One chunk per (row, head) once

@@ -37,7 +37,7 @@ from .data import (
     generate_color_permutations,
 )
 from .engine import GRID_MAX_X, GRID_MAX_Y, HipEngine, PackedWeights, Scratch, choose_split_len
-from .engine import pack_prompt
+from .engine import choose_split_len_f32, pack_prompt
 from .engine import engine_for, gemm_f32, model_form, tiles_supported
 from .transformer import TinyTransformer, attention_q_scale
 
@@ -296,7 +296,7 @@ class Generator:
                     row_holes=holes, row_shift=row_shift)
         # longest rows first: the decode-attention launch dispatches them before the short ones
         order = torch.argsort(kv_start, stable=True).to(torch.int32)
-        split = choose_split_len(B * H, total)
+        split = (choose_split_len_f32 if f32 else choose_split_len)(B * H, total)
         nbytes = K.attn_decode_workspace_bytes(B, H, total, split)
         ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev) if nbytes else None
         out_ids = torch.empty(B, total, dtype=torch.int64, device=dev)
@@ -944,7 +944,7 @@ def _decode_step(model: TinyTransformer, token: torch.Tensor, position: torch.Te
         if attention_mask is not None:
             pmask = attention_mask[:, :t + 1].to(device=dev, dtype=torch.uint8).contiguous()
         slots = cache.max_seq_len
-        split = choose_split_len(B * H, slots)
+        split = (choose_split_len_f32 if f32 else choose_split_len)(B * H, slots)
         nbytes = K.attn_decode_workspace_bytes(B, H, slots, split)
         i32 = lambda: torch.zeros(B, dtype=torch.int32, device=dev)  # noqa: E731
         st = DecodeState(

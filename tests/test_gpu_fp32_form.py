@@ -359,3 +359,25 @@ def test_attn_decode_f32(slots, t, with_mask, split_len):
         ref = rp.attention((q.double() * 8 / LOG2E)[:, :, None], kc[:, :, :t + 1].double(),
                            vc[:, :, :t + 1].double(), keymask, causal=False)[:, :, 0]
         _attn_close(unsplit(got).view(B, H, 64), ref, f"seq_dev={dev_seq}")
+
+
+@pytest.mark.parametrize("n_split", [2, 8, 9, 63, 64, 65, 130])
+def test_decode_merge_of_many_splits(n_split):
+    """The merge takes 64 splits at a time and their values 8 at a time: equal to one chunk over
+    the same slots, to the fp32 rounding of n_split rescaled sums (each weight and sum is within a
+    few 2^-24, and the output is stored to 2^-17)."""
+    g = torch.Generator().manual_seed(n_split)
+    B, H, slots = 3, 2, 16 * n_split - 5
+    q = (torch.randn(B, H, 64, generator=g) * 0.3).to(DEV)
+    kc, vc = (torch.randn(B, H, slots, 64, generator=g).to(DEV) for _ in range(2))
+    kv = torch.tensor([0, 7, slots - 3], dtype=torch.int32, device=DEV)   # most chunks empty
+    outs = []
+    for split in (16, 16 * n_split):
+        nbytes = K().attn_decode_workspace_bytes(B, H, slots, split)
+        ws = torch.full((nbytes // 4,), float("nan"), device=DEV) if nbytes else None
+        out = torch.empty(B, 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+        K().attn_decode_f32(q, kc, vc, B, H, None, 0, kv, slots - 1, None, ws, split, out)
+        torch.cuda.synchronize()
+        outs.append(unsplit(out))
+    a, b = outs
+    assert bool(((a - b).abs() <= 2 ** -16 * b.abs() + 2 ** -20).all()), (a - b).abs().max()

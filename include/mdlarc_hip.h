@@ -309,6 +309,16 @@ int mdl_gemm_norm_qkv(const float* x, const float* gamma, float eps, const uint1
                       uint16_t* q_out, uint16_t* k_cache, uint16_t* v_cache, int cache_slots,
                       int slot0, const int32_t* slot_dev, int tile, void* stream);
 /*
+ * mdl_gemm_norm_qkv of an fp32 weight (w its bf16 part, w_lo the low part, both tiled) for a model
+ * with an fp32 cache: q_out, k_cache and v_cache are fp32 and 16-byte aligned; w_lo not NULL.
+ */
+int mdl_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps, const uint16_t* w,
+                           const uint16_t* w_lo, int m, int n_heads, float* rstd_out,
+                           const int64_t* pos, const float* rope_tab, int max_x, int max_y,
+                           int max_z, int px, int py, int pz, float q_scale, float* q_out,
+                           float* k_cache, float* v_cache, int cache_slots, int slot0,
+                           const int32_t* slot_dev, int tile, void* stream);
+/*
  * mdl_gemm_norm feeding the SwiGLU epilogue of mdl_gemm_split_swiglu (rstd from the prologue):
  * h = split(silu(rstd g + bias_gate) * (rstd u + bias_up)) with g / u the gate / up rows of
  * w_gu against split(x * gamma).  w_gu_lo (may be NULL): the low part of an fp32 w_gu, as
@@ -416,6 +426,19 @@ int mdl_prefill_gemm_norm_qkv(const float* x, const float* gamma, float eps, con
                               int py, int pz, float q_scale, uint16_t* q_out, uint16_t* k_cache,
                               uint16_t* v_cache, int cache_slots, int batch, int seq,
                               const int32_t* token_row, const int32_t* token_slot, void* stream);
+/*
+ * mdl_prefill_gemm_norm_qkv of an fp32 weight (w, w_lo) for an fp32 cache: fp32 q [m, d], K and V,
+ * no lead rows.  Small row counts run as mdl_gemm_norm and mdl_qkv_rope_cache through the scratch
+ * qkv [m, ldq >= 3 d] and rstd [m], which are otherwise not written.
+ */
+int mdl_prefill_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps,
+                                   const uint16_t* w, const uint16_t* w_lo, int m, int n_heads,
+                                   float* qkv, int64_t ldq, float* rstd, const int64_t* pos,
+                                   const float* rope_tab, int max_x, int max_y, int max_z, int px,
+                                   int py, int pz, float q_scale, float* q_out, float* k_cache,
+                                   float* v_cache, int cache_slots, int batch, int seq,
+                                   const int32_t* token_row, const int32_t* token_slot,
+                                   void* stream);
 /*
  * dst = src ([rows, cols] bf16, row stride ld) in MDL_LAYOUT_TILES, rows padded to a multiple
  * of 16 with zeros (dst holds ceil(rows / 16) * 16 * cols elements).  cols a multiple of 32.

@@ -133,6 +133,16 @@ __device__ __forceinline__ void st_u2(void* p, uint2 v) {
     *reinterpret_cast<uint2*>(p) = v;
 }
 
+// four consecutive q / k / v channels in the cache dtype: bf16 (8 bytes) or fp32 (16)
+template <bool NT>
+__device__ __forceinline__ void st_ch4(uint16_t* p, float a, float b, float c, float d) {
+  st_u2<NT>(p, make_uint2(pack_bf2(a, b), pack_bf2(c, d)));
+}
+template <bool NT>
+__device__ __forceinline__ void st_ch4(float* p, float a, float b, float c, float d) {
+  st_f4<NT>(p, make_float4(a, b, c, d));
+}
+
 template <bool NT>
 __device__ __forceinline__ void st_u4(void* p, uint4 v) {
   if constexpr (NT)

@@ -59,6 +59,8 @@
 // not depend on how many rows run beside it.
 #include <algorithm>
 
+#include <type_traits>
+
 #include "common.h"
 #include "lds_dma.h"
 #include "mfma.h"
@@ -106,9 +108,9 @@ struct Args {
   const float* rope_tab;
   RopeArgs ra;
   float q_scale;
-  uint16_t* q_out;
-  uint16_t* kc;
-  uint16_t* vc;
+  void* q_out;   // bf16, or fp32 with fp32 weights (WL), like the caches
+  void* kc;
+  void* vc;
   const int32_t* tok_row;
   const int32_t* tok_slot;
   const int32_t* kv_start;
@@ -456,7 +458,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
         // clamped below at 0 as the lead-attention pass (K4c) clamps it, so the rows written
         // here are exactly the rows it reads
         const int ks = (p.kv_start && b >= 0 && b < p.batch) ? max(p.kv_start[b], 0) : 0;
-        const bool lead_row = p.out != nullptr && slot >= ks && slot - ks < p.lead;
+        const bool lead_row = !WL && p.out != nullptr && slot >= ks && slot - ks < p.lead;
         const float rs = rstd_s[r];
         const int64_t* pos3 = p.pos + static_cast<int64_t>(m) * 3;
         float cs[2 * kQ], sn[2 * kQ];
@@ -483,26 +485,20 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
           const int head = e / kHeadDim, dim = e - head * kHeadDim;
           const int q4 = i % kQ;
           const float a0 = v[0] * rs, a1 = v[1] * rs, a2 = v[2] * rs, a3 = v[3] * rs;
-          uint2 o;
+          using TO = std::conditional_t<WL, float, uint16_t>;
+          const int64_t at = cache_row + head * head_stride + dim;
           if (part == 2) {
-            if (!in_cache) continue;
-            o.x = pack_bf2(a0, a1);
-            o.y = pack_bf2(a2, a3);
-            *reinterpret_cast<uint2*>(p.vc + cache_row + head * head_stride + dim) = o;
+            if (in_cache) st_ch4<false>(static_cast<TO*>(p.vc) + at, a0, a1, a2, a3);
             continue;
           }
           float y0, y1, y2, y3;
           rope_rot(a0, a1, cs[2 * q4], sn[2 * q4], y0, y1);
           rope_rot(a2, a3, cs[2 * q4 + 1], sn[2 * q4 + 1], y2, y3);
-          if (part == 0) {
-            o.x = pack_bf2(y0 * p.q_scale, y1 * p.q_scale);
-            o.y = pack_bf2(y2 * p.q_scale, y3 * p.q_scale);
-            *reinterpret_cast<uint2*>(p.q_out + static_cast<int64_t>(m) * d + e) = o;
-          } else if (in_cache) {
-            o.x = pack_bf2(y0, y1);
-            o.y = pack_bf2(y2, y3);
-            *reinterpret_cast<uint2*>(p.kc + cache_row + head * head_stride + dim) = o;
-          }
+          if (part == 0)
+            st_ch4<false>(static_cast<TO*>(p.q_out) + static_cast<int64_t>(m) * d + e,
+                          y0 * p.q_scale, y1 * p.q_scale, y2 * p.q_scale, y3 * p.q_scale);
+          else if (in_cache)
+            st_ch4<false>(static_cast<TO*>(p.kc) + at, y0, y1, y2, y3);
         }
       }
     } else if constexpr (EPI == E_SWIGLU) {
@@ -1020,6 +1016,54 @@ extern "C" int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, fl
   p.x = x; p.gamma = gamma; p.eps = eps; p.w = w; p.wl = w_lo; p.out = out; p.ldo = ldo;
   p.rstd_out = rstd_out; p.M = m; p.N = n; p.K = k;
   return launch_f32w<E_STORE>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdl_prefill_gemm_norm_qkv_f32w(
+    const float* x, const float* gamma, float eps, const uint16_t* w, const uint16_t* w_lo, int m,
+    int n_heads, float* qkv, int64_t ldq, float* rstd, const int64_t* pos, const float* rope_tab,
+    int max_x, int max_y, int max_z, int px, int py, int pz, float q_scale, float* q_out,
+    float* k_cache, float* v_cache, int cache_slots, int batch, int seq, const int32_t* token_row,
+    const int32_t* token_slot, void* stream) {
+  if (n_heads <= 0 || n_heads * kHeadDim > kMaxNormK) return MDL_ERR_SHAPE;
+  const int d = n_heads * kHeadDim;
+  int rc = check_common(w, m, 3 * d, d);
+  if (rc != MDL_OK) return rc;
+  if (!w_lo || !x || !gamma || !qkv || !rstd || !pos || !rope_tab || !q_out || !k_cache ||
+      !v_cache)
+    return MDL_ERR_NULL;
+  if ((token_row == nullptr) != (token_slot == nullptr)) return MDL_ERR_NULL;
+  if (max_x <= 0 || max_y <= 0 || max_z <= 0 || px < 0 || py < 0 || pz < 0 ||
+      px + py + pz != kHeadDim / 2 || batch < 0 || cache_slots <= 0 || ldq < 3 * d)
+    return MDL_ERR_SHAPE;
+  if (!token_slot) {   // [batch, seq] rows: token i of row b is slot i
+    if (seq <= 0 || static_cast<int64_t>(batch) * seq != m) return MDL_ERR_SHAPE;
+    if (seq > cache_slots) return MDL_ERR_CACHE;
+  }
+  if (!aligned16(w_lo) || !aligned16(x) || !aligned16(gamma) || !aligned16(qkv) || ldq % 4 != 0 ||
+      !aligned16(q_out) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned4(rope_tab))
+    return MDL_ERR_ALIGN;
+  if (m == 0) return MDL_OK;
+  if (m <= kK5Rows) {
+    rc = mdl_gemm_norm(x, gamma, eps, w, w_lo, qkv, ldq, rstd, m, 3 * d, d, 0, stream);
+    if (rc != MDL_OK) return rc;
+    return token_slot
+               ? mdl_qkv_rope_cache_packed(qkv, ldq, rstd, pos, rope_tab, m, token_row, token_slot,
+                                           batch, n_heads, kHeadDim, max_x, max_y, max_z, px, py,
+                                           pz, q_scale, q_out, k_cache, v_cache, MDL_DTYPE_F32,
+                                           cache_slots, stream)
+               : mdl_qkv_rope_cache(qkv, ldq, rstd, pos, rope_tab, batch, seq, n_heads, kHeadDim,
+                                    max_x, max_y, max_z, px, py, pz, q_scale, q_out, k_cache,
+                                    v_cache, MDL_DTYPE_F32, cache_slots, 0, nullptr, stream);
+  }
+  Args p{};
+  p.x = x; p.gamma = gamma; p.eps = eps; p.w = w; p.wl = w_lo;
+  p.pos = pos; p.rope_tab = rope_tab;
+  p.ra = RopeArgs{max_x, max_y, max_z, px, py, pz};
+  p.q_scale = q_scale; p.q_out = q_out; p.kc = k_cache; p.vc = v_cache;
+  p.tok_row = token_row; p.tok_slot = token_slot;
+  p.slots = cache_slots; p.seq = seq; p.batch = batch;
+  p.M = m; p.N = 3 * d; p.K = d;
+  return launch_f32w<E_QKV>(p, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mdl_prefill_gemm_norm_swiglu_f32w(const float* x, const float* gamma, float eps,

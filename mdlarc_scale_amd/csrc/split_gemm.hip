@@ -18,7 +18,8 @@
 //               (each element has one owner block, so the update needs no synchronisation);
 //   E_QKV       K2 for the decode token of each row on the qkv accumulators (A_NORM): rstd,
 //               3D RoPE of q and k, the softmax scale on q; q bf16 [M, d] and K / V into cache
-//               slot t (*slot_dev) of row m, so the attention launch needs no prologue.
+//               slot t (*slot_dev) of row m, so the attention launch needs no prologue.  With fp32
+//               weights q, K and V are fp32, as that form's cache is.
 //
 // Why not the library GEMM at decode: at M <= 256 rows hipBLASLt runs 64x64 or 32x32 tiles over
 // the doubled K of [W | W] (each weight byte read twice) on at most 144 workgroups for the small
@@ -45,6 +46,8 @@
 // matrices in the same tile layout, w = bf16(W) and w_lo = bf16(W - w).  Every k-step then adds
 // a third product, a_hi . w_lo, after the hi and lo products, so the GEMM sees W to ~2^-17 like
 // the activation (the dropped a_lo . w_lo term is ~2^-18 of the product).
+#include <type_traits>
+
 #include "common.h"
 #include "mfma.h"
 #include "rope.h"
@@ -82,9 +85,9 @@ struct GemmArgs {
   const float* rope_tab;
   RopeArgs ra;
   float q_scale;
-  uint16_t* q_out;
-  uint16_t* kc;
-  uint16_t* vc;
+  void* q_out;             // bf16, or fp32 with fp32 weights (WL), like the caches
+  void* kc;
+  void* vc;
   const int32_t* slot_dev;
   int slot0, slots;
   int M, N, K, n_tiles, m_tiles, per_xcd;
@@ -393,30 +396,22 @@ __global__ __launch_bounds__(64 * kGemmWaves) void split_gemm_kernel(const GemmA
           const float a0 = v[0] * r, a1 = v[1] * r, a2 = v[2] * r, a3 = v[3] * r;
           const int t = p.slot_dev ? *p.slot_dev : p.slot0;
           const bool in_cache = t >= 0 && t < p.slots;
-          // K / V go out with the non-temporal hint: 8 bytes per (row, head, slot t) of cache
+          // K / V go out with the non-temporal hint: a few bytes per (row, head, slot t) of cache
           // rows megabytes apart, read next by the attention's non-temporal loads
+          using TO = std::conditional_t<WL, float, uint16_t>;
           const int64_t crow =
               ((static_cast<int64_t>(m) * (d / kHeadDim) + head) * p.slots + t) * kHeadDim + dim;
-          uint2 o;
           if (part == 2) {
-            if (in_cache) {
-              o.x = pack_bf2(a0, a1);
-              o.y = pack_bf2(a2, a3);
-              st_u2<true>(p.vc + crow, o);
-            }
+            if (in_cache) st_ch4<true>(static_cast<TO*>(p.vc) + crow, a0, a1, a2, a3);
           } else {
             float y0, y1, y2, y3;
             rope_rot(a0, a1, rcs[gi][0], rcs[gi][1], y0, y1);
             rope_rot(a2, a3, rcs[gi][2], rcs[gi][3], y2, y3);
-            if (part == 0) {
-              o.x = pack_bf2(y0 * p.q_scale, y1 * p.q_scale);
-              o.y = pack_bf2(y2 * p.q_scale, y3 * p.q_scale);
-              *reinterpret_cast<uint2*>(p.q_out + static_cast<int64_t>(m) * d + e) = o;
-            } else if (in_cache) {
-              o.x = pack_bf2(y0, y1);
-              o.y = pack_bf2(y2, y3);
-              st_u2<true>(p.kc + crow, o);
-            }
+            if (part == 0)
+              st_ch4<false>(static_cast<TO*>(p.q_out) + static_cast<int64_t>(m) * d + e,
+                            y0 * p.q_scale, y1 * p.q_scale, y2 * p.q_scale, y3 * p.q_scale);
+            else if (in_cache)
+              st_ch4<true>(static_cast<TO*>(p.kc) + crow, y0, y1, y2, y3);
           }
         } else if constexpr (EPI == E_RESIDUAL) {
           // x + delta, then + bias: the order of the add+RMSNorm kernel it replaces
@@ -610,13 +605,16 @@ extern "C" int mdl_gemm_norm(const float* x, const float* gamma, float eps, cons
   return launch_w<A_NORM, E_STORE>(tile, p, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int mdl_gemm_norm_qkv(const float* x, const float* gamma, float eps,
-                                 const uint16_t* w, int m, int n_heads, float* rstd_out,
-                                 const int64_t* pos, const float* rope_tab, int max_x, int max_y,
-                                 int max_z, int px, int py, int pz, float q_scale,
-                                 uint16_t* q_out, uint16_t* k_cache, uint16_t* v_cache,
-                                 int cache_slots, int slot0, const int32_t* slot_dev, int tile,
-                                 void* stream) {
+namespace mdl {
+
+namespace {
+
+// w_lo: fp32 q / caches; NULL: bf16 ones
+int gemm_norm_qkv(const float* x, const float* gamma, float eps, const uint16_t* w,
+                  const uint16_t* w_lo, int m, int n_heads, float* rstd_out, const int64_t* pos,
+                  const float* rope_tab, int max_x, int max_y, int max_z, int px, int py, int pz,
+                  float q_scale, void* q_out, void* k_cache, void* v_cache, int cache_slots,
+                  int slot0, const int32_t* slot_dev, int tile, void* stream) {
   if (!x || !gamma || !w || !pos || !rope_tab || !q_out || !k_cache || !v_cache)
     return MDL_ERR_NULL;
   if (n_heads <= 0 || n_heads > (1 << 16)) return MDL_ERR_SHAPE;
@@ -628,12 +626,15 @@ extern "C" int mdl_gemm_norm_qkv(const float* x, const float* gamma, float eps,
   if (!aligned16(x) || !aligned16(gamma) || !aligned16(w) || !aligned8(q_out) ||
       !aligned8(k_cache) || !aligned8(v_cache) || !aligned4(rope_tab))
     return MDL_ERR_ALIGN;
+  if (w_lo && (!aligned16(w_lo) || !aligned16(q_out) || !aligned16(k_cache) || !aligned16(v_cache)))
+    return MDL_ERR_ALIGN;
   if (m == 0) return MDL_OK;
   GemmArgs p{};
   p.x = x;
   p.gamma = gamma;
   p.eps = eps;
   p.w = w;
+  p.wl = w_lo;
   p.rstd_out = rstd_out;
   p.pos = pos;
   p.rope_tab = rope_tab;
@@ -648,7 +649,36 @@ extern "C" int mdl_gemm_norm_qkv(const float* x, const float* gamma, float eps,
   p.M = m;
   p.N = 3 * d;
   p.K = d;
-  return launch<true, A_NORM, E_QKV>(tile, p, static_cast<hipStream_t>(stream));
+  return launch_w<A_NORM, E_QKV>(tile, p, static_cast<hipStream_t>(stream));
+}
+
+}  // namespace
+
+}  // namespace mdl
+
+extern "C" int mdl_gemm_norm_qkv(const float* x, const float* gamma, float eps,
+                                 const uint16_t* w, int m, int n_heads, float* rstd_out,
+                                 const int64_t* pos, const float* rope_tab, int max_x, int max_y,
+                                 int max_z, int px, int py, int pz, float q_scale,
+                                 uint16_t* q_out, uint16_t* k_cache, uint16_t* v_cache,
+                                 int cache_slots, int slot0, const int32_t* slot_dev, int tile,
+                                 void* stream) {
+  return gemm_norm_qkv(x, gamma, eps, w, nullptr, m, n_heads, rstd_out, pos, rope_tab, max_x,
+                       max_y, max_z, px, py, pz, q_scale, q_out, k_cache, v_cache, cache_slots,
+                       slot0, slot_dev, tile, stream);
+}
+
+extern "C" int mdl_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps,
+                                      const uint16_t* w, const uint16_t* w_lo, int m, int n_heads,
+                                      float* rstd_out, const int64_t* pos, const float* rope_tab,
+                                      int max_x, int max_y, int max_z, int px, int py, int pz,
+                                      float q_scale, float* q_out, float* k_cache, float* v_cache,
+                                      int cache_slots, int slot0, const int32_t* slot_dev,
+                                      int tile, void* stream) {
+  if (!w_lo) return MDL_ERR_NULL;
+  return gemm_norm_qkv(x, gamma, eps, w, w_lo, m, n_heads, rstd_out, pos, rope_tab, max_x, max_y,
+                       max_z, px, py, pz, q_scale, q_out, k_cache, v_cache, cache_slots, slot0,
+                       slot_dev, tile, stream);
 }
 
 extern "C" int mdl_gemm_norm_swiglu(const float* x, const float* gamma, float eps,

@@ -414,9 +414,15 @@ class HipEngine:
             if sc.f32:
                 # fp32 form: projection with the low weight part, K2 into the fp32 cache, K4f (the
                 # attention is exact, so no lead pass)
-                self._qkv_f32(W, li, sc)
-                K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
-                                 sc.q, kc, vc, slot0=0)
+                if sc.fused_f32:
+                    K.prefill_gemm_norm_qkv_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li],
+                                                 W.qkv_lo[li], B * S, H, sc.qkv, sc.rstd, pos,
+                                                 W.rope_tab, W.rope_geom, qa, sc.q, kc, vc, seq=S)
+                else:
+                    K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
+                                w_lo=W.qkv_lo[li])
+                    K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
+                                     sc.q, kc, vc, slot0=0)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, None, B * S,
                                    causal, sc.attn, out_tiled=True)
                 self._mlp(W, li, sc)
@@ -466,9 +472,16 @@ class HipEngine:
         for li in range(cfg.n_layers):
             kc, vc = kv_layers(li)
             if sc.f32:   # fp32 form (see run_prompt)
-                self._qkv_f32(W, li, sc)
-                K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
-                                        pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
+                if sc.fused_f32:
+                    K.prefill_gemm_norm_qkv_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li],
+                                                 W.qkv_lo[li], pk.n_tokens, H, sc.qkv, sc.rstd,
+                                                 pos_p, W.rope_tab, W.rope_geom, qa, sc.q, kc, vc,
+                                                 token_row=pk.token_row, token_slot=pk.token_slot)
+                else:
+                    K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
+                                w_lo=W.qkv_lo[li])
+                    K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
+                                            pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, pk.q_offset,
                                    pk.n_tokens, True, sc.attn, out_tiled=True)
                 self._mlp(W, li, sc)
@@ -489,17 +502,6 @@ class HipEngine:
                                 key_mask, kv_start, pk.q_offset, pk.n_tokens, sc.attn,
                                 out_tiled=fused)
             self._mlp(W, li, sc)
-
-    @staticmethod
-    def _qkv_f32(W: PackedWeights, li: int, sc: Scratch) -> None:
-        """ln1 + qkv_proj of a prompt in the fp32 form: the fp32 projection rows and rstd."""
-        k = W.ln1[li].numel()
-        if sc.fused_f32:
-            K.prefill_gemm_norm_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li], W.qkv_lo[li], sc.qkv,
-                                     sc.rstd, k)
-        else:
-            K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, k,
-                        w_lo=W.qkv_lo[li])
 
     def _mlp(self, W: PackedWeights, li: int, sc: Scratch) -> None:
         """out_proj + residual, ln2, SwiGLU MLP + residual, next norm (shared by both phases)."""

@@ -356,11 +356,10 @@ class Generator:
             kc, vc = st.cache.layer(li)
             if sc.f32:
                 # fp32 form: projection with the low weight part, K2 of the token into slot t
-                # of the fp32 cache, K4f over slots [kv_start, t]
-                K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, cfg.d_model,
-                            w_lo=W.qkv_lo[li])
-                K.qkv_rope_cache(sc.qkv, sc.rstd, st.pos, W.rope_tab, W.rope_geom, B, 1, H, qs,
-                                 sc.q, kc, vc, slot_dev=slot)
+                # of the fp32 cache in its epilogue, K4f over slots [kv_start, t]
+                K.gemm_norm_qkv(sc.x, W.ln1[li], W.eps, W.qkv_t[li], B, H, None, st.pos,
+                                W.rope_tab, W.rope_geom, qs, sc.q, kc, vc, slot_dev=slot,
+                                w_lo=W.qkv_lo[li])
                 K.attn_decode_f32(sc.q, kc, vc, B, H, st.pmask, st.S, st.kv_start, 0, slot,
                                   st.ws, st.split_len, sc.attn, tiled=True)
             elif sc.tiled:

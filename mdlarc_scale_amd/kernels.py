@@ -382,24 +382,33 @@ def gemm_norm_qkv(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Ten
                   rope_tab: torch.Tensor, rope_geom: tuple[int, int, int, int, int, int],
                   q_scale: float, q_out: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, slot0: int = 0, slot_dev: torch.Tensor | None = None,
-                  tile: int = 0) -> None:
+                  tile: int = 0, w_lo: torch.Tensor | None = None) -> None:
     """ln1 + qkv_proj + K2 of the decode token of each row in one K5 launch: q (bf16 [m, d]),
     K / V into slot slot_dev[0] (or slot0) of each cache row; x the fp32 tile-layout residual
-    stream, w the tiled qkv weight."""
+    stream, w the tiled qkv weight.  With w_lo (the low part of an fp32 weight) q and the caches
+    are fp32."""
     d = n_heads * HEAD_DIM
+    dt = BF16 if w_lo is None else F32
+    _need(w_lo, "w_lo", BF16, tile_rows(3 * d) * d, optional=True)
     _need(x, "x", F32, tile_rows(m) * d)
     _need(gamma, "gamma", F32, d)
     _need(w, "w", BF16, tile_rows(3 * d) * d)
     _need(rstd_out, "rstd_out", F32, m, optional=True)
     _need(pos, "pos", I64, m * 3)
     _need(rope_tab, "rope_tab", F32)
-    _need(q_out, "q_out", BF16, m * d)
+    _need(q_out, "q_out", dt, m * d)
     for name, c in (("k_cache", k_cache), ("v_cache", v_cache)):
-        _need(c, name, BF16)
+        _need(c, name, dt)
         if c.dim() != 4 or c.shape[0] != m or c.shape[1] != n_heads or c.shape[3] != 64:
             raise ValueError(f"{name} must be [m, n_heads, slots, 64]")
     _need(slot_dev, "slot_dev", I32, 1, optional=True)
     mx, my, mz, px, py, pz = rope_geom
+    if w_lo is not None:
+        _lib.check(_lib.lib().mdl_gemm_norm_qkv_f32w(
+            _p(x), _p(gamma), eps, _p(w), _p(w_lo), m, n_heads, _p(rstd_out), _p(pos),
+            _p(rope_tab), mx, my, mz, px, py, pz, q_scale, _p(q_out), _p(k_cache), _p(v_cache),
+            k_cache.shape[2], slot0, _p(slot_dev), tile, _stream()), "mdl_gemm_norm_qkv_f32w")
+        return
     _lib.check(_lib.lib().mdl_gemm_norm_qkv(
         _p(x), _p(gamma), eps, _p(w), m, n_heads, _p(rstd_out), _p(pos), _p(rope_tab), mx, my,
         mz, px, py, pz, q_scale, _p(q_out), _p(k_cache), _p(v_cache), k_cache.shape[2], slot0,
@@ -610,6 +619,46 @@ def prefill_gemm_norm_qkv(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: t
         _p(kv_start), _p(pos), _p(rope_tab), mx, my, mz, px, py, pz, q_scale, _p(q_out),
         _p(k_cache), _p(v_cache), slots, batch, seq, _p(token_row), _p(token_slot), _stream()),
         "mdl_prefill_gemm_norm_qkv")
+
+
+def prefill_gemm_norm_qkv_f32w(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor,
+                               w_lo: torch.Tensor, rows: int, n_heads: int, qkv: torch.Tensor,
+                               rstd: torch.Tensor, pos: torch.Tensor, rope_tab: torch.Tensor,
+                               rope_geom: tuple[int, int, int, int, int, int], q_scale: float,
+                               q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                               token_row: torch.Tensor | None = None,
+                               token_slot: torch.Tensor | None = None, seq: int = 0) -> None:
+    """prefill_gemm_norm_qkv of an fp32 weight (w, w_lo) for an fp32 cache: fp32 q [rows, d], K and
+    V; qkv [rows, 3d] and rstd [rows] are scratch of small row counts."""
+    d = n_heads * HEAD_DIM
+    _need(x, "x", F32, tile_rows(rows) * d)
+    _need(gamma, "gamma", F32, d)
+    _need(w, "w", BF16, tile_rows(3 * d) * d)
+    _need(w_lo, "w_lo", BF16, tile_rows(3 * d) * d)
+    _need(qkv, "qkv", F32, rows * 3 * d)
+    if qkv.dim() != 2 or qkv.shape[1] != 3 * d:
+        raise ValueError(f"qkv must be [rows, {3 * d}]")
+    _need(rstd, "rstd", F32, rows)
+    _need(pos, "pos", I64, rows * 3)
+    _need(rope_tab, "rope_tab", F32)
+    _need(q_out, "q_out", F32, rows * d)
+    for name, c in (("k_cache", k_cache), ("v_cache", v_cache)):
+        _need(c, name, F32)
+        if c.dim() != 4 or c.shape[1] != n_heads or c.shape[3] != 64:
+            raise ValueError(f"{name} must be [batch, n_heads, slots, 64]")
+    batch, slots = k_cache.shape[0], k_cache.shape[2]
+    if (token_row is None) != (token_slot is None):
+        raise ValueError("token_row and token_slot go together")
+    if token_row is not None:
+        _need(token_row, "token_row", I32, rows)
+        _need(token_slot, "token_slot", I32, rows)
+    elif seq * batch != rows:
+        raise ValueError("unpacked rows need rows == batch * seq")
+    mx, my, mz, px, py, pz = rope_geom
+    _lib.check(_lib.lib().mdl_prefill_gemm_norm_qkv_f32w(
+        _p(x), _p(gamma), eps, _p(w), _p(w_lo), rows, n_heads, _p(qkv), 3 * d, _p(rstd), _p(pos),
+        _p(rope_tab), mx, my, mz, px, py, pz, q_scale, _p(q_out), _p(k_cache), _p(v_cache), slots,
+        batch, seq, _p(token_row), _p(token_slot), _stream()), "mdl_prefill_gemm_norm_qkv_f32w")
 
 
 def tile_f32(x: torch.Tensor) -> torch.Tensor:

@@ -428,3 +428,63 @@ def test_fp32_weight_forms(k):
     m = 640                                              # on K5: another order of the sums
     store = forms(m)[0]
     assert rel(store, acc[:m]) < 2e-6
+
+
+def _f32w_qkv_inputs(m, H, seed):
+    d = 64 * H
+    g = torch.Generator(DEV).manual_seed(seed)
+    wh, wl = split(0.05 * torch.randn(3 * d, d, generator=g, device=DEV))
+    x = K().tile_f32(torch.randn(m, d, generator=g, device=DEV))
+    gam = 1 + 0.1 * torch.randn(d, generator=g, device=DEV)
+    pos = torch.randint(-2, 40, (m, 3), generator=g, device=DEV)   # clamped past the table's ends
+    return x, gam, K().tile_matrix(wh), K().tile_matrix(wl), pos, *_rope()
+
+
+@pytest.mark.parametrize("H", [3, 4, 12])
+@pytest.mark.parametrize("m", [1, 640, 641, 1100, 4097, 12345])
+@pytest.mark.parametrize("packed", [False, True])
+def test_norm_qkv_of_fp32_weights(m, H, packed):
+    """The fp32 qkv epilogue against the E_STORE form and K2, bit for bit; a packed list with
+    tokens that have no slot, in a cache whose other slots stay as they were."""
+    d = 64 * H
+    x, gam, w, wl, pos, tab, geom = _f32w_qkv_inputs(m, H, m + H)
+    qkv, rs = torch.empty(m, 3 * d, device=DEV), torch.empty(m, device=DEV)
+    K().prefill_gemm_norm_f32w(x, gam, 1e-5, w, wl, qkv, rs, d)
+    full = lambda *s: torch.full(s, 7.0, device=DEV)  # noqa: E731
+    B, slots = (5, m + 3) if packed else (1, m + 3)
+    want = full(m, d), full(B, H, slots, 64), full(B, H, slots, 64)
+    got = full(m, d), full(B, H, slots, 64), full(B, H, slots, 64)
+    scratch = torch.empty(m, 3 * d, device=DEV), torch.empty(m, device=DEV)
+    if packed:
+        row = torch.arange(m, device=DEV, dtype=torch.int32) * 5 // m
+        slot = torch.arange(m, device=DEV, dtype=torch.int32) + 2
+        slot[::7] = -1
+        K().qkv_rope_cache_packed(qkv, rs, pos, tab, geom, row, slot, H, 0.125, *want)
+        K().prefill_gemm_norm_qkv_f32w(x, gam, 1e-5, w, wl, m, H, *scratch, pos, tab, geom, 0.125,
+                                       *got, token_row=row, token_slot=slot)
+    else:
+        K().qkv_rope_cache(qkv, rs, pos, tab, geom, 1, m, H, 0.125, *want, slot0=0)
+        K().prefill_gemm_norm_qkv_f32w(x, gam, 1e-5, w, wl, m, H, *scratch, pos, tab, geom, 0.125,
+                                       *got, seq=m)
+    for name, a, b in zip("q K V".split(), got, want):
+        assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("m,H", [(1, 4), (16, 12), (17, 3), (250, 20)])
+@pytest.mark.parametrize("t", [0, 5, 9])
+def test_decode_norm_qkv_of_fp32_weights(m, H, t):
+    """K5's fp32 qkv epilogue against gemm_norm and K2, bit for bit, in slot t of 10 alone."""
+    d = 64 * H
+    x, gam, w, wl, pos, tab, geom = _f32w_qkv_inputs(m, H, m + t)
+    qkv, rs = torch.empty(m, 3 * d, device=DEV), torch.empty(m, device=DEV)
+    slot = torch.tensor([t], dtype=torch.int32, device=DEV)
+    for tile in range(0, 7):
+        full = lambda *s: torch.full(s, 7.0, device=DEV)  # noqa: E731
+        want = full(m, d), full(m, H, 10, 64), full(m, H, 10, 64)
+        got = full(m, d), full(m, H, 10, 64), full(m, H, 10, 64)
+        K().gemm_norm(x, gam, 1e-5, w, qkv, rs, d, tile=tile, w_lo=wl)
+        K().qkv_rope_cache(qkv, rs, pos, tab, geom, m, 1, H, 0.125, *want, slot_dev=slot)
+        K().gemm_norm_qkv(x, gam, 1e-5, w, m, H, None, pos, tab, geom, 0.125, *got,
+                          slot_dev=slot, tile=tile, w_lo=wl)
+        for name, a, b in zip("q K V".split(), got, want):
+            assert torch.equal(a, b), f"{name} at tile {tile}"

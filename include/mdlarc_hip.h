@@ -114,6 +114,18 @@ int mdl_embed_rmsnorm(const int64_t* ids, const int64_t* example_ids, const void
                       uint16_t* xs_out, float* rstd_out, int layout, void* stream);
 
 /*
+ * x of mdl_embed_rmsnorm (fp32 tile layout, no norm outputs) for a packed token list: row m is
+ * token gather[m] of the flat [batch, seq] ids and belongs to batch row token_row[m], whose example
+ * id it takes; pos_out[m] = pos[gather[m]] (x, y, z).  x_out holds ceil(n_tokens / 16) * 16 rows;
+ * d a multiple of 32.  Indexes are clamped into range (callers build them).
+ */
+int mdl_embed_packed(const int64_t* ids, const int64_t* pos, const int64_t* example_ids,
+                     const void* tok_table, const void* ex_table, int table_dtype, int vocab,
+                     int n_examples, int batch, int seq, int n_tokens, const int32_t* gather,
+                     const int32_t* token_row, int d, float* x_out, int64_t* pos_out,
+                     void* stream);
+
+/*
  * Decode-step entry: grid position of the token each row just emitted, then K1 on that token.
  * Replaces: GridStateUpdater.update (src/inference.py:127-168) followed by the embedding and
  *           blocks[0].ln1 of _decode_step (src/inference.py:433-437).
@@ -446,6 +458,8 @@ int mdl_prefill_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps
  */
 int mdl_tile_matrix(const uint16_t* src, int64_t ld, int rows, int cols, uint16_t* dst,
                     void* stream);
+/* Rows [r0, r1) of a bf16 matrix in MDL_LAYOUT_TILES to zero; cols a multiple of 32. */
+int mdl_zero_tiled_rows(uint16_t* buf, int r0, int r1, int cols, void* stream);
 
 /*
  * K4a -- prefill / full-sequence attention on bf16 MFMA (flash style, online softmax).

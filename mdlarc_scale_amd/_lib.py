@@ -36,6 +36,8 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "mdl_error_string": (ctypes.c_char_p, [c_int]),
     "mdl_embed_rmsnorm": (c_int, [P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P,
                                   c_float, P, P, P, c_int, P]),
+    "mdl_embed_packed": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P,
+                                 c_int, P, P, P]),
     "mdl_decode_embed": (c_int, [P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, c_float, P,
                                  P, P, c_int, c_int, P, P, P, P, P, c_int, P]),
     "mdl_add_rmsnorm": (c_int, [P, P, P, c_int, c_int, P, c_float, P, P, c_int, P]),
@@ -86,6 +88,7 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "mdl_prefill_gemm_norm_qkv_f32w": (c_int, [P, P, c_float, P, P, c_int, c_int, P, c_int64, P, P,
                                                P, c_int, c_int, c_int, c_int, c_int, c_int,
                                                c_float, P, P, P, c_int, c_int, c_int, P, P, P]),
+    "mdl_zero_tiled_rows": (c_int, [P, c_int, c_int, c_int, P]),
     "mdl_tile_matrix": (c_int, [P, c_int64, c_int, c_int, P, P]),
     "mdl_attn_prefill": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, c_int, P,
                                  c_int, P]),

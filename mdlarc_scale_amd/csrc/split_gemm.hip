@@ -513,6 +513,16 @@ __global__ void tile_matrix_kernel(const uint16_t* __restrict__ src, int64_t ld,
   *reinterpret_cast<uint4*>(dst + 8 * q) = v;
 }
 
+// rows [r0, r0 + n) of a tiled bf16 matrix to zero: one thread per 8 columns of a row
+__global__ void zero_tiled_rows_kernel(uint16_t* __restrict__ buf, int r0, int64_t chunks,
+                                       int cols) {
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (q >= chunks) return;
+  const int64_t r = q / (cols / 8);
+  const int col = 8 * static_cast<int>(q - r * (cols / 8));
+  *reinterpret_cast<uint4*>(buf + tile_off(r0 + r, col, cols)) = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // common host checks of the tiled decode entries: k a positive multiple of 32, n of 16
 inline bool decode_shape_ok(int m, int n, int k, int tile) {
   return m >= 0 && n >= 0 && k > 0 && k % 32 == 0 && n % 16 == 0 && tile >= 0 &&
@@ -748,5 +758,18 @@ extern "C" int mdl_tile_matrix(const uint16_t* src, int64_t ld, int rows, int co
   if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
   hipLaunchKernelGGL(tile_matrix_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), src, ld, rows, cols, chunks, dst);
+  return launch_status();
+}
+
+extern "C" int mdl_zero_tiled_rows(uint16_t* buf, int r0, int r1, int cols, void* stream) {
+  if (!buf) return MDL_ERR_NULL;
+  if (r0 < 0 || r1 < r0 || cols <= 0 || cols % 32 != 0) return MDL_ERR_SHAPE;
+  if (!aligned16(buf)) return MDL_ERR_ALIGN;
+  if (r0 == r1) return MDL_OK;
+  const int64_t chunks = static_cast<int64_t>(r1 - r0) * (cols / 8);
+  const int64_t blocks = (chunks + 255) / 256;
+  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
+  hipLaunchKernelGGL(zero_tiled_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), buf, r0, chunks, cols);
   return launch_status();
 }

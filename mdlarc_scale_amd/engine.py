@@ -88,15 +88,6 @@ def tiles_supported(d_model: int, d_ff: int) -> bool:
     return d_model % 32 == 0 and d_ff % 32 == 0
 
 
-def zero_tiled_rows(buf: torch.Tensor, r0: int, r1: int, cols: int) -> None:
-    """Zero rows [r0, r1) of a bf16 [rows, cols] matrix in the MFMA tile layout: each row is
-    cols / 8 chunks of 8 contiguous elements (tile_off of include/mdlarc_hip.h)."""
-    m = torch.arange(r0, r1, device=buf.device)[:, None]
-    q = torch.arange(cols // 8, device=buf.device)[None, :]
-    chunk = 64 * ((m >> 4) * (cols >> 5) + (q >> 2)) + 16 * (q & 3) + (m & 15)
-    buf.view(-1, 8)[chunk.reshape(-1)] = 0
-
-
 # Activation parts of the bf16 form's prompt MLP on K6 (2: split hi | lo, as every other
 # projection; 1: the lo term dropped, as the reference's bf16 model rounds a projection's input
 # to bf16).  PROMPT_GATE_UP_PARTS is the gate / up input's (bf16(ln2(x)) at 1),
@@ -455,16 +446,22 @@ class HipEngine:
         H, d = cfg.n_heads, cfg.d_model
         tok, ex = self._tables()
         use_ex = ex_ids is not None and cfg.use_example_embedding
-        ids_p = ids.reshape(-1).index_select(0, pk.gather)
-        pos_p = pos.reshape(-1, 3).index_select(0, pk.gather)
-        ex_p = ex_ids.reshape(-1).index_select(0, pk.token_row) if use_ex else None
         fused = sc.fused
         nx = fused or sc.f32   # ln1 inside the projection: the embedding writes x only
-        K.embed_rmsnorm(ids_p, ex_p, tok, ex if use_ex else None, 1, W.ln1[0], W.eps, sc.x,
-                        None if nx else sc.xs, None if nx else sc.rstd, tiled=nx)
+        if nx:
+            pos_p = torch.empty(pk.n_tokens, 3, dtype=pos.dtype, device=pos.device)
+            K.embed_packed(ids.contiguous(), pos.contiguous(),
+                           ex_ids.reshape(-1) if use_ex else None, tok, ex if use_ex else None,
+                           pk.gather, pk.token_row, sc.x, pos_p)
+        else:
+            ids_p = ids.reshape(-1).index_select(0, pk.gather)
+            pos_p = pos.reshape(-1, 3).index_select(0, pk.gather)
+            ex_p = ex_ids.reshape(-1).index_select(0, pk.token_row) if use_ex else None
+            K.embed_rmsnorm(ids_p, ex_p, tok, ex if use_ex else None, 1, W.ln1[0], W.eps, sc.x,
+                            sc.xs, sc.rstd)
         if pk.n_tokens > pk.n_valid:   # padding queries: no visible key, attention output 0
             if nx:
-                zero_tiled_rows(sc.attn, pk.n_valid, pk.n_tokens, 2 * d)
+                K.zero_tiled_rows(sc.attn, pk.n_valid, pk.n_tokens, 2 * d)
             else:
                 sc.attn[pk.n_valid:pk.n_tokens].zero_()
         qs = softmax_scale(d // H)          # the exact lead pass (K4c)

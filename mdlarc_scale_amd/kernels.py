@@ -106,6 +106,31 @@ def embed_rmsnorm(ids: torch.Tensor, example_ids: torch.Tensor | None, tok_table
         _layout(tiled), _stream()), "mdl_embed_rmsnorm")
 
 
+def embed_packed(ids: torch.Tensor, pos: torch.Tensor, example_ids: torch.Tensor | None,
+                 tok_table: torch.Tensor, ex_table: torch.Tensor | None, gather: torch.Tensor,
+                 token_row: torch.Tensor, x_out: torch.Tensor, pos_out: torch.Tensor) -> None:
+    """x = tok[ids] + ex[example_ids] of a packed token list in the fp32 tile layout: row m is
+    token gather[m] of the flat [B, S] ids, its batch row token_row[m]; pos_out[m] its position."""
+    rows, (batch, seq), (vocab, d) = gather.numel(), ids.shape, tok_table.shape
+    _need(ids, "ids", I64)
+    _need(pos, "pos", I64, ids.numel() * 3)
+    _need(example_ids, "example_ids", I64, batch, optional=True)
+    _need(tok_table, "tok_table", tok_table.dtype)
+    if example_ids is not None:
+        _need(ex_table, "ex_table", tok_table.dtype)
+        if ex_table.shape[1] != d:
+            raise ValueError("example table width differs from token table width")
+    _need(gather, "gather", I32)
+    _need(token_row, "token_row", I32, rows)
+    _need(x_out, "x_out", F32, tile_rows(rows) * d)
+    _need(pos_out, "pos_out", I64, rows * 3)
+    n_ex = ex_table.shape[0] if ex_table is not None else 0
+    _lib.check(_lib.lib().mdl_embed_packed(
+        _p(ids), _p(pos), _p(example_ids), _p(tok_table), _p(ex_table),
+        table_dtype_code(tok_table), vocab, n_ex, batch, seq, rows, _p(gather), _p(token_row), d,
+        _p(x_out), _p(pos_out), _stream()), "mdl_embed_packed")
+
+
 def decode_embed(token: torch.Tensor, example_ids: torch.Tensor | None, tok_table: torch.Tensor,
                  ex_table: torch.Tensor | None, gamma: torch.Tensor, eps: float,
                  gx: torch.Tensor, gy: torch.Tensor, in_out: torch.Tensor, pos_out: torch.Tensor,
@@ -677,6 +702,13 @@ def untile_f32(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     """The inverse of tile_f32: the [rows, cols] matrix."""
     v = t[:tile_rows(rows) * cols].view(-1, cols // 32, 2, 4, 16, 4)
     return v.permute(0, 4, 1, 3, 2, 5).reshape(-1, cols)[:rows]
+
+
+def zero_tiled_rows(buf: torch.Tensor, r0: int, r1: int, cols: int) -> None:
+    """Zero rows [r0, r1) of a bf16 [rows, cols] matrix in the MFMA tile layout."""
+    _need(buf, "buf", BF16, tile_rows(r1) * cols)
+    _lib.check(_lib.lib().mdl_zero_tiled_rows(_p(buf), r0, r1, cols, _stream()),
+               "mdl_zero_tiled_rows")
 
 
 def untile_matrix(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:

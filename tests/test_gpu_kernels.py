@@ -1409,3 +1409,69 @@ def test_gemm_split_residual(m, n, k):
             # padding rows of the last row block stay as they were
             full = K().untile_f32(xt, K().tile_rows(m), n)
             assert torch.equal(full[m:], K().untile_f32(pad, K().tile_rows(m), n)[m:])
+
+
+@pytest.mark.parametrize("d", [32, 128, 800, 1280, 2048])
+@pytest.mark.parametrize("table_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("with_ex", [True, False])
+def test_embed_x_alone_in_tiles(d, table_dtype, with_ex):
+    """x alone (no norm outputs) in the tile layout, rows in order and as a packed token list, equals
+    the row kernel's x bit for bit, and the padding rows of the last 16 stay as they were; the
+    same for rows zeroed in a bf16 tile layout."""
+    g = torch.Generator().manual_seed(d)
+    tok = torch.randn(14, d, generator=g).to(table_dtype).to(DEV)
+    ex = torch.randn(5, d, generator=g).to(table_dtype).to(DEV) if with_ex else None
+    gamma = torch.ones(d, device=DEV)
+    for B, S in ((1, 1), (3, 5), (2, 16), (7, 33), (31, 34)):
+        ids = torch.randint(-2, 17, (B, S), generator=g).to(DEV)      # clamped into the table
+        exi = torch.randint(0, 5, (B,), generator=g).to(DEV) if with_ex else None
+        pos = torch.randint(0, 30, (B, S, 3), generator=g).to(DEV)
+        xr = torch.empty(B * S, d, device=DEV)
+        K().embed_rmsnorm(ids.reshape(-1), exi, tok, ex, S, gamma, 1e-5, xr, None, None)
+        pad = torch.full((K().tile_rows(B * S), d), 7.0, device=DEV)
+        pad[:B * S] = xr
+        got = torch.full((pad.numel(),), 7.0, device=DEV)
+        K().embed_rmsnorm(ids.reshape(-1), exi, tok, ex, S, gamma, 1e-5, got, None, None,
+                          tiled=True)
+        assert torch.equal(got, K().tile_f32(pad))
+        at = torch.randperm(B * S, generator=g)[:max(1, B * S - 2)].to(DEV)
+        n = at.numel()
+        pad = torch.full((K().tile_rows(n), d), 7.0, device=DEV)
+        pad[:n] = xr[at]
+        got = torch.full((pad.numel(),), 7.0, device=DEV)
+        where = torch.full((n + 1, 3), 99, dtype=torch.int64, device=DEV)
+        K().embed_packed(ids, pos, exi, tok, ex, at.int(), (at // S).int(), got, where[:n])
+        assert torch.equal(got, K().tile_f32(pad))
+        assert torch.equal(where[:n], pos.reshape(-1, 3)[at]) and bool((where[n] == 99).all())
+        m = K().tile_rows(B * S)
+        a = torch.randn(m, d, generator=g).to(torch.bfloat16).to(DEV)
+        t = K().tile_matrix(a)
+        r0, r1 = B * S // 3, B * S
+        K().zero_tiled_rows(t, r0, r1, d)
+        a[r0:r1] = 0
+        assert torch.equal(t, K().tile_matrix(a))
+
+
+@pytest.mark.parametrize("S", [1, 63, 65, 300])
+@pytest.mark.parametrize("causal", [True, False])
+def test_attn_prefill_block_sizes_agree(S, causal):
+    """A row's output is the same bits in a small launch (64-query blocks) and in a large one
+    (128-query blocks), with a start, a hole and a row of no valid key."""
+    H, n = 4, 640 // (4 * -(-S // 128)) + 1
+    g = torch.Generator().manual_seed(S)
+    rows = 5
+    pm = torch.ones(rows, S, dtype=torch.uint8)
+    pm[1, :S // 3] = 0
+    pm[2, S // 2:S // 2 + 9] = 0
+    pm[3] = 0
+    kv = torch.tensor([0, S // 3, 0, S, 0], dtype=torch.int32)
+    q = bf(torch.randn(rows, S, H * 64, generator=g) * 0.3)
+    kc, vc = (bf(torch.randn(rows, H, S + 3, 64, generator=g)) for _ in range(2))
+    outs = []
+    for idx in (torch.arange(rows), torch.arange(max(n, rows)) % rows):
+        B = idx.numel()
+        out = torch.empty(B * S, 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+        K().attn_prefill(q[idx].to(DEV).view(B * S, -1), kc[idx].to(DEV), vc[idx].to(DEV), B, S, H,
+                         pm[idx].to(DEV), kv[idx].to(DEV), causal, out)
+        outs.append(out.view(B, S, -1))
+    assert torch.equal(outs[1], outs[0][torch.arange(outs[1].shape[0]) % rows])

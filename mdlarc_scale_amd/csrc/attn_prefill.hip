@@ -1,7 +1,8 @@
 // K4a -- prefill / full-sequence attention on bf16 MFMA (gfx950 v_mfma_f32_16x16x32_bf16).
 //
 // Block = 4 wavefronts = 128 queries of one (b, h); wave w owns queries q0+32w .. q0+32w+31 as
-// two groups of 16 (j = 0, 1).  Working with S^T = K Q^T instead of S makes the MFMA accumulator
+// two groups of 16 (j = 0, 1); small launches take one group per wave (QG = 1), 64 queries a
+// block.  Working with S^T = K Q^T instead of S makes the MFMA accumulator
 // of the scores (lane = one query, 4 keys per 16-key block) exactly the B-operand layout P^T
 // needs in O^T = V^T P^T, so the probabilities never leave registers:
 //   score block nb (keys 16nb..16nb+15), lane (c = lane%16, g = lane/16) holds keys 16nb+4g+i,
@@ -57,8 +58,6 @@
 
 namespace mdl {
 
-constexpr int kQW = 32;          // queries per wave
-constexpr int kBM = 4 * kQW;     // queries per block
 constexpr int kBN = 64;          // keys per tile
 constexpr int kXcds = 8;
 constexpr int kTileBytes = kBN * kHeadDim * 2;   // one K or V tile: 64 rows of 128 bytes
@@ -72,12 +71,14 @@ __device__ __forceinline__ int tile_swz(int r) {
   return ((r ^ (r >> 3)) & 1) | (((r ^ (r >> 2)) & 1) << 1) | (((r >> 1) & 1) << 2);
 }
 
+template <int QG>
 __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int S, int H, int slots, const uint8_t* __restrict__ kmask,
     const uint8_t* __restrict__ row_holes, const int32_t* __restrict__ kv_start,
     const int32_t* __restrict__ q_offset, int causal, uint16_t* __restrict__ out, int out_tiled,
     int nqt, int n_bh) {
+  constexpr int kQW = 16 * QG, kBM = 4 * kQW;   // queries per wave, per block
   const int slot = blockIdx.x / kXcds;
   const int kq = slot / nqt;
   const int bh = blockIdx.x % kXcds + kXcds * kq;
@@ -101,10 +102,10 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t Vs[2][kBN * kHeadDim];
 
   const int wq0 = q0 + kQW * wave;
-  int qi[2];
-  bf16x8_t qf[2][2];
+  int qi[QG];
+  bf16x8_t qf[QG][2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < QG; ++j) {
     qi[j] = wq0 + 16 * j + c16;
     if (qi[j] < S && qi[j] >= qlo) {
       const uint16_t* qp = q + ((qbase + qi[j]) * H + h) * kHeadDim;
@@ -141,8 +142,8 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
   }
   auto issue = [&](int kt, int st) {
     if (kt >= kstart && kt + kBN <= S) {
-      const uint16_t* kb = Kg + static_cast<int64_t>(kt) * kHeadDim;
-      const uint16_t* vb = Vg + static_cast<int64_t>(kt) * kHeadDim;
+      const uint16_t* kb = scalar_ptr(Kg + static_cast<int64_t>(kt) * kHeadDim);
+      const uint16_t* vb = scalar_ptr(Vg + static_cast<int64_t>(kt) * kHeadDim);
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
         const uint32_t run = st * kTileBytes + (4 * r + wave) * 1024;
@@ -191,10 +192,12 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
   // Per query: negm = -m, the negated reference maximum (0 before the first visible key), and
   // thr, the tile maximum (relative to m) that moves the reference: -inf before the first
   // visible key, then the gap.  Both change only when the reference moves.
-  float negm[2] = {0.f, 0.f}, thr[2] = {-INFINITY, -INFINITY};
-  f32x4_t lsum[2], o[2][4];
+  float negm[QG], thr[QG];
+  f32x4_t lsum[QG], o[QG][4];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < QG; ++j) {
+    negm[j] = 0.f;
+    thr[j] = -INFINITY;
     lsum[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[j][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -204,10 +207,10 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
     // S^T = K Q^T: 4 blocks of 16 keys for both query groups.  Every accumulator starts at -m,
     // its query's reference maximum (0 before the query's first visible key); q carries log2(e),
     // so the MFMA yields the exponents s - m of the log2-domain softmax directly.
-    f32x4_t sc[2][4];
-    f32x4_t minit[2];
+    f32x4_t sc[QG][4];
+    f32x4_t minit[QG];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QG; ++j) {
       minit[j] = f32x4_t{negm[j], negm[j], negm[j], negm[j]};
     }
 #pragma unroll
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
         const bf16x8_t a =
             as_bf16x8(*reinterpret_cast<const uint4*>(Kt + kofs[kk] + 2048 * nb));
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < QG; ++j)
           sc[j][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[j][kk],
                                                               kk == 0 ? minit[j] : sc[j][nb],
                                                               0, 0, 0);
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
     const bool full = (mw == ~0ull) && (!causal || kt + kBN - 1 <= wq0);
     if (!full) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < QG; ++j) {
         uint64_t vis = mw;
         if (causal) {
           const int x = qi[j] - kt;    // offset of the last key query qi[j] may see
@@ -245,9 +248,9 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
       }
     }
 
-    bf16x8_t pb[2][2];
+    bf16x8_t pb[QG][2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QG; ++j) {
       float lmax = -INFINITY;
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb)
@@ -299,12 +302,14 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        o[0][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[db], pb[0][kk], o[0][db], 0, 0, 0);
-        o[1][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[db], pb[1][kk], o[1][db], 0, 0, 0);
-      }
-      lsum[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[0][kk], lsum[0], 0, 0, 0);
-      lsum[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[1][kk], lsum[1], 0, 0, 0);
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int j = 0; j < QG; ++j)
+          o[j][db] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[db], pb[j][kk], o[j][db], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < QG; ++j)
+        lsum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[j][kk], lsum[j], 0, 0, 0);
     }
   };
 
@@ -348,7 +353,7 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
   // or in the bf16 MFMA tile layout, where each 4-column group stays contiguous)
   const int64_t d = static_cast<int64_t>(H) * kHeadDim;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < QG; ++j) {
     if (qi[j] >= S || qi[j] < qlo) continue;
     const float l = lsum[j][0];     // every row of the ones product holds the query's sum
     const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -539,6 +544,14 @@ using namespace mdl;
 
 namespace mdl {
 
+// Launches of up to this many 128-query blocks run as twice as many 64-query ones, a wave holding
+// one query group: with a block or two per CU a tile's time is one wave's chain of MFMAs and
+// exponentials, which half the queries halve (same bits per query).  Causal, us at two groups / at
+// one: 72 blocks 16.7 / 11.1, 256 21.6 / 17.4, 576 23.9 / 21.5; above, each key tile read from LDS
+// for half as many queries costs as much (1,640: 179 / 186; without the causal limit 576: 28.6 /
+// 28.4 and 820: 174 / 202).
+constexpr int kOneGroupBlocks = 640;
+
 int launch_prefill(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
                    int batch, int seq, int n_heads, int head_dim, int cache_slots,
                    const uint8_t* key_mask, const uint8_t* row_holes, const int32_t* kv_start,
@@ -554,10 +567,12 @@ int launch_prefill(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v
     return MDL_ERR_ALIGN;
   if (batch == 0 || seq == 0) return MDL_OK;
   const int64_t heads = static_cast<int64_t>(batch) * n_heads;
-  const int64_t nqt = (seq + kBM - 1) / kBM;
+  const bool small = heads * ((seq + 127) / 128) <= kOneGroupBlocks;
+  const int64_t nqt = small ? (seq + 63) / 64 : (seq + 127) / 128;
   const int64_t blocks = (heads + kXcds - 1) / kXcds * kXcds * nqt;
   if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
-  attn_prefill_kernel<<<static_cast<unsigned>(blocks), 256, 0, st>>>(
+  auto* kernel = small ? attn_prefill_kernel<1> : attn_prefill_kernel<2>;
+  kernel<<<static_cast<unsigned>(blocks), 256, 0, st>>>(
       q, k_cache, v_cache, seq, n_heads, cache_slots, key_mask, row_holes, kv_start, q_offset,
       causal ? 1 : 0, out, out_layout == MDL_LAYOUT_TILES ? 1 : 0, static_cast<int>(nqt),
       static_cast<int>(heads));

@@ -47,6 +47,15 @@ __device__ __forceinline__ void dma16_sbase(const void* base, uint32_t off, uint
                :: "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
+// A wave-uniform pointer in scalar registers, also where the compiler computed it in vector ones.
+template <typename T>
+__device__ __forceinline__ const T* scalar_ptr(const T* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32));
+  return reinterpret_cast<const T*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
 // dma16_sbase without the memory clobber: the compiler may move its own memory accesses across
 // the copy.  For a kernel that spreads its copies over the work on the stage before: the copy's
 // stage is neither read nor written by the kernel between its two barriers (asm volatile with the

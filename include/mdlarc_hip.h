@@ -633,6 +633,57 @@ int mdl_attn_decode_f32(const float* q, const float* k_cache, const float* v_cac
                         int split_len, uint16_t* out, int out_layout, void* stream);
 
 /*
+ * Every layer of a prompt or decode step from one call (host code over the entries above, which
+ * check their arguments as always; the first error ends the call).  Activations are in the tile
+ * layouts; f32: the fp32 form (fp32 q and caches, every *_lo given).
+ *   mdl_prompt_layers: per layer mdl_prefill_gemm_norm_qkv, mdl_attn_prefill (_packed with
+ *     q_offset), mdl_attn_prefill_lead when causal, mdl_prefill_gemm_split_residual,
+ *     mdl_prefill_gemm_norm_swiglu, mdl_prefill_gemm_split_residual, or their _f32w / _f32 forms;
+ *     mask is the key mask [batch, seq].
+ *   mdl_decode_layers: per layer mdl_gemm_norm_qkv, mdl_attn_decode, mdl_gemm_split_residual,
+ *     mdl_gemm_norm_swiglu, mdl_gemm_split_residual, with rows == batch; mask is the prompt mask
+ *     [batch, seq], the token's slot is *slot_dev.
+ * Replaces: the layer loops of _prefill / _decode_step (src/inference.py:397-415, :437-456) and
+ *           TinyTransformer.forward (src/transformer.py:591-604).
+ */
+typedef struct {
+  const float *ln1, *ln2;
+  const uint16_t *qkv, *qkv_lo, *out, *out_lo, *gu, *gu_lo, *down, *down_lo;
+  const float *b_gate, *b_up, *b_down;
+  void *k_cache, *v_cache;   /* [batch, n_heads, slots, 64] */
+  int64_t slots;
+} mdl_layer;
+
+typedef struct {
+  const mdl_layer* layers;
+  float* x;
+  void* q;
+  float *qkv, *rstd;
+  uint16_t *attn, *h;
+  const int64_t* pos;
+  const float* rope_tab;
+  const uint8_t *mask, *row_holes;
+  const int32_t *kv_start, *token_row, *token_slot, *q_offset;
+  const int32_t *slot_dev, *row_order;
+  float* ws;
+  int64_t ws_bytes;
+  int n_layers, f32, rows, batch, seq, n_heads, d_ff;
+  int max_x, max_y, max_z, px, py, pz;
+  int causal, lead, gate_up_parts, down_parts, split_len;
+  float eps, q_scale, lead_scale;
+} mdl_stack;
+
+int mdl_prompt_layers(const mdl_stack* stack, void* stream);
+int mdl_decode_layers(const mdl_stack* stack, void* stream);
+/*
+ * Smallest and largest of two id lists, per block of the launch: out[4][blocks] (device memory) =
+ * ids min, ids max, example ids min, example ids max (INT64_MAX / INT64_MIN where a block saw
+ * none).  The range check of a call's inputs with one read back.  1 <= blocks <= 1024.
+ */
+int mdl_id_range(const int64_t* ids, int64_t n_ids, const int64_t* example_ids,
+                 int64_t n_examples, int blocks, int64_t* out, void* stream);
+
+/*
  * Final RMSNorm + LM head + greedy argmax.
  * Replaces: model.lm_head(model.ln_f(x)) in _prefill / _decode_step (src/inference.py:417-424,
  *           :459) including the x[b, lengths-1] row pick, and logits.argmax(-1)

@@ -29,7 +29,28 @@ class LogitConstraints(ctypes.Structure):
                 ("grid_y", c_void_p), ("shape_penalty", c_float)]
 
 
+class Layer(ctypes.Structure):
+    """``mdl_layer`` (include/mdlarc_hip.h), field for field."""
+
+    _fields_ = [(n, c_void_p) for n in (
+        "ln1", "ln2", "qkv", "qkv_lo", "out", "out_lo", "gu", "gu_lo", "down", "down_lo", "b_gate",
+        "b_up", "b_down", "k_cache", "v_cache")] + [("slots", c_int64)]
+
+
+class Stack(ctypes.Structure):
+    """``mdl_stack`` (include/mdlarc_hip.h), field for field."""
+
+    _fields_ = [("layers", ctypes.POINTER(Layer))] + [(n, c_void_p) for n in (
+        "x", "q", "qkv", "rstd", "attn", "h", "pos", "rope_tab", "mask", "row_holes", "kv_start",
+        "token_row", "token_slot", "q_offset", "slot_dev", "row_order", "ws")] + [
+        ("ws_bytes", c_int64)] + [(n, c_int) for n in (
+            "n_layers", "f32", "rows", "batch", "seq", "n_heads", "d_ff", "max_x", "max_y",
+            "max_z", "px", "py", "pz", "causal", "lead", "gate_up_parts", "down_parts",
+            "split_len")] + [(n, c_float) for n in ("eps", "q_scale", "lead_scale")]
+
+
 CONS = ctypes.POINTER(LogitConstraints)
+STACK = ctypes.POINTER(Stack)
 # argtypes per entry point, in header order
 SIGNATURES: dict[str, tuple[object, list]] = {
     "mdl_version": (c_int, []),
@@ -89,6 +110,9 @@ SIGNATURES: dict[str, tuple[object, list]] = {
                                                P, c_int, c_int, c_int, c_int, c_int, c_int,
                                                c_float, P, P, P, c_int, c_int, c_int, P, P, P]),
     "mdl_zero_tiled_rows": (c_int, [P, c_int, c_int, c_int, P]),
+    "mdl_prompt_layers": (c_int, [STACK, P]),
+    "mdl_decode_layers": (c_int, [STACK, P]),
+    "mdl_id_range": (c_int, [P, c_int64, P, c_int64, c_int, P, P]),
     "mdl_tile_matrix": (c_int, [P, c_int64, c_int, c_int, P, P]),
     "mdl_attn_prefill": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, c_int, P,
                                  c_int, P]),

@@ -35,6 +35,7 @@ SOURCES = [
     "prompt_build.hip",
     "split_gemm.hip",
     "prefill_gemm.hip",
+    "layers.hip",
 ]
 
 FLAGS = [

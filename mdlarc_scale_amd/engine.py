@@ -190,6 +190,7 @@ class PackedWeights:
         self.rope_tab = rope.device_table(device)
         self.rope_geom = (rope.max_x, rope.max_y, rope.max_z, rope.px, rope.py, rope.pz)
         self.eps = cfg.norm_eps
+        self.layers = K.layer_table(self) if self.tiles_ok else None
 
 
 @dataclass
@@ -344,9 +345,19 @@ class HipEngine:
         self._packed, self._sig = None, None
 
     def _signature(self) -> tuple:
-        return tuple((p.data_ptr(), p._version, p.dtype, p.device)
-                     for n, p in self.model.named_parameters()
-                     if not n.startswith(("token_embed", "example_embed")))
+        # every parameter outside the embedding tables, straight from the module tree:
+        # named_parameters builds a name and a set entry for each (60 us for 43 of them, this 15)
+        sig, todo = [], [self.model]
+        while todo:
+            m = todo.pop()
+            for p in m._parameters.values():
+                if p is not None:
+                    sig.append((p.data_ptr(), p._version, p.dtype, p.device))
+            for n, child in m._modules.items():
+                if child is not None and not (m is self.model and
+                                              n.startswith(("token_embed", "example_embed"))):
+                    todo.append(child)
+        return tuple(sig)
 
     def packed(self, device: torch.device) -> PackedWeights:
         sig = self._signature()
@@ -373,10 +384,11 @@ class HipEngine:
         return t.device
 
     def _validate_ids(self, ids: torch.Tensor, ex: torch.Tensor | None) -> None:
-        if ids.numel() and (int(ids.min()) < 0 or int(ids.max()) >= self.cfg.vocab_size):
+        # one kernel and one read back for both ranges
+        lo, hi, ex_lo, ex_hi = K.id_range(ids, ex)
+        if lo < 0 or hi >= self.cfg.vocab_size:
             raise IndexError("input_ids out of range of the token embedding")
-        if ex is not None and ex.numel() and (int(ex.min()) < 0 or
-                                              int(ex.max()) >= self.cfg.num_examples):
+        if ex_lo < 0 or ex_hi >= self.cfg.num_examples:
             raise IndexError("example_ids out of range of the example embedding")
 
     # -- full-sequence layers (prefill / forward) ------------------------------------------------
@@ -400,37 +412,33 @@ class HipEngine:
                         None if nx else sc.rstd, tiled=nx)
         qs = softmax_scale(d // H)          # the exact lead pass (K4c)
         qa = attention_q_scale(d // H)      # q for the attention kernels (log2-domain softmax)
+        if fused or sc.fused_f32:
+            # ln1 + qkv_proj + K2 in one launch (fp32 qkv only for the lead rows), K4a and the exact
+            # lead pass, the MLP; the fp32 form: the low weight parts, K2 into the fp32 cache and
+            # K4f (exact, so no lead pass)
+            K.prompt_layers(W, cfg, sc, kv_layers, B, S, B * S, pos, qa, qs, key_mask, row_holes,
+                            kv_start, causal, PROMPT_GATE_UP_PARTS,
+                            PROMPT_DOWN_PARTS if fused else 2)
+            return
         for li in range(cfg.n_layers):
             kc, vc = kv_layers(li)
             if sc.f32:
-                # fp32 form: projection with the low weight part, K2 into the fp32 cache, K4f (the
-                # attention is exact, so no lead pass)
-                if sc.fused_f32:
-                    K.prefill_gemm_norm_qkv_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li],
-                                                 W.qkv_lo[li], B * S, H, sc.qkv, sc.rstd, pos,
-                                                 W.rope_tab, W.rope_geom, qa, sc.q, kc, vc, seq=S)
-                else:
-                    K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
-                                w_lo=W.qkv_lo[li])
-                    K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
-                                     sc.q, kc, vc, slot0=0)
+                K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
+                            w_lo=W.qkv_lo[li])
+                K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
+                                 sc.q, kc, vc, slot0=0)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, None, B * S,
                                    causal, sc.attn, out_tiled=True)
                 self._mlp(W, li, sc)
                 continue
-            if fused:   # ln1 + qkv_proj + K2 in one launch (fp32 qkv only for the lead rows)
-                K.prefill_gemm_norm_qkv(sc.x, W.ln1[li], W.eps, W.qkv_t[li], B * S, H, sc.rstd,
-                                        sc.qkv, K.LEAD_QUERIES if causal else 0, kv_start, pos,
-                                        W.rope_tab, W.rope_geom, qa, sc.q, kc, vc, seq=S)
-            else:
-                gemm_f32(sc.xs, W.qkv[li], sc.qkv)
-                K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa,
-                                 sc.q, kc, vc, slot0=0)
+            gemm_f32(sc.xs, W.qkv[li], sc.qkv)
+            K.qkv_rope_cache(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, B, S, H, qa, sc.q, kc,
+                             vc, slot0=0)
             K.attn_prefill(sc.q, kc, vc, B, S, H, key_mask, kv_start, causal, sc.attn,
-                           out_tiled=fused, row_holes=row_holes)
+                           row_holes=row_holes)
             if causal:
                 K.attn_prefill_lead(sc.qkv, sc.rstd, pos, W.rope_tab, W.rope_geom, qs, B, S, H,
-                                    key_mask, kv_start, None, B * S, sc.attn, out_tiled=fused)
+                                    key_mask, kv_start, None, B * S, sc.attn)
             self._mlp(W, li, sc)
 
     def run_packed(self, W: PackedWeights, ids: torch.Tensor, pos: torch.Tensor,
@@ -466,65 +474,36 @@ class HipEngine:
                 sc.attn[pk.n_valid:pk.n_tokens].zero_()
         qs = softmax_scale(d // H)          # the exact lead pass (K4c)
         qa = attention_q_scale(d // H)      # q for the attention kernels (log2-domain softmax)
+        if fused or sc.fused_f32:   # as in run_prompt
+            K.prompt_layers(W, cfg, sc, kv_layers, B, S, pk.n_tokens, pos_p, qa, qs, key_mask,
+                            row_holes, kv_start, True, PROMPT_GATE_UP_PARTS,
+                            PROMPT_DOWN_PARTS if fused else 2, token_row=pk.token_row,
+                            token_slot=pk.token_slot, q_offset=pk.q_offset)
+            return
         for li in range(cfg.n_layers):
             kc, vc = kv_layers(li)
-            if sc.f32:   # fp32 form (see run_prompt)
-                if sc.fused_f32:
-                    K.prefill_gemm_norm_qkv_f32w(sc.x, W.ln1[li], W.eps, W.qkv_t[li],
-                                                 W.qkv_lo[li], pk.n_tokens, H, sc.qkv, sc.rstd,
-                                                 pos_p, W.rope_tab, W.rope_geom, qa, sc.q, kc, vc,
-                                                 token_row=pk.token_row, token_slot=pk.token_slot)
-                else:
-                    K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
-                                w_lo=W.qkv_lo[li])
-                    K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
-                                            pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
+            if sc.f32:
+                K.gemm_norm(sc.x, W.ln1[li], W.eps, W.qkv_t[li], sc.qkv, sc.rstd, d,
+                            w_lo=W.qkv_lo[li])
+                K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
+                                        pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
                 K.attn_prefill_f32(sc.q, kc, vc, B, S, H, key_mask, kv_start, pk.q_offset,
                                    pk.n_tokens, True, sc.attn, out_tiled=True)
                 self._mlp(W, li, sc)
                 continue
-            if fused:
-                K.prefill_gemm_norm_qkv(sc.x, W.ln1[li], W.eps, W.qkv_t[li], pk.n_tokens, H,
-                                        sc.rstd, sc.qkv, K.LEAD_QUERIES, kv_start, pos_p,
-                                        W.rope_tab, W.rope_geom, qa, sc.q, kc, vc,
-                                        token_row=pk.token_row, token_slot=pk.token_slot)
-            else:
-                gemm_f32(sc.xs, W.qkv[li], sc.qkv)
-                K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom,
-                                    pk.token_row, pk.token_slot, H, qa, sc.q, kc, vc)
+            gemm_f32(sc.xs, W.qkv[li], sc.qkv)
+            K.qkv_rope_cache_packed(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom, pk.token_row,
+                                    pk.token_slot, H, qa, sc.q, kc, vc)
             K.attn_prefill_packed(sc.q, kc, vc, B, S, H, key_mask, kv_start, pk.q_offset,
-                                  pk.n_valid, True, sc.attn, out_tiled=fused,
-                                  row_holes=row_holes)
+                                  pk.n_valid, True, sc.attn, row_holes=row_holes)
             K.attn_prefill_lead(sc.qkv, sc.rstd, pos_p, W.rope_tab, W.rope_geom, qs, B, S, H,
-                                key_mask, kv_start, pk.q_offset, pk.n_tokens, sc.attn,
-                                out_tiled=fused)
+                                key_mask, kv_start, pk.q_offset, pk.n_tokens, sc.attn)
             self._mlp(W, li, sc)
 
     def _mlp(self, W: PackedWeights, li: int, sc: Scratch) -> None:
         """out_proj + residual, ln2, SwiGLU MLP + residual, next norm (shared by both phases)."""
         cfg = self.cfg
         d, F = cfg.d_model, cfg.d_ff
-        if sc.fused:
-            # prompt on K6: residual adds in the out / down epilogues, ln2 in the gate / up
-            # prologue with the SwiGLU in its epilogue; the next layer's ln1 runs in its qkv
-            # launch (_qkv) and ln_f in the head kernel.  The MLP's inputs carry
-            # PROMPT_GATE_UP_PARTS / PROMPT_DOWN_PARTS parts.
-            m, parts = sc.rows, PROMPT_DOWN_PARTS
-            K.prefill_gemm_split_residual(sc.attn, W.out_t[li], sc.x, None, m, d, d, a_tiled=True)
-            K.prefill_gemm_norm_swiglu(sc.x, W.ln2[li], W.eps, W.gu_t[li], W.b_gate[li],
-                                       W.b_up[li], sc.h, m, F, d, a_parts=PROMPT_GATE_UP_PARTS,
-                                       h_parts=parts)
-            K.prefill_gemm_split_residual(sc.h, W.down_t[li], sc.x, W.b_down[li], m, d, F,
-                                          a_tiled=True, a_parts=parts)
-            return
-        if sc.fused_f32:
-            K.prefill_gemm_split_residual_f32w(sc.attn, W.out_t[li], W.out_lo[li], sc.x, None,
-                                               sc.rows, d, d)
-            K.prefill_gemm_norm_swiglu_f32w(sc.x, W.ln2[li], W.eps, W.gu_t[li], W.gu_lo[li],
-                                            W.b_gate[li], W.b_up[li], sc.h, sc.rows, F, d)
-            K.prefill_gemm_split_residual_f32w(sc.h, W.down_t[li], W.down_lo[li], sc.x,
-                                               W.b_down[li], sc.rows, d, F)
-            return
         if sc.tiled:
             # decode: three K5 launches, the residual adds in the epilogues and ln2 in the
             # gate / up prologue; the next layer's ln1 runs in its qkv launch (gemm_norm) and

@@ -352,31 +352,19 @@ class Generator:
         H = cfg.n_heads
         qs = attention_q_scale(cfg.d_model // H)   # q for the attention kernels
         slot = st.counters[0:1]
+        if sc.tiled:
+            # K5: ln1 in the projection's prologue, K2 (RoPE, q scale, K/V into slot t) in its
+            # epilogue; K4b reads q and the cache (the fp32 form: the low weight parts, K4f)
+            K.decode_layers(W, cfg, sc, st.cache.layer, B, st.S, st.pos, qs, st.pmask, st.holes,
+                            st.kv_start, slot, st.order, st.ws, st.split_len)
+            return
         for li in range(cfg.n_layers):
             kc, vc = st.cache.layer(li)
-            if sc.f32:
-                # fp32 form: projection with the low weight part, K2 of the token into slot t
-                # of the fp32 cache in its epilogue, K4f over slots [kv_start, t]
-                K.gemm_norm_qkv(sc.x, W.ln1[li], W.eps, W.qkv_t[li], B, H, None, st.pos,
-                                W.rope_tab, W.rope_geom, qs, sc.q, kc, vc, slot_dev=slot,
-                                w_lo=W.qkv_lo[li])
-                K.attn_decode_f32(sc.q, kc, vc, B, H, st.pmask, st.S, st.kv_start, 0, slot,
-                                  st.ws, st.split_len, sc.attn, tiled=True)
-            elif sc.tiled:
-                # ln1 in the projection's prologue, K2 (RoPE, q scale, K/V into slot t) in its
-                # epilogue; the attention reads q and the cache
-                K.gemm_norm_qkv(sc.x, W.ln1[li], W.eps, W.qkv_t[li], B, H, None, st.pos,
-                                W.rope_tab, W.rope_geom, qs, sc.q, kc, vc, slot_dev=slot)
-                K.attn_decode(sc.q, kc, vc, B, H, st.pmask, st.S, st.kv_start, 0, slot, st.ws,
-                              st.split_len, sc.attn, row_holes=st.holes, row_order=st.order,
-                              tiled=True)
-            else:
-                gemm_f32(sc.xs, W.qkv[li], sc.qkv)
-                # RMSNorm scale + split + 3D RoPE + cache write fused into the attention launch
-                K.attn_decode_rope(sc.qkv, sc.rstd, st.pos, W.rope_tab, W.rope_geom, qs, kc, vc,
-                                   B, H, st.pmask, st.S, st.kv_start, 0, slot, st.ws,
-                                   st.split_len, sc.attn, row_holes=st.holes, row_order=st.order,
-                                   tiled=False)
+            gemm_f32(sc.xs, W.qkv[li], sc.qkv)
+            # RMSNorm scale + split + 3D RoPE + cache write fused into the attention launch
+            K.attn_decode_rope(sc.qkv, sc.rstd, st.pos, W.rope_tab, W.rope_geom, qs, kc, vc, B, H,
+                               st.pmask, st.S, st.kv_start, 0, slot, st.ws, st.split_len, sc.attn,
+                               row_holes=st.holes, row_order=st.order, tiled=False)
             self.eng._mlp(W, li, sc)
 
     def decode_layers(self, st: DecodeState, W: PackedWeights, want_logits: bool) -> None:
@@ -945,16 +933,15 @@ def _decode_step(model: TinyTransformer, token: torch.Tensor, position: torch.Te
         slots = cache.max_seq_len
         split = (choose_split_len_f32 if f32 else choose_split_len)(B * H, slots)
         nbytes = K.attn_decode_workspace_bytes(B, H, slots, split)
-        i32 = lambda: torch.zeros(B, dtype=torch.int32, device=dev)  # noqa: E731
+        # one step alone: nothing reads the grid state, prefill rows or outputs of a generation
+        none = torch.empty(0, dtype=torch.int32, device=dev)
         st = DecodeState(
             B=B, S=0 if pmask is None else pmask.shape[1], total=slots, ex=ex, pmask=pmask,
-            kv_start=None, last_row=i32(), holes=None, order=None, gx=i32(), gy=i32(),
-            gio=torch.zeros(B, dtype=torch.uint8, device=dev),
+            kv_start=None, last_row=none, holes=None, order=None, gx=none, gy=none, gio=none,
             pos=position.reshape(B, 3).to(device=dev, dtype=torch.int64).contiguous(), tok=tok,
-            counters=torch.tensor([t, 0], dtype=torch.int32, device=dev),
-            out_ids=torch.empty(B, 0, dtype=torch.int64, device=dev),
-            finish=i32(), logits=torch.empty(B, cfg.vocab_size, dtype=torch.float32, device=dev),
-            cache=cache,
+            counters=torch.full((2,), t, dtype=torch.int32, device=dev),   # [0]: the slot
+            out_ids=none, finish=none,
+            logits=torch.empty(B, cfg.vocab_size, dtype=torch.float32, device=dev), cache=cache,
             ws=(torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev)
                 if nbytes else None),
             sc=Scratch.alloc(B, cfg.d_model, cfg.d_ff, dev, f32=f32,

@@ -24,7 +24,8 @@ def _p(t: torch.Tensor | None) -> ctypes.c_void_p | None:
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the raw handle of torch.cuda.current_stream(), without building a Stream object
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _need(t: torch.Tensor | None, name: str, dtype: torch.dtype, numel: int | None = None,
@@ -870,6 +871,119 @@ def attn_prefill_lead(qkv: torch.Tensor, rstd: torch.Tensor, pos: torch.Tensor,
         _p(qkv), qkv.shape[1], _p(rstd), _p(pos), _p(rope_tab), mx, my, mz, px, py, pz, q_scale,
         batch, seq, n_heads, HEAD_DIM, _p(key_mask), _p(kv_start), _p(q_offset), _p(out),
         _layout(out_tiled), _stream()), "mdl_attn_prefill_lead")
+
+
+def id_range(ids: torch.Tensor, example_ids: torch.Tensor | None) -> list[int]:
+    """[ids min, max, example ids min, max] of int64 lists ([0, -1] for an empty or missing one)."""
+    _need(ids, "ids", I64)
+    _need(example_ids, "example_ids", I64, optional=True)
+    n, n_ex = ids.numel(), 0 if example_ids is None else example_ids.numel()
+    blocks = max(1, min(64, max(n, n_ex) // 4096))
+    out = torch.empty(4, blocks, dtype=I64, device=ids.device)
+    _lib.check(_lib.lib().mdl_id_range(_p(ids), n, _p(example_ids), n_ex, blocks, _p(out),
+                                       _stream()), "mdl_id_range")
+    lo, hi, ex_lo, ex_hi = out.tolist()
+    return [min(lo) if n else 0, max(hi) if n else -1, min(ex_lo) if n_ex else 0,
+            max(ex_hi) if n_ex else -1]
+
+
+def layer_table(W) -> bytes:
+    """The weights of every layer of a PackedWeights as mdl_layer records (no caches yet)."""
+    table = (_lib.Layer * len(W.ln1))()
+    for i, rec in enumerate(table):
+        for name in ("ln1", "ln2", "b_gate", "b_up", "b_down"):
+            setattr(rec, name, getattr(W, name)[i].data_ptr())
+        for name in ("qkv", "out", "gu", "down"):
+            setattr(rec, name, getattr(W, name + "_t")[i].data_ptr())
+            lo = getattr(W, name + "_lo")[i]
+            setattr(rec, name + "_lo", None if lo is None else lo.data_ptr())
+    return bytes(table)
+
+
+def _stack(W, cfg, sc, kv_layers, rows: int, batch: int, seq: int, pos: torch.Tensor,
+           q_scale: float, mask: torch.Tensor | None, row_holes: torch.Tensor | None,
+           kv_start: torch.Tensor | None) -> _lib.Stack:
+    """The mdl_stack of the layers of ``W`` over ``rows`` rows of ``sc``, its tensors checked."""
+    H, d = cfg.n_heads, cfg.n_heads * HEAD_DIM
+    dt = F32 if W.f32 else BF16
+    _need(sc.x, "x", F32, tile_rows(rows) * d)
+    _need(sc.q, "q", dt, rows * d)
+    _need(sc.qkv, "qkv", F32, rows * 3 * d)
+    _need(sc.rstd, "rstd", F32, rows)
+    _need(sc.attn, "attn", BF16, split_numel(rows, d, True))
+    _need(pos, "pos", I64, rows * 3)
+    _need(W.rope_tab, "rope_tab", F32)
+    _need(mask, "mask", U8, batch * seq, optional=True)
+    _need(row_holes, "row_holes", U8, batch, optional=True)
+    _need(kv_start, "kv_start", I32, batch, optional=True)
+    n = cfg.n_layers
+    layers = (_lib.Layer * n).from_buffer_copy(W.layers)
+    for li in range(n):
+        rec = layers[li]
+        kc, vc = kv_layers(li)
+        for name, c in (("k_cache", kc), ("v_cache", vc)):
+            _need(c, name, dt)
+            shape = c.shape
+            if len(shape) != 4 or shape[0] != batch or shape[1] != H or shape[3] != HEAD_DIM:
+                raise ValueError(f"{name} must be [batch, n_heads, slots, 64]")
+        if vc.shape[2] != kc.shape[2]:
+            raise ValueError("k_cache and v_cache must have the same slots")
+        rec.k_cache, rec.v_cache, rec.slots = kc.data_ptr(), vc.data_ptr(), kc.shape[2]
+    p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    mx, my, mz, px, py, pz = W.rope_geom
+    return _lib.Stack(
+        layers=layers, n_layers=n, f32=int(W.f32), eps=W.eps, d_ff=cfg.d_ff, n_heads=H, rows=rows,
+        batch=batch, seq=seq, x=p(sc.x), q=p(sc.q), qkv=p(sc.qkv), rstd=p(sc.rstd), attn=p(sc.attn),
+        h=p(sc.h), pos=p(pos), rope_tab=p(W.rope_tab), max_x=mx, max_y=my, max_z=mz, px=px, py=py,
+        pz=pz, q_scale=q_scale, mask=p(mask), row_holes=p(row_holes), kv_start=p(kv_start))
+
+
+def prompt_layers(W, cfg, sc, kv_layers, batch: int, seq: int, rows: int, pos: torch.Tensor,
+                  q_scale: float, lead_scale: float, key_mask: torch.Tensor | None,
+                  row_holes: torch.Tensor | None, kv_start: torch.Tensor | None, causal: bool,
+                  gate_up_parts: int, down_parts: int, token_row: torch.Tensor | None = None,
+                  token_slot: torch.Tensor | None = None,
+                  q_offset: torch.Tensor | None = None) -> None:
+    """Every layer of a prompt of ``rows`` tokens ([batch, seq], or a packed list with token_row /
+    token_slot / q_offset) on K6 and K4a / K4c (fp32 form: K4f), launched from one native call."""
+    if rows > sc.rows or (token_row is None and batch * seq != rows):
+        raise ValueError(f"{rows} prompt rows do not fit the scratch or the batch")
+    _need(sc.h, "h", BF16, tile_rows(rows) * down_parts * cfg.d_ff)
+    _need(token_row, "token_row", I32, rows, optional=q_offset is None)
+    _need(token_slot, "token_slot", I32, rows, optional=q_offset is None)
+    _need(q_offset, "q_offset", I32, batch, optional=True)
+    if q_offset is not None:
+        _need(kv_start, "kv_start", I32, batch)
+    s = _stack(W, cfg, sc, kv_layers, rows, batch, seq, pos, q_scale, key_mask, row_holes,
+               kv_start)
+    s.token_row = None if token_row is None else token_row.data_ptr()
+    s.token_slot = None if token_slot is None else token_slot.data_ptr()
+    s.q_offset = None if q_offset is None else q_offset.data_ptr()
+    s.causal, s.lead, s.lead_scale = int(causal), LEAD_QUERIES if causal else 0, lead_scale
+    s.gate_up_parts, s.down_parts = gate_up_parts, down_parts
+    _lib.check(_lib.lib().mdl_prompt_layers(ctypes.byref(s), _stream()), "mdl_prompt_layers")
+
+
+def decode_layers(W, cfg, sc, kv_layers, batch: int, prompt_len: int, pos: torch.Tensor,
+                  q_scale: float, prompt_mask: torch.Tensor | None,
+                  row_holes: torch.Tensor | None, kv_start: torch.Tensor | None,
+                  slot_dev: torch.Tensor, row_order: torch.Tensor | None,
+                  workspace: torch.Tensor | None, split_len: int) -> None:
+    """Every layer of a decode step of ``batch`` rows on K5 and K4b (fp32 form: K4f), the token's
+    K / V in slot slot_dev[0], launched from one native call."""
+    if sc.rows < batch:
+        raise ValueError(f"the scratch holds {sc.rows} rows, not {batch}")
+    _need(sc.h, "h", BF16, split_numel(batch, cfg.d_ff, True))
+    _need(slot_dev, "slot_dev", I32, 1)
+    _need(row_order, "row_order", I32, batch, optional=True)
+    _need(workspace, "workspace", F32, optional=True)
+    s = _stack(W, cfg, sc, kv_layers, batch, batch, prompt_len, pos, q_scale, prompt_mask,
+               row_holes, kv_start)
+    s.slot_dev, s.split_len = slot_dev.data_ptr(), split_len
+    s.row_order = None if row_order is None else row_order.data_ptr()
+    if workspace is not None:
+        s.ws, s.ws_bytes = workspace.data_ptr(), workspace.numel() * 4
+    _lib.check(_lib.lib().mdl_decode_layers(ctypes.byref(s), _stream()), "mdl_decode_layers")
 
 
 def attn_decode_workspace_bytes(batch: int, n_heads: int, slots: int, split_len: int) -> int:

@@ -1475,3 +1475,13 @@ def test_attn_prefill_block_sizes_agree(S, causal):
                          pm[idx].to(DEV), kv[idx].to(DEV), causal, out)
         outs.append(out.view(B, S, -1))
     assert torch.equal(outs[1], outs[0][torch.arange(outs[1].shape[0]) % rows])
+
+
+@pytest.mark.parametrize("n,n_ex", [(1, 0), (5, 3), (4097, 16), (70_001, 1), (500_000, 300_000)])
+def test_id_range(n, n_ex):
+    g = torch.Generator().manual_seed(n)
+    ids = torch.randint(-2 ** 40, 2 ** 40, (n,), generator=g).to(DEV)
+    ex = torch.randint(0, 2 ** 33, (n_ex,), generator=g).to(DEV) if n_ex else None
+    want = [int(ids.min()), int(ids.max())] + ([int(ex.min()), int(ex.max())] if n_ex else [0, -1])
+    assert K().id_range(ids, ex) == want
+    assert K().id_range(ids[:0], ids[:1]) == [0, -1, int(ids[0]), int(ids[0])]

@@ -27,7 +27,8 @@ epilogue; x (fp32) lives in the fp32 tile layout.  Per layer:
     x += h @ Wd^T + b_down                          <- split_residual
 
 At decode (M = batch rows) these are K5 launches (tall thin GEMMs: the weights are the traffic);
-for a prompt (M = batch * prompt length) they are K6 launches (persistent 256 x 256 tiles).
+for a prompt (M = batch * prompt length) they are K6 launches (persistent tiles, shaped by size).
+Either way one native call launches every layer (kernels.prompt_layers, decode_layers).
 The head kernel takes ln_f itself.  Shapes outside K6's limits (d_model > 2048, or a width that
 is not a multiple of 32) run the prompt's projections on hipBLASLt against [W | W] with K1,
 add_rmsnorm, K2 and K3 as separate passes.
@@ -53,8 +54,7 @@ Two forms, chosen by the model's parameter dtype as the reference chooses its ca
   ~2^-17), q / K / V and the cache are fp32 (K2 with fp32 outputs) and the attention is K4f
   (fp32 MFMA).  Per layer of a prompt or a decode step:
 
-    qkv, rstd = split(x * g1) @ (w + w_lo)^T                     <- K5 norm (E_STORE), fp32 out
-    q, K, V = K2(qkv) in fp32, K / V into the fp32 cache        <- qkv_rope_cache (fp32)
+    q, K, V = K2(split(x * g1) @ (w + w_lo)^T) in fp32           <- K5 norm (E_QKV), fp32 cache
     attn = K4f(q, cache)                                         <- attn_prefill_f32 / decode_f32
     then the three K5 launches of the bf16 decode form, each with its w_lo.
 
@@ -134,7 +134,8 @@ def pack_split_weight(w: torch.Tensor, device: torch.device) -> torch.Tensor:
 class PackedWeights:
     """Device copies of the weights in the layout the kernels and GEMMs consume.  ``f32`` marks
     the fp32 form: the tiled weights then come with their low parts (``*_lo``) and no [W | W]
-    copies are kept (the fp32 form runs every projection on K5)."""
+    copies are kept (the fp32 form runs its projections on K5 and K6).  ``layers`` is the native
+    table of these buffers (mdl_layer records); they live as long as it does."""
 
     def __init__(self, model: TinyTransformer, device: torch.device):
         cfg = model.config
@@ -501,14 +502,14 @@ class HipEngine:
             self._mlp(W, li, sc)
 
     def _mlp(self, W: PackedWeights, li: int, sc: Scratch) -> None:
-        """out_proj + residual, ln2, SwiGLU MLP + residual, next norm (shared by both phases)."""
+        """out_proj + residual, ln2, SwiGLU MLP + residual, next norm of the layers that no native
+        stack launches: on hipBLASLt, and fp32 prompts too wide for K6."""
         cfg = self.cfg
         d, F = cfg.d_model, cfg.d_ff
         if sc.tiled:
-            # decode: three K5 launches, the residual adds in the epilogues and ln2 in the
-            # gate / up prologue; the next layer's ln1 runs in its qkv launch (gemm_norm) and
-            # ln_f in the head kernel
-            # (the fp32 form adds each weight's low part)
+            # three K5 launches, the residual adds in the epilogues and ln2 in the gate / up
+            # prologue; the next layer's ln1 runs in its qkv launch (gemm_norm) and ln_f in the
+            # head kernel (the fp32 form adds each weight's low part)
             K.gemm_split_residual(sc.attn, W.out_t[li], sc.x, None, sc.rows, d, d,
                                   w_lo=W.out_lo[li])
             K.gemm_norm_swiglu(sc.x, W.ln2[li], W.eps, W.gu_t[li], W.b_gate[li], W.b_up[li],

@@ -31,14 +31,18 @@
 // kv_start[b] <= j < n_keys, (causal) j <= i, and (j >= mask_len or mask[b * mask_len + j] != 0);
 // a query with no visible key outputs 0 (what torch's CPU SDPA returns for an all -inf row).
 //
-// Prefill (attn_f32_prefill_kernel): a block of four waves takes 64 queries, and key tiles of 32
+// Prefill (attn_f32_prefill_kernel): a block of QW = 4 waves takes 64 queries, and key tiles of 32
 // go through a ring of two LDS stages (K and V, 8 KB each) filled by direct global -> LDS copies,
 // the next tile's while this one is worked on; one barrier per tile.  The 16-byte chunks of a
 // 256-byte row are XOR-swizzled with the row's low four bits, so both reads (16 rows of one chunk;
 // four whole rows) touch every bank once.  What bounds it is the fp32 matrix rate (154 TFLOP/s in
 // a large product on this card).  A wave that loaded its own 16 queries' keys from L2 waited for
 // every tile and moved four times the bytes: 16 rows of up to 811 tokens and 12 heads
-// 271 -> 178 us (92 us of MFMAs), 8 of up to 1,001 and 4 heads 126 -> 61.
+// 271 -> 178 us (92 us of MFMAs), 8 of up to 1,001 and 4 heads 126 -> 61.  A small launch is
+// bound by its longest block, whose SIMDs each work through all keys of 16 queries (64 fp32 MFMAs
+// of 32 cycles for 32 keys): there KG = 4 groups of QW waves take the tiles in turn, each with a
+// ring of its own, and merge their states in LDS at the end (8 ragged rows of up
+// to 1,001 tokens and 4 heads 61 -> 45 us).
 //
 // Decode (attn_f32_decode_kernel): a work item is one split_len-slot chunk of one (row, head), a
 // wave of its own without LDS or barriers; the chunks are what fills the GPU.  The query fills all
@@ -58,8 +62,7 @@ namespace mdl {
 namespace {
 
 constexpr int kQT = 16;          // queries of a wave
-constexpr int kWavesF = 4;       // waves per block
-constexpr int kQB = kQT * kWavesF;   // prefill: queries of a block
+constexpr int kWavesF = 4;       // decode: waves per block
 constexpr int kKT = 32;              // prefill: keys of a tile
 constexpr int kTileF = kKT * kHeadDim * 4;   // bytes of a K or V tile
 
@@ -127,7 +130,10 @@ __device__ __forceinline__ void store_out(const F32Args& p, int64_t qrow, int h,
 // Blocks: (row, head) pair i % 8 + 8 j on XCD i % 8, the latest (longest) query block of every pair
 // first, so that the short ones fill the end of the launch (pair by pair, the last pair's longest
 // blocks ran on alone: 213 -> 178 us).
-__global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const F32Args p) {
+template <int QW, int KG>
+__global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefill_kernel(
+    const F32Args p) {
+  constexpr int kQB = kQT * QW;   // queries of a block
   const int slot = blockIdx.x >> 3, pairs = gridDim.x / (8 * p.q_tiles);   // pairs of an XCD
   const int qt = p.q_tiles - 1 - slot / pairs;
   const int bh = (blockIdx.x & 7) + 8 * (slot % pairs);
@@ -141,12 +147,13 @@ __global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const
   const int64_t qbase = p.q_offset ? static_cast<int64_t>(p.q_offset[b]) - kstart
                                    : static_cast<int64_t>(b) * S;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wv % QW, kg = wv / QW;   // query group, key group
   const int wq0 = q0 + kQT * wave;
   const int qi = wq0 + c;
   const int64_t qrow = qbase + min(qi, S - 1);
 
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][kTileF];   // [stage][K, V]
+  __shared__ __attribute__((aligned(16))) uint8_t lds[KG][2][2][kTileF];   // [stage][K, V]
   const int64_t head = (static_cast<int64_t>(b) * p.heads + h) * p.slots * kHeadDim;
   const float* K = p.kc + head;
   const float* V = p.vc + head;
@@ -160,13 +167,13 @@ __global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const
   // Tile kt -> stage st: wave w copies key rows 16 j + 4 w .. + 3 of K and V (j = 0, 1), one
   // kilobyte each; lane l takes physical chunk l % 16 of its row, i.e. logical chunk
   // (l % 16) ^ (row % 16).  Rows past S copy the last key (their weights are 0).
-  const uint32_t lds0 = lds_addr(lds);
+  const uint32_t lds0 = lds_addr(lds) + kg * 4 * kTileF;
   auto issue = [&](int kt, int st) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int row = 16 * j + 4 * wave + (lane >> 4);
+    for (int j = 0; j < 8 / QW; ++j) {
+      const int row = 4 * (QW * j + wave) + (lane >> 4);
       const uint32_t off = min(row, S - 1 - kt) * (kHeadDim * 4) + 16 * (c ^ (row & 15));
-      const uint32_t dst = lds0 + 2 * st * kTileF + (16 * j + 4 * wave) * 256;
+      const uint32_t dst = lds0 + 2 * st * kTileF + 4 * (QW * j + wave) * 256;
       const int64_t tile = static_cast<int64_t>(kt) * kHeadDim;
       dma16_sbase(K + tile, off, __builtin_amdgcn_readfirstlane(dst));
       dma16_sbase(V + tile, off, __builtin_amdgcn_readfirstlane(dst + kTileF));
@@ -184,25 +191,29 @@ __global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const
 #pragma unroll
   for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  constexpr int kStep = kKT * KG;
   int ok_next = 0;
-  if (kstart < kend) {
-    ok_next = key_ok(kstart);
-    issue(kstart, 0);
+  if (kstart + kKT * kg < kend) {
+    ok_next = key_ok(kstart + kKT * kg);
+    issue(kstart + kKT * kg, 0);
   }
-  // every wave of the block runs the same tiles, so the barriers match
-  for (int kt = kstart, st = 0; kt < kend; kt += kKT, st ^= 1) {
+  // every wave of the block makes the same number of turns, so the barriers match; a group whose
+  // tile would start past the end neither copies nor computes
+  for (int t0 = kstart, st = 0; t0 < kend; t0 += kStep, st ^= 1) {
+    const int kt = t0 + kKT * kg;
     // tile kt has landed for every wave, and every wave is done with the other stage (the builtin
     // wait, so that the compiler counts its own loads, q and the mask bytes, as landed too)
     __builtin_amdgcn_s_waitcnt(kWaitAll);
     asm volatile("s_barrier" ::: "memory");
     const uint32_t valid = static_cast<uint32_t>(__ballot(ok_next != 0));
-    if (kt + kKT < kend) {
-      ok_next = key_ok(kt + kKT);
-      issue(kt + kKT, st ^ 1);
+    if (kt + kStep < kend) {
+      ok_next = key_ok(kt + kStep);
+      issue(kt + kStep, st ^ 1);
     }
+    if (kt >= kend) continue;
     if (p.causal && kt > wq0 + kQT - 1) continue;   // the whole tile is in this wave's future
-    const uint8_t* Kt = lds[st][0];
-    const uint8_t* Vt = lds[st][1];
+    const uint8_t* Kt = lds[kg][st][0];
+    const uint8_t* Vt = lds[kg][st][1];
     f32x4 s[2];
     float kv[2][16];
 #pragma unroll
@@ -264,6 +275,33 @@ __global__ __launch_bounds__(64 * kWavesF, 4) void attn_f32_prefill_kernel(const
         for (int db = 0; db < 4; ++db)
           o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[db], 0, 0, 0);
       }
+  }
+  if constexpr (KG > 1) {
+    // the other groups' states (m, l, o) through the ring's memory, one float per lane at a time
+    __syncthreads();   // every wave is done with its tiles
+    float* part = reinterpret_cast<float*>(lds);
+    if (kg > 0) {
+      float* w = part + ((kg - 1) * QW + wave) * 18 * kWave + lane;
+      w[0] = m;
+      w[kWave] = l;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) w[(2 + i) * kWave] = o[i >> 2][i & 3];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int j = 0; j < KG - 1; ++j) {
+      const float* w = part + (j * QW + wave) * 18 * kWave + lane;
+      const float mj = w[0];
+      const float m_new = fmaxf(m, mj);
+      const float base = m_new == -INFINITY ? 0.f : m_new;
+      const float a = __builtin_amdgcn_exp2f(m - base), aj = __builtin_amdgcn_exp2f(mj - base);
+      m = m_new;
+      l = fmaf(w[kWave], aj, l * a);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        o[i >> 2][i & 3] = fmaf(w[(2 + i) * kWave], aj, o[i >> 2][i & 3] * a);
+    }
   }
   if (qi >= S) return;
   l += __shfl_xor(l, 16, kWave);
@@ -414,6 +452,18 @@ __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __re
   }
 }
 
+constexpr int kBlocksSplit32 = 256, kBlocksSplit64 = 512;   // 64-query blocks
+
+template <int QW, int KG>
+int launch_prefill_f32(F32Args p, hipStream_t st) {
+  p.q_tiles = (p.seq + kQT * QW - 1) / (kQT * QW);
+  const int64_t blocks = (p.items + 7) / 8 * 8 * p.q_tiles;
+  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
+  hipLaunchKernelGGL((attn_f32_prefill_kernel<QW, KG>), dim3(static_cast<unsigned>(blocks)),
+                     dim3(64 * QW * KG), 0, st, p);
+  return launch_status();
+}
+
 int check_f32(const float* q, const float* k_cache, const float* v_cache, int batch,
               int n_heads, int head_dim, int cache_slots, const uint16_t* out, int out_layout) {
   if (!q || !k_cache || !v_cache || !out) return MDL_ERR_NULL;
@@ -449,15 +499,20 @@ extern "C" int mdl_attn_prefill_f32(const float* q, const float* k_cache, const 
   p.kv_start = kv_start; p.q_offset = q_offset;
   p.batch = batch; p.heads = n_heads; p.slots = cache_slots; p.seq = seq;
   p.causal = causal != 0;
-  p.q_tiles = (seq + kQB - 1) / kQB;
   p.items = static_cast<int64_t>(batch) * n_heads;
   p.out = out; p.out_layout = out_layout;
   if (p.items == 0) return MDL_OK;
-  const int64_t blocks = (p.items + 7) / 8 * 8 * p.q_tiles;
-  if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
-  hipLaunchKernelGGL(attn_f32_prefill_kernel, dim3(static_cast<unsigned>(blocks)),
-                     dim3(64 * kWavesF), 0, static_cast<hipStream_t>(stream), p);
-  return launch_status();
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  // How the longest block's chain of key tiles is cut while 64-query blocks number one or two per
+  // CU: four groups of waves take the tiles in turn, on 32 queries at up to one block per CU (so
+  // that twice as many CUs work) and on 64 at up to two.  Causal, us as one group of 64 / here:
+  // 144 blocks 34.6 / 20.0, 336 98 / 67, 512 60 / 47; at 940 265 / 265, at 2,496 110 / 140.  Without
+  // the causal limit every block is as long as the longest, and one group is as good or better
+  // (144: 37.5 / 39.2, 432: 47.6 / 49.7).
+  const int64_t blocks = p.items * ((seq + 63) / 64);
+  if (p.causal && blocks <= kBlocksSplit32) return launch_prefill_f32<2, 4>(p, st);
+  if (p.causal && blocks <= kBlocksSplit64) return launch_prefill_f32<4, 4>(p, st);
+  return launch_prefill_f32<4, 1>(p, st);
 }
 
 extern "C" int mdl_attn_decode_f32(const float* q, const float* k_cache, const float* v_cache,

@@ -381,3 +381,44 @@ def test_decode_merge_of_many_splits(n_split):
         outs.append(unsplit(out))
     a, b = outs
     assert bool(((a - b).abs() <= 2 ** -16 * b.abs() + 2 ** -20).all()), (a - b).abs().max()
+
+
+@pytest.mark.parametrize("S", [1, 31, 33, 130, 300])
+@pytest.mark.parametrize("blocks", [100, 400, 700])
+@pytest.mark.parametrize("packed", [False, True])
+def test_attn_prefill_f32_block_shapes(S, blocks, packed):
+    """K4f prefill in each block shape (launches of up to 256, 512 and more 64-query blocks; causal)
+    against fp64: a row from 0, one from S/3, one with a hole, one with no key (padded rows only),
+    the key tiles split over four groups of waves in the small launches."""
+    g = torch.Generator().manual_seed(S + blocks)
+    H, rows, slots = 4, 4, S + 2
+    B = max(rows, blocks // (H * -(-S // 64)))
+    pm = torch.ones(rows, S, dtype=torch.bool)
+    pm[1, :S // 3] = False
+    pm[2, S // 2:S // 2 + 9] = False
+    if not packed:
+        pm[3] = False
+    kv = torch.tensor([0, S // 3, 0, 0 if packed else S], dtype=torch.int32)
+    q = torch.randn(rows, H, S, 64, generator=g) * 0.3
+    kc, vc = (torch.randn(rows, H, slots, 64, generator=g) for _ in range(2))
+    ref = _attn_ref(q.transpose(1, 2), kc, vc, pm, True, S)
+    idx = torch.arange(B) % rows
+    qr = q.transpose(1, 2)[idx]                              # [B, S, H, 64]
+    off = None
+    if packed:
+        qr = torch.cat([qr[b, int(kv[idx[b]]):] for b in range(B)])
+        n = S - kv[idx]
+        off = (torch.cumsum(n, 0) - n).to(torch.int32).to(DEV)
+    qr = qr.reshape(-1, H * 64).contiguous().to(DEV)
+    out = torch.empty(qr.shape[0], 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+    K().attn_prefill_f32(qr, kc[idx].to(DEV), vc[idx].to(DEV), B, S, H,
+                         pm[idx].to(torch.uint8).to(DEV), kv[idx].to(DEV), off, qr.shape[0], True,
+                         out)
+    torch.cuda.synchronize()
+    got = unsplit(out).view(-1, H, 64)
+    for b in {0, 1, 2, 3, B - 1}:
+        i = int(idx[b])
+        lo = int(kv[i]) if packed else 0
+        r0 = int(off[b]) if packed else b * S
+        want = ref[i].transpose(0, 1)[lo:]                   # [S - lo, H, 64]
+        _attn_close(got[r0:r0 + S - lo], want, f"row {b}")

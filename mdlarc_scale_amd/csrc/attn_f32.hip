@@ -506,9 +506,9 @@ extern "C" int mdl_attn_prefill_f32(const float* q, const float* k_cache, const 
   // How the longest block's chain of key tiles is cut while 64-query blocks number one or two per
   // CU: four groups of waves take the tiles in turn, on 32 queries at up to one block per CU (so
   // that twice as many CUs work) and on 64 at up to two.  Causal, us as one group of 64 / here:
-  // 144 blocks 34.6 / 20.0, 336 98 / 67, 512 60 / 47; at 940 265 / 265, at 2,496 110 / 140.  Without
-  // the causal limit every block is as long as the longest, and one group is as good or better
-  // (144: 37.5 / 39.2, 432: 47.6 / 49.7).
+  // 144 blocks 34.6 / 20.0, 336 98 / 67, 512 60 / 47; at 940 265 / 265, at 2,496 110 / 140.
+  // Without the causal limit every block is as long as the longest, and one group is as good or
+  // better (144: 37.5 / 39.2, 432: 47.6 / 49.7).
   const int64_t blocks = p.items * ((seq + 63) / 64);
   if (p.causal && blocks <= kBlocksSplit32) return launch_prefill_f32<2, 4>(p, st);
   if (p.causal && blocks <= kBlocksSplit64) return launch_prefill_f32<4, 4>(p, st);

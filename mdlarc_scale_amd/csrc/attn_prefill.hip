@@ -388,19 +388,35 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(
 // Those queries see only keys among the same kLead tokens (causal), so one block holds them all
 // in LDS.  Later queries average over more than kLead keys and keep K4a's output.
 //
-// Block = one (b, h), four waves; wave w owns the 16 queries 16 w .. and lane (c, g) of it
-// (c = lane % 16, g = lane / 16) query 16 w + c and dims 16 g .. + 15: it rotates those dims of
-// its token's q (kept in registers) and k (to LDS) -- RoPE pairs 8 g .. + 7 -- and scales its v
-// dims (to LDS).  Then S^T = K Q^T and O^T = V^T P^T on fp32 MFMA (v_mfma_f32_16x16x4_f32) with the
-// operand layouts of K4f (attn_f32.hip): the probabilities never leave registers, and with all
-// scores of a query at hand its softmax takes one maximum and one sum.  A wave needs the key
-// blocks up to its own only.  One thread a query and a loop over its keys, a dot product with two
-// shuffles and an exponential for each, was a chain of 64 such steps: 12 (row,
-// head) pairs 29 -> 10 us, 3,072 of them 121 -> 66 us.
+// Block = one (b, h), eight waves; a wave owns 8 queries, 8 lanes each: lane 8 i + e holds dims
+// 8 e .. 8 e + 7 of query i of its wave.  It rotates those dims of its token's q (kept in registers)
+// and k (to LDS) -- RoPE pairs 4 e .. + 3 -- and scales its v dims (to LDS).  Then, over the wave's
+// visible keys, three passes that each have work for every lane at every step:
+//   the scores: sixteen chains of four products, added in pairs, two in a lane and the rest over
+//     the query's lanes by DPP;
+//   the running maximum (a scan over lanes, one key each), a key's weight against it, and what a
+//     new maximum multiplies the sums by;
+//   the sums of the weights and of P V, key by key.
+// That is the recurrence of a loop over the keys, with its rounding: the scores, maxima and weights
+// depend on no sum.  A key that a query does not see adds zero times zero, so a value that is
+// not finite stays with the queries that see it, which a matrix product over whole blocks of keys
+// (9.1 / 50 us below) does not give.  Waves 0..3 take queries 8 w .. and waves 4..7 the others from
+// the end, so that the two waves of a SIMD have nine blocks of 8 keys between them.
+// What bounds it: the instructions of a block's four SIMDs (4.5 us are loads, rotation and store).
+// Four lanes a query, a loop with an exponential and two shuffles through the LDS unit for each
+// key, took 28 us at 12 (row, head) pairs and 102 at 3,072; this 11.3 and 73.
 constexpr int kLead = 64;
 constexpr int kLeadLd = kHeadDim + 4;   // LDS row stride (floats): 16-byte aligned rows
+constexpr int kLeadLanes = 8;           // lanes of a query, and keys of a step
+constexpr int kLeadBlocks = 36;         // 8 queries x 8 keys at or below the diagonal
 
-__global__ __launch_bounds__(256) void attn_lead_kernel(
+// v of another lane of the eight: CTRL a DPP control within 8 lanes
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+__global__ __launch_bounds__(512, 6) void attn_lead_kernel(
     const float* __restrict__ qkv, int64_t ld, const float* __restrict__ rstd,
     const int64_t* __restrict__ pos, const float* __restrict__ tab, RopeArgs ra, float q_scale,
     int S, int H, const uint8_t* __restrict__ kmask, const int32_t* __restrict__ kv_start,
@@ -416,36 +432,38 @@ __global__ __launch_bounds__(256) void attn_lead_kernel(
   const int64_t d = static_cast<int64_t>(H) * kHeadDim;
   __shared__ __attribute__((aligned(16))) float ks[kLead * kLeadLd];
   __shared__ __attribute__((aligned(16))) float vs[kLead * kLeadLd];
+  __shared__ __attribute__((aligned(16))) float ps[kLeadBlocks * 64], as[kLeadBlocks * 64];
   __shared__ uint8_t ok[kLead];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = lane & 15, g = lane >> 4;
-  const int r = 16 * wave + c;
-  float q[16], kr[16], va[16];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wv < 4 ? wv : 11 - wv;
+  const int i = lane >> 3, e = lane & 7;
+  const int r = 8 * wave + i;
+  float q[8], kr[8], va[8];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) q[e] = kr[e] = va[e] = 0.f;   // rows past n: finite, and masked
+  for (int c = 0; c < 8; ++c) q[c] = kr[c] = va[c] = 0.f;   // rows past n are masked
   uint8_t valid = 0;
   if (r < n) {
     const int64_t row = row0 + r;
     const float rs = rstd[row];
-    const float* src = qkv + row * ld + h * kHeadDim + 16 * g;
-    float qa[16], ka[16];
+    const float* src = qkv + row * ld + h * kHeadDim + 8 * e;
+    float qa[8], ka[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<float4*>(qa + 4 * i) = *reinterpret_cast<const float4*>(src + 4 * i);
-      *reinterpret_cast<float4*>(ka + 4 * i) = *reinterpret_cast<const float4*>(src + d + 4 * i);
-      *reinterpret_cast<float4*>(va + 4 * i) =
-          *reinterpret_cast<const float4*>(src + 2 * d + 4 * i);
+    for (int c = 0; c < 8; c += 4) {
+      *reinterpret_cast<float4*>(qa + c) = *reinterpret_cast<const float4*>(src + c);
+      *reinterpret_cast<float4*>(ka + c) = *reinterpret_cast<const float4*>(src + d + c);
+      *reinterpret_cast<float4*>(va + c) = *reinterpret_cast<const float4*>(src + 2 * d + c);
     }
     valid = !kmask || kmask[static_cast<int64_t>(b) * S + kstart + r] != 0;
-    // the token's three positions once, then the sixteen table entries as independent loads
+    // the token's three positions once, then the eight table entries as independent loads
     const int64_t* p3 = pos + row * 3;
     const int64_t P0 = p3[0], P1 = p3[1], P2 = p3[2];
-    float csv[8], snv[8];
+    float csv[4], snv[4];
 #pragma unroll
-    for (int pp = 0; pp < 8; ++pp)
-      rope_cos_sin3(g * 8 + pp, P0, P1, P2, tab, ra, csv[pp], snv[pp]);
+    for (int pp = 0; pp < 4; ++pp)
+      rope_cos_sin3(e * 4 + pp, P0, P1, P2, tab, ra, csv[pp], snv[pp]);
 #pragma unroll
-    for (int pp = 0; pp < 8; ++pp) {
+    for (int pp = 0; pp < 4; ++pp) {
       const float cs = csv[pp], sn = snv[pp];
       const float q0 = qa[2 * pp] * rs, q1 = qa[2 * pp + 1] * rs;
       const float k0 = ka[2 * pp] * rs, k1 = ka[2 * pp + 1] * rs;
@@ -457,84 +475,123 @@ __global__ __launch_bounds__(256) void attn_lead_kernel(
       va[2 * pp + 1] *= rs;
     }
   }
+  // a row's 16-byte chunks: the even ones, then the odd ones, so that the lanes of a query read
+  // (and write) 128 contiguous bytes at a time
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    *reinterpret_cast<float4*>(ks + r * kLeadLd + 16 * g + 4 * i) =
-        *reinterpret_cast<const float4*>(kr + 4 * i);
-    *reinterpret_cast<float4*>(vs + r * kLeadLd + 16 * g + 4 * i) =
-        *reinterpret_cast<const float4*>(va + 4 * i);
+  for (int c = 0; c < 2; ++c) {
+    *reinterpret_cast<float4*>(ks + r * kLeadLd + 32 * c + 4 * e) =
+        *reinterpret_cast<const float4*>(kr + 4 * c);
+    *reinterpret_cast<float4*>(vs + r * kLeadLd + 32 * c + 4 * e) =
+        *reinterpret_cast<const float4*>(va + 4 * c);
   }
-  if (g == 0) ok[r] = valid;
+  if (e == 0) ok[r] = valid;
   __syncthreads();
-  if (16 * wave >= n) return;   // whole wave; no barrier follows
+  if (8 * wave >= n) return;   // whole wave; no barrier follows
+  const uint64_t keys = __ballot(ok[lane] != 0);   // bit j: key j is valid
 
-  constexpr int kBlocks = kLead / 16;
-  f32x4_t sc[kBlocks];
-  float mx = -INFINITY;
+  // The scores, 8 keys at a time; lane e keeps that of key j0 + e, -inf where it is not seen.  Each
+  // lane reads back what it wrote.
+  float* pw = ps + 32 * wave * (wave + 1);   // the wave's 64-float blocks, one per 8 keys
+  float* aw = as + 32 * wave * (wave + 1);
+#pragma unroll 2
+  for (int t = 0; t <= wave; ++t) {
+    float s[kLeadLanes];
 #pragma unroll
-  for (int nb = 0; nb < kBlocks; ++nb) {
-    sc[nb] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    if (nb > wave) continue;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 k4 =
-          *reinterpret_cast<const float4*>(ks + (16 * nb + c) * kLeadLd + 16 * g + 4 * i);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, q[4 * i], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, q[4 * i + 1], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, q[4 * i + 2], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, q[4 * i + 3], acc, 0, 0, 0);
+    for (int u = 0; u < kLeadLanes; ++u) {
+      const int at = (8 * t + u) * kLeadLd + 4 * e;
+      const float4 ka = *reinterpret_cast<const float4*>(ks + at);
+      const float4 kb = *reinterpret_cast<const float4*>(ks + at + 32);
+      float a0 = 0.f, a1 = 0.f;
+      a0 = fmaf(q[0], ka.x, a0); a1 = fmaf(q[4], kb.x, a1);
+      a0 = fmaf(q[1], ka.y, a0); a1 = fmaf(q[5], kb.y, a1);
+      a0 = fmaf(q[2], ka.z, a0); a1 = fmaf(q[6], kb.z, a1);
+      a0 = fmaf(q[3], ka.w, a0); a1 = fmaf(q[7], kb.w, a1);
+      float v = a0 + a1;
+      v += dpp<0xb1>(v);          // lane e ^ 1 (quad_perm 1, 0, 3, 2)
+      v += dpp<0x4e>(v);          // lane e ^ 2 (quad_perm 2, 3, 0, 1)
+      s[u] = v + dpp<0x141>(v);   // the other four, which hold the same sum (row_half_mirror)
     }
+    float se = s[0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = 16 * nb + 4 * g + i;
-      if (j <= r && ok[j]) sc[nb][i] = acc[i];
-      mx = fmaxf(mx, sc[nb][i]);
+    for (int u = 1; u < kLeadLanes; ++u) se = e == u ? s[u] : se;
+    const bool see = 8 * t + e <= r && ((keys >> (8 * t + e)) & 1u);
+    pw[64 * t + lane] = see ? se : -INFINITY;
+  }
+
+  // Each key's weight against the maximum so far, and what a new maximum multiplies the sums by:
+  // the maximum within the eight lanes' keys by a scan, then over the blocks of keys
+  {
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < kLead / 8; ++t) {
+      if (t > wave) break;
+      const float se = pw[64 * t + lane];
+      float me = se, v = dpp<0x111>(me);   // row_shr 1, 2, 4
+      me = fmaxf(me, e >= 1 ? v : -INFINITY);
+      v = dpp<0x112>(me);
+      me = fmaxf(me, e >= 2 ? v : -INFINITY);
+      v = dpp<0x114>(me);
+      me = fmaxf(me, e >= 4 ? v : -INFINITY);
+      v = dpp<0x111>(me);
+      const float before = fmaxf(e >= 1 ? v : -INFINITY, top);
+      const float last =
+          __uint_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane | 7), __float_as_uint(me)));
+      me = fmaxf(me, top);
+      top = fmaxf(last, top);
+      aw[64 * t + lane] = se > before ? expf(before - se) : 1.f;   // 0 at the first visible key
+      pw[64 * t + lane] = expf(se - me);
     }
   }
-  mx = max_over_groups(mx);
-  const float base = mx == -INFINITY ? 0.f : mx;   // no visible key: weights 0, as in K4a
-  float l = 0.f;
-  f32x4_t o[4];
+
+  // The sums, key by key; a lane reads the weights that the other lanes of its query wrote, in this
+  // wave.  `all`: every query of the wave sees the eight keys.
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  float l = 0.f, o[8];
 #pragma unroll
-  for (int db = 0; db < 4; ++db) o[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < 8; ++c) o[c] = 0.f;
+  auto sums = [&](int t, auto all, uint32_t valid8) {
+#pragma clang fp contract(off)
 #pragma unroll
-  for (int nb = 0; nb < kBlocks; ++nb) {
-    if (nb > wave) continue;
+    for (int u0 = 0; u0 < kLeadLanes; u0 += 4) {
+      const float4 p4 = *reinterpret_cast<const float4*>(pw + 64 * t + 8 * i + u0);
+      const float4 a4 = *reinterpret_cast<const float4*>(aw + 64 * t + 8 * i + u0);
+      const float pv[4] = {p4.x, p4.y, p4.z, p4.w}, av[4] = {a4.x, a4.y, a4.z, a4.w};
+      float v[4][8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float pj = expf(sc[nb][i] - base);
-      l += pj;
-      const float4 v4 =
-          *reinterpret_cast<const float4*>(vs + (16 * nb + 4 * g + i) * kLeadLd + 4 * c);
-      o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, pj, o[0], 0, 0, 0);
-      o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, pj, o[1], 0, 0, 0);
-      o[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, pj, o[2], 0, 0, 0);
-      o[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, pj, o[3], 0, 0, 0);
+      for (int u = 0; u < 4; ++u) {
+        const int at = (8 * t + u0 + u) * kLeadLd + 4 * e;
+        *reinterpret_cast<float4*>(v[u]) = *reinterpret_cast<const float4*>(vs + at);
+        *reinterpret_cast<float4*>(v[u] + 4) = *reinterpret_cast<const float4*>(vs + at + 32);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool see = all || (8 * t + u0 + u <= r && ((valid8 >> (u0 + u)) & 1u));
+        l = l * av[u] + (see ? pv[u] : 0.f);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          o[c] = fmaf(see ? pv[u] : 0.f, see ? v[u][c] : 0.f, o[c] * av[u]);
+      }
     }
+  };
+  for (int t = 0; t <= wave; ++t) {
+    const uint32_t valid8 = static_cast<uint32_t>(keys >> (8 * t)) & 0xffu;
+    if (valid8 == 0xffu && t < wave)
+      sums(t, std::true_type{}, 0xffu);
+    else
+      sums(t, std::false_type{}, valid8);
   }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
   if (r >= n) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  // element i of dim block db is dim 16 g + 4 i + db of query r
-  float res[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int db = 0; db < 4; ++db) res[4 * i + db] = o[db][i] * inv;
+  const float inv = l > 0.f ? 1.f / l : 0.f;   // no visible key: 0, as in K4a
   const int64_t orow = row0 + r;
-  const int col0 = h * kHeadDim + 16 * g, d2 = static_cast<int>(2 * d);
+  const int col0 = h * kHeadDim + 8 * e, d2 = static_cast<int>(2 * d);
 #pragma unroll
-  for (int e = 0; e < 16; e += 4) {
-    uint2 hi, lo;
-    split4(res + e, hi, lo);
-    uint16_t* oh = out_tiled ? out + tile_off(orow, col0 + e, d2) : out + orow * d2 + col0 + e;
-    uint16_t* ol = out_tiled ? out + tile_off(orow, static_cast<int>(d) + col0 + e, d2) : oh + d;
-    *reinterpret_cast<uint32_t*>(oh) = hi.x;   // the entry asks for 4-byte alignment only
-    *reinterpret_cast<uint32_t*>(oh + 2) = hi.y;
-    *reinterpret_cast<uint32_t*>(ol) = lo.x;
-    *reinterpret_cast<uint32_t*>(ol + 2) = lo.y;
+  for (int c = 0; c < 8; c += 2) {
+    uint32_t hi, lo;
+    split_bf2(o[c] * inv, o[c + 1] * inv, hi, lo);
+    uint16_t* oh = out_tiled ? out + tile_off(orow, col0 + c, d2) : out + orow * d2 + col0 + c;
+    uint16_t* ol = out_tiled ? out + tile_off(orow, static_cast<int>(d) + col0 + c, d2) : oh + d;
+    *reinterpret_cast<uint32_t*>(oh) = hi;   // the entry asks for 4-byte alignment only
+    *reinterpret_cast<uint32_t*>(ol) = lo;
   }
 }
 
@@ -624,7 +681,7 @@ extern "C" int mdl_attn_prefill_lead(const float* qkv, int64_t qkv_ld, const flo
   if (blocks == 0 || seq == 0) return MDL_OK;
   if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
   const RopeArgs ra{max_x, max_y, max_z, px, py, pz};
-  attn_lead_kernel<<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
+  attn_lead_kernel<<<static_cast<unsigned>(blocks), 512, 0, static_cast<hipStream_t>(stream)>>>(
       qkv, qkv_ld, rstd, pos, rope_tab, ra, q_scale, seq, n_heads, key_mask, kv_start, q_offset,
       out, out_layout == MDL_LAYOUT_TILES ? 1 : 0);
   return launch_status();

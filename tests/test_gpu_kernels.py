@@ -682,6 +682,96 @@ def test_attn_prefill_lead_exact(packed):
     assert torch.equal(K().untile_matrix(out_t, rows, 2 * d), out)
 
 
+def _fma(a, b, c):
+    """fp32 a * b + c in one rounding (the product is exact in fp64)."""
+    return (a.double() * b.double() + c.double()).float()
+
+
+def _lead_inputs(B, H, S, seed):
+    """Projection outputs at position 0 of every axis, where the rotation is the identity."""
+    from mdlarc_scale_amd.transformer import RotaryEmbedding3D
+
+    g = torch.Generator().manual_seed(seed)
+    qkv = (3 * torch.randn(B * S, 3 * 64 * H, generator=g)).to(DEV)
+    rstd = (0.5 + torch.rand(B * S, generator=g)).to(DEV)
+    pos = torch.zeros(B * S, 3, dtype=torch.int64, device=DEV)
+    rope = RotaryEmbedding3D(64, 30, 30, 8)
+    return (qkv, rstd, pos, rope.device_table(DEV),
+            (rope.max_x, rope.max_y, rope.max_z, rope.px, rope.py, rope.pz))
+
+
+def _lead(inputs, B, H, S, mask, kv):
+    out = torch.full((B * S, 2 * 64 * H), 5.0, device=DEV, dtype=torch.bfloat16)
+    K().attn_prefill_lead(*inputs, 0.125, B, S, H, mask, kv, None, B * S, out)
+    return out
+
+
+@pytest.mark.parametrize("S", [1, 7, 8, 9, 33, 63, 64, 90])
+def test_attn_prefill_lead_takes_the_keys_in_order(S):
+    """K4c, bit for bit the fp32 recurrence written out in torch: sixteen chains of four products a
+    score, added in pairs; then key by key the maximum, the weight, the sum and the output."""
+    B, H = 4, 3
+    n = min(S, 64)
+    inputs = _lead_inputs(B, H, S, S)
+    mask = torch.ones(B, S, dtype=torch.bool, device=DEV)
+    kv = torch.tensor([0, 0, S // 3, 0], dtype=torch.int32, device=DEV)
+    mask[1, 1:4] = False
+    mask[2, :S // 3] = False
+    mask[3, ::2] = False                       # the first query of row 3 sees no key
+    out = _lead(inputs, B, H, S, mask.to(torch.uint8), kv)
+    qkv = inputs[0].view(B, S, 3, H, 64) * inputs[1].view(B, S, 1, 1, 1)
+    for b in range(B):
+        k0 = int(kv[b])
+        q, k, v = (t.transpose(0, 1) for t in qkv[b, k0:k0 + n].unbind(1))   # [H, m, 64]
+        q, m = q * 0.125, q.shape[1]
+        seen = mask[b, k0:k0 + n]
+        qc, kc = q.reshape(H, m, 1, 16, 4), k.reshape(H, 1, m, 16, 4)
+        a = qc[..., 0] * kc[..., 0]
+        for i in (1, 2, 3):
+            a = _fma(qc[..., i], kc[..., i], a)
+        for _ in range(4):
+            a = a[..., 0::2] + a[..., 1::2]
+        s = a[..., 0]                                                        # [H, query, key]
+        top = torch.full((H, m), float("-inf"), device=DEV)
+        L, o = torch.zeros(H, m, device=DEV), torch.zeros(H, m, 64, device=DEV)
+        r = torch.arange(m, device=DEV)
+        for j in range(m):
+            see = (j <= r) & seen[j]
+            new = torch.where(see & (s[:, :, j] > top), s[:, :, j], top)
+            alpha = torch.where(new > top, torch.exp(top - new), 1.0)
+            top, L, o = new, L * alpha, o * alpha[..., None]
+            p = torch.exp(s[:, :, j] - top)
+            L = torch.where(see, L + p, L)
+            o = torch.where(see[:, None], _fma(p[..., None], v[:, j, None], o), o)
+        want = (o * torch.where(L > 0, 1.0 / L, 0.0)[..., None]).transpose(0, 1).reshape(m, H * 64)
+        hi = want.to(torch.bfloat16)
+        rows = out[b * S + k0:b * S + k0 + m]
+        assert torch.equal(rows[:, :H * 64], hi), b
+        assert torch.equal(rows[:, H * 64:], (want - hi.float()).to(torch.bfloat16)), b
+        assert bool((out[b * S + k0 + m:(b + 1) * S] == 5).all())
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attn_prefill_lead_leaves_unseen_values_out(bad):
+    """A value that is not finite, of a masked key or of a later one, changes no lead query that
+    does not see it."""
+    B, H, S = 3, 2, 70
+    inputs = _lead_inputs(B, H, S, 3)
+    kv = torch.zeros(B, dtype=torch.int32, device=DEV)
+    mask = torch.ones(B, S, dtype=torch.uint8, device=DEV)
+    mask[1, 20] = 0
+    want = _lead(inputs, B, H, S, mask, kv).view(B, S, -1)
+    v = inputs[0].view(B, S, 3, H, 64)[:, :, 2]
+    v[0, 29, 1, 7] = bad                       # seen from query 29 on
+    v[1, 20] = bad                             # masked
+    v[2, 63] = bad                             # the last lead key
+    got = _lead(inputs, B, H, S, mask, kv).view(B, S, -1)
+    assert torch.equal(got[0, :29], want[0, :29]) and torch.equal(got[1], want[1])
+    assert torch.equal(got[2, :63], want[2, :63])
+    assert not bool(got[0, 29:64, 64 + 7].isfinite().any())
+    assert not bool(got[2, 63, :128].isfinite().any())
+
+
 # ---------------------------------------------------------------------------- K4b decode
 
 @pytest.mark.parametrize("split_len,slots,t", [(128, 700, 611), (256, 700, 611),

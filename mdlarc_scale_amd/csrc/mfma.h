@@ -68,11 +68,17 @@ __device__ __forceinline__ float max_over_groups(float v) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+// `v` of lane `i` (the same for the whole wave) in every lane, without a trip through the LDS unit.
+__device__ __forceinline__ float from_lane(float v, int i) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), i));
+}
+
 // Channel `lane` of the merge of one (row, head)'s split states (m, l, o[64] unnormalised, PART
 // floats apart; base 2): o / l at their largest m, 0 if no split saw a key.  A lane reads one
 // split's m and l, so a wave has all of them (64 at a time) after one round trip, and the o
-// values, whose addresses depend on nothing read, come eight at a time
-// (a chain of one dependent load per split took 6 us at 7 splits of 12 pairs, this 2.9).
+// values, whose addresses depend on nothing read, come eight at a time (a chain of one dependent
+// load per split took 6 us at 7 splits of 12 pairs, this 2.9).  Both sums run over the
+// splits in order, whatever lane holds them.
 template <int PART>
 __device__ __forceinline__ float merge_parts(const float* __restrict__ part, int n_split,
                                              int lane) {
@@ -82,9 +88,8 @@ __device__ __forceinline__ float merge_parts(const float* __restrict__ part, int
   float L = 0.f, O = 0.f;
   for (int s0 = 0; s0 < n_split; s0 += kWave) {
     const int s = min(s0 + lane, n_split - 1);
-    const float ms = part[s * PART];
-    const float sc = s0 + lane < n_split && ms != -INFINITY ? exp2f(ms - M) : 0.f;
-    L = fmaf(part[s * PART + 1], sc, L);
+    const float ms = part[s * PART], ls = part[s * PART + 1];
+    const float sc = ms == -INFINITY ? 0.f : exp2f(ms - M);
     const int n = min(kWave, n_split - s0);
     for (int q0 = 0; q0 < n; q0 += 8) {
       float o[8];
@@ -92,11 +97,14 @@ __device__ __forceinline__ float merge_parts(const float* __restrict__ part, int
       for (int q = 0; q < 8; ++q)
         o[q] = part[(s0 + min(q0 + q, n - 1)) * PART + 2 + lane];
 #pragma unroll
-      for (int q = 0; q < 8; ++q)   // lanes past the last split hold a weight of 0
-        O = fmaf(o[q], __shfl(sc, min(q0 + q, kWave - 1), kWave), O);
+      for (int q = 0; q < 8; ++q) {
+        if (q0 + q >= n) break;   // whole wave
+        const float w = from_lane(sc, q0 + q);
+        L = fmaf(from_lane(ls, q0 + q), w, L);
+        O = fmaf(o[q], w, O);
+      }
     }
   }
-  L = wave_sum(L);
   return L > 0.f ? O / L : 0.f;
 }
 

@@ -872,6 +872,41 @@ def test_attn_decode_rope_equals_k2_then_decode(split_len, slots, t):
     assert torch.allclose(unsplit(out2), unsplit(out1), rtol=2e-3, atol=2e-4)
 
 
+@pytest.mark.parametrize("n_split", [2, 7, 8, 9, 64, 65, 70])
+@pytest.mark.parametrize("f32", [False, True])
+def test_decode_merge_adds_the_splits_in_order(n_split, f32):
+    """The merge of a launch's split states, bit for bit the two sums taken split by split (the
+    states are read from the workspace that the launch left), and an infinite value of the last
+    split reaches its own channel as it is: nothing is multiplied by a weight of zero."""
+    g = torch.Generator().manual_seed(n_split)
+    B, H, step = 5, 3, 16 if f32 else 128
+    slots = step * n_split
+    t = slots - 4
+    dt = torch.float32 if f32 else torch.bfloat16
+    q = (torch.randn(B, H, 64, generator=g) * 0.4).to(dt).to(DEV)
+    kc, vc = (torch.randn(B, H, slots, 64, generator=g).to(dt).to(DEV) for _ in range(2))
+    vc[1, 1, t - 1, 5] = float("inf")
+    kv = torch.tensor([0, 0, 3, step + 1, t], dtype=torch.int32, device=DEV)
+    ws = torch.full((B * H * n_split, 66), float("nan"), device=DEV)
+    out = torch.empty(B, 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+    (K().attn_decode_f32 if f32 else K().attn_decode)(q, kc, vc, B, H, None, 0, kv, t, None, ws,
+                                                      step, out)
+    torch.cuda.synchronize()
+    p = ws.view(B * H, n_split, 66)
+    top = p[:, :, 0].max(1).values
+    L, acc = torch.zeros(B * H, device=DEV), torch.zeros(B * H, 64, device=DEV)
+    for s in range(n_split):
+        w = torch.where(p[:, s, 0] == float("-inf"), 0.0, torch.exp2(p[:, s, 0] - top))
+        L = _fma(p[:, s, 1], w, L)
+        acc = _fma(p[:, s, 2:], w[:, None], acc)
+    want = (acc / L[:, None]).view(B, H * 64)
+    hi = want.to(torch.bfloat16)
+    lo = (want - hi.float()).to(torch.bfloat16)
+    assert torch.equal(out[:, :H * 64], hi)
+    assert torch.equal(out[:, H * 64:].nan_to_num(0.0), lo.nan_to_num(0.0))
+    assert int(hi.isinf().sum()) == 1
+
+
 # ---------------------------------------------------------------------------- head + state
 
 @pytest.mark.parametrize("d", [128, 768, 1280])

@@ -87,20 +87,22 @@ __device__ __forceinline__ float merge_parts(const float* __restrict__ part, int
   M = wave_max(M);
   float L = 0.f, O = 0.f;
   for (int s0 = 0; s0 < n_split; s0 += kWave) {
-    const int s = min(s0 + lane, n_split - 1);
-    const float ms = part[s * PART], ls = part[s * PART + 1];
-    const float sc = ms == -INFINITY ? 0.f : exp2f(ms - M);
     const int n = min(kWave, n_split - s0);
+    const int s = s0 + min(lane, n - 1);
+    const float ms = part[s * PART], ls = part[s * PART + 1];
+    const float sc = lane >= n || ms == -INFINITY ? 0.f : exp2f(ms - M);
+    const float ln = lane < n ? ls : 0.f;
     for (int q0 = 0; q0 < n; q0 += 8) {
       float o[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        o[q] = part[(s0 + min(q0 + q, n - 1)) * PART + 2 + lane];
+      for (int q = 0; q < 8; ++q) {   // past the last split: its values once more, as zeros
+        const float v = part[(s0 + min(q0 + q, n - 1)) * PART + 2 + lane];
+        o[q] = q0 + q < n ? v : 0.f;
+      }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        if (q0 + q >= n) break;   // whole wave
         const float w = from_lane(sc, q0 + q);
-        L = fmaf(from_lane(ls, q0 + q), w, L);
+        L = fmaf(from_lane(ln, q0 + q), w, L);
         O = fmaf(o[q], w, O);
       }
     }

@@ -403,8 +403,9 @@ int mdl_prefill_gemm_split_residual(const uint16_t* a, int64_t lda, int a_layout
  * The same for an fp32 weight, passed as its high and low bf16 parts w = bf16(W), w_lo =
  * bf16(W - w), both tiled (as mdl_gemm_norm takes them): each k-step adds a_hi . w_lo after the hi
  * and lo products, so the weight is seen to ~2^-17 like the activation.  a is the tiled split
- * activation, h_out the tiled split [m, 2 d_ff]; the other arguments and limits as above.  Up to
- * 640 rows run on K5 (mdl_gemm_norm and its kind), with that kernel's order of the sums.
+ * activation, h_out the tiled split [m, 2 d_ff]; the other arguments and limits as above.  The sums
+ * are in the order of K5 (mdl_gemm_norm and its kind), on which few rows run: the same bits for a
+ * row however many run beside it.
  */
 int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, float eps, const uint16_t* w,
                                const uint16_t* w_lo, float* out, int64_t ldo, float* rstd_out,

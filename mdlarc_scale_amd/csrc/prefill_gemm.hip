@@ -56,7 +56,8 @@
 // i runs on XCD i mod 8) takes a contiguous run of tiles, row tile major: the N tiles of one row
 // tile share its activation rows in one L2.  Summation order is fixed (k-steps in order, hi
 // before lo), so results are reproducible, and it is the same in every shape: a row's results do
-// not depend on how many rows run beside it.
+// not depend on how many rows run beside it.  The forms for fp32 weights take K5's order (eight
+// runs of k-steps, each summed from zero, added in order), because a few rows run on K5.
 #include <algorithm>
 
 #include <type_traits>
@@ -255,13 +256,62 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
 
   f32x4_t acc[FN][FM];
   float ss[FM];   // A_NORM: this lane's part of sum(x^2) of row 16 (FM wm + j) + c
-  auto reset = [&]() {
+  // WL: the sums of the runs of k-steps before this one (acc and ss are of the present run)
+  f32x4_t tot[WL ? FN : 1][WL ? FM : 1];
+  float ss_tot[WL ? FM : 1];
+  auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
       for (int j = 0; j < FM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < FM; ++j) ss[j] = 0.f;
+  };
+  auto over_groups = [&](float v) {   // a row's four lane groups, in a fixed order
+    v += __shfl_xor(v, 16, kWave);
+    return v + __shfl_xor(v, 32, kWave);
+  };
+  // WL: run w of a tile's k-steps is [nk w / 8, nk (w + 1) / 8), what wave w of a K5 block takes;
+  // each is summed from zero and the sums are added in order, as that block's reduction does.
+  // `run_end` is where the present one ends (the tile's first k-step moves past empty ones).
+  int run = 0, run_end = 0;
+  auto next_run = [&](int s) {   // s: the next k-step
+    do {
+      ++run;
+      run_end = (nk * run) >> 3;
+    } while (run_end <= s && run < 8);
+  };
+  auto reset = [&]() {
+    clear();
+    if constexpr (WL) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) tot[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < FM; ++j) ss_tot[j] = 0.f;
+      run = 0;
+      next_run(0);
+    }
+  };
+  auto fold = [&](int s) {   // after k-step s
+    if constexpr (WL) {
+      if (s + 1 != run_end) return;
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) tot[i][j] += acc[i][j];
+      if constexpr (AMODE == A_NORM) {
+#pragma unroll
+        for (int j = 0; j < FM; ++j) ss_tot[j] += over_groups(ss[j]);
+      }
+      clear();
+      next_run(s + 1);
+    }
+  };
+  auto result = [&](int i, int j) -> const f32x4_t& {
+    if constexpr (WL) return tot[i][j];
+    else return acc[i][j];
   };
 
   // k-step s from LDS, with the copies q0 .. q1 - 1 of the stage at `dst` spread over its MFMAs:
@@ -420,9 +470,9 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
       // previous tile's epilogue, ns >= 1 stage barriers ago)
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
-        float v = ss[j];
-        v += __shfl_xor(v, 16, kWave);
-        v += __shfl_xor(v, 32, kWave);
+        float v;
+        if constexpr (WL) v = ss_tot[j];
+        else v = over_groups(ss[j]);
         if (g == 0) rstd_s[16 * (FM * wm + j) + c] = rsqrtf(v / static_cast<float>(K) + p.eps);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -477,7 +527,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
         for (int i = 0; i < FN; ++i) {
           const int n = n0 + 16 * (FN * wn + i) + 4 * g;
           if (n >= N) continue;
-          const f32x4_t v = acc[i][j];
+          const f32x4_t v = result(i, j);
           if (lead_row)
             *reinterpret_cast<float4*>(p.out + static_cast<int64_t>(m) * p.ldo + n) =
                 make_float4(v[0], v[1], v[2], v[3]);
@@ -534,7 +584,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
             const int m = m0 + r;
             if (m >= M) continue;
             const float rs = AMODE == A_NORM ? rstd_s[r] : 1.f;
-            const f32x4_t gs = acc[2 * pb][j], us = acc[2 * pb + 1][j];
+            const f32x4_t gs = result(2 * pb, j), us = result(2 * pb + 1, j);
             // the arithmetic of K3 (swiglu.hip)
             const float o[4] = {silu_mul(fmaf(rs, gs[0], bg[q].x), fmaf(rs, us[0], bu[q].x)),
                                 silu_mul(fmaf(rs, gs[1], bg[q].y), fmaf(rs, us[1], bu[q].y)),
@@ -592,7 +642,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
           for (int j = 0; j < FM; ++j) {
             const int m = row(j);
             if (m >= M) continue;
-            const f32x4_t v = acc[i0 + u][j];
+            const f32x4_t v = result(i0 + u, j);
             if constexpr (EPI == E_RESIDUAL) {
               // x + delta, then + bias: the order of the add+RMSNorm kernel it replaces
               float4 x = xv[u][j];
@@ -673,6 +723,7 @@ __global__ __launch_bounds__(64 * S::NW, S::NW * S::OCC / 4) void prefill_gemm_k
     for (int ks = 0; ks < KS; ++ks) {
       constexpr int n = S::SPREAD ? kLoads : 0;
       compute(KS * cs + ks, lds + b * kStage + ks * kStep, dst, n * ks / KS, n * (ks + 1) / KS);
+      fold(KS * cs + ks);
     }
     advance_issue();
     stage_barrier<(kAhead - 1) * kLoads>();
@@ -812,11 +863,12 @@ int pick_shape(bool norm, int m, int n, int k) {
   return norm ? cheapest(kNorm, true, m, n, k) : cheapest(kSplit, false, m, n, k);
 }
 
-// The same for fp32 weights, against K5 (norm / out / gate-up / down, us; d = 768, F = 2048):
-//   731 rows     17 / 8 / 24 / 19         17 / 8 / 23 / 22
-//   2,300 rows   55 / 22 / 86 / 41        34 / 12 / 52 / 26
-//   11,242 rows  243 / 101 / 413 / 213    117 / 45 / 185 / 102
-// At 256 rows K5 takes 9 / 5 / 9 / 8 against 11 / 8 / 12 / 16: see kK5Rows.
+// The same for fp32 weights, us on K5 / here (qkv and K2, out, gate-up, down; d = 768, F = 2048):
+//   1,536 rows   45 / 18 / 57 / 39        31 / 13 / 40 / 27
+//   2,304 rows   68 / 23 / 87 / 45        45 / 14 / 74 / 31
+//   11,242 rows  260 / 98 / 388 / 211     171 / 53 / 297 / 128
+// The fold of the runs of k-steps (`fold`) is in these: in one run over all k-steps 28 / 12 / 35 /
+// 25, 41 / 13 / 80 / 30 and 160 / 52 / 280 / 126.
 int pick_shape_f32(bool norm, int m, int n, int k) {
   static constexpr StepCost kNorm[] = {step_cost<NormShapesF32::S0>(0.47f, 0.2f, 0.52f),
                                        step_cost<NormShapesF32::S1>(0.72f, 0.3f, 0.65f),
@@ -854,8 +906,11 @@ int launch_f32w(const Args& p, hipStream_t st) {
 }
 
 // fp32 weights: up to this many rows the projections run on K5, whose waves split K and need no
-// ring to fill (d = 768: 31 us a layer against 45 at 256 rows, 67 against 70 at 731)
-constexpr int kK5Rows = 640;
+// ring to fill, with the same bits; qkv up to the second, since past it K5 and K2 are slower than the
+// one launch.  Out, gate / up and down together, us on K5 / on K6: d = 768 at 384 rows 37 / 53, 768
+// 53 / 60, 896 60 / 63, 1,536 114 / 80; d = 1,280 at 768 rows 104 / 116, 896 150 / 120.  qkv: d = 768
+// at 384 rows 17.3 / 19.0, 512 24.5 / 22.4; d = 1,280 at 256 24.9 / 28.9, 384 35.0 / 32.2.
+constexpr int kK5Rows = 768, kK5RowsQkv = 448;
 
 // the split forms by A layout and parts: row-major activations, and the forms with the hi part
 // alone, are not on the prompt path and run on the large shape
@@ -1043,7 +1098,7 @@ extern "C" int mdl_prefill_gemm_norm_qkv_f32w(
       !aligned16(q_out) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned4(rope_tab))
     return MDL_ERR_ALIGN;
   if (m == 0) return MDL_OK;
-  if (m <= kK5Rows) {
+  if (m <= kK5RowsQkv) {
     rc = mdl_gemm_norm(x, gamma, eps, w, w_lo, qkv, ldq, rstd, m, 3 * d, d, 0, stream);
     if (rc != MDL_OK) return rc;
     return token_slot

@@ -792,9 +792,9 @@ struct SplitShapes {
 struct NormShapesF32 {
   using S0 = Shape<64, 64, 4, 1, 2, 2, 2, true, 1920>;
   using S1 = Shape<64, 128, 4, 1, 1, 3, 2, true, 1920>;
-  using S2 = Shape<128, 128, 4, 1, 1, 2, 2, true>;
-  using S3 = Shape<256, 128, 8, 1, 1, 3, 1, true>;
-  using S4 = S3;
+  using S2 = Shape<128, 128, 4, 1, 1, 2, 2, true>;   // every K
+  using S3 = S2;
+  using S4 = S2;
 };
 struct SplitShapesF32 {
   using S0 = Shape<64, 64, 4, 2, 2, 2, 2, true>;
@@ -872,8 +872,7 @@ int pick_shape(bool norm, int m, int n, int k) {
 int pick_shape_f32(bool norm, int m, int n, int k) {
   static constexpr StepCost kNorm[] = {step_cost<NormShapesF32::S0>(0.47f, 0.2f, 0.52f),
                                        step_cost<NormShapesF32::S1>(0.72f, 0.3f, 0.65f),
-                                       step_cost<NormShapesF32::S2>(1.1f, 0.2f, 1.25f, 12),
-                                       step_cost<NormShapesF32::S3>(1.5f, 1.5f, 1.42f)};
+                                       step_cost<NormShapesF32::S2>(1.1f, 0.2f, 1.25f)};
   static constexpr StepCost kSplit[] = {step_cost<SplitShapesF32::S0>(0.35f, 0.1f, 0.37f),
                                         step_cost<SplitShapesF32::S1>(0.5f, 0.1f, 0.63f),
                                         step_cost<SplitShapesF32::S2>(1.05f, 0.05f, 1.27f)};

@@ -42,7 +42,15 @@
 // bound by its longest block, whose SIMDs each work through all keys of 16 queries (64 fp32 MFMAs
 // of 32 cycles for 32 keys): there KG = 4 groups of QW waves take the tiles in turn, each with a
 // ring of its own, and merge their states in LDS at the end (8 ragged rows of up
-// to 1,001 tokens and 4 heads 61 -> 45 us).
+// to 1,001 tokens and 4 heads 61 -> 49 us).
+//
+// Order of the sums, causal: tile t of a row (from kv_start) belongs to chain t % 4, each chain is
+// an online softmax of its own, and chains 1, 2 and 3 are merged into chain 0 in that order.  The
+// four groups of waves hold one chain each; a block of one group holds all four (CH = 4, 72
+// registers: 3 waves per SIMD in place of 4), so a query's result does not depend on the size of
+// the launch.  That costs the large launches little (16 rows of up to 811 tokens and 12 heads 138 ->
+// 142 us, 64 of 200 and 16 heads 66 -> 69, 6 of 811 and 12 heads 72 -> 67).  Without the causal limit
+// there is one chain.
 //
 // Decode (attn_f32_decode_kernel): a work item is one split_len-slot chunk of one (row, head), a
 // wave of its own without LDS or barriers; the chunks are what fills the GPU.  The query fills all
@@ -130,9 +138,11 @@ __device__ __forceinline__ void store_out(const F32Args& p, int64_t qrow, int h,
 // Blocks: (row, head) pair i % 8 + 8 j on XCD i % 8, the latest (longest) query block of every pair
 // first, so that the short ones fill the end of the launch (pair by pair, the last pair's longest
 // blocks ran on alone: 213 -> 178 us).
-template <int QW, int KG>
-__global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefill_kernel(
-    const F32Args p) {
+template <int QW, int KG, int CH>
+__global__ __launch_bounds__(64 * QW * KG, CH > 1 ? 3 : QW == 2 ? 2 : 4) void
+attn_f32_prefill_kernel(const F32Args p) {
+  static_assert(KG == 1 || CH == 1, "the key groups or the chains take the tiles in turn");
+  static_assert(CH % 2 == 0 || CH == 1, "a turn of the chains ends on the ring's first stage");
   constexpr int kQB = kQT * QW;   // queries of a block
   const int slot = blockIdx.x >> 3, pairs = gridDim.x / (8 * p.q_tiles);   // pairs of an XCD
   const int qt = p.q_tiles - 1 - slot / pairs;
@@ -186,34 +196,18 @@ __global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefil
     return mrow && j < p.mask_len ? mrow[j] : 1;
   };
 
-  float m = -INFINITY, l = 0.f;   // l: this lane group's part of the sum
-  f32x4 o[4];
+  float m[CH], l[CH];   // l: this lane group's part of the sum
+  f32x4 o[CH][4];
 #pragma unroll
-  for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  constexpr int kStep = kKT * KG;
-  int ok_next = 0;
-  if (kstart + kKT * kg < kend) {
-    ok_next = key_ok(kstart + kKT * kg);
-    issue(kstart + kKT * kg, 0);
+  for (int ch = 0; ch < CH; ++ch) {
+    m[ch] = -INFINITY;
+    l[ch] = 0.f;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) o[ch][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // every wave of the block makes the same number of turns, so the barriers match; a group whose
-  // tile would start past the end neither copies nor computes
-  for (int t0 = kstart, st = 0; t0 < kend; t0 += kStep, st ^= 1) {
-    const int kt = t0 + kKT * kg;
-    // tile kt has landed for every wave, and every wave is done with the other stage (the builtin
-    // wait, so that the compiler counts its own loads, q and the mask bytes, as landed too)
-    __builtin_amdgcn_s_waitcnt(kWaitAll);
-    asm volatile("s_barrier" ::: "memory");
-    const uint32_t valid = static_cast<uint32_t>(__ballot(ok_next != 0));
-    if (kt + kStep < kend) {
-      ok_next = key_ok(kt + kStep);
-      issue(kt + kStep, st ^ 1);
-    }
-    if (kt >= kend) continue;
-    if (p.causal && kt > wq0 + kQT - 1) continue;   // the whole tile is in this wave's future
-    const uint8_t* Kt = lds[kg][st][0];
-    const uint8_t* Vt = lds[kg][st][1];
+
+  // the tile of keys kt .. kt + 31 at Kt / Vt into the state of chain ch
+  auto work = [&](int kt, uint32_t valid, const uint8_t* Kt, const uint8_t* Vt, int ch) {
     f32x4 s[2];
     float kv[2][16];
 #pragma unroll
@@ -249,10 +243,10 @@ __global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefil
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[nb][r]);
-    const float m_new = fmaxf(m, max_over_groups(tmax));
+    const float m_new = fmaxf(m[ch], max_over_groups(tmax));
     const float base = m_new == -INFINITY ? 0.f : m_new;   // no visible key yet: weights 0
-    const float alpha = __builtin_amdgcn_exp2f(m - base);
-    m = m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m[ch] - base);
+    m[ch] = m_new;
     float psum = 0.f;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
@@ -261,9 +255,9 @@ __global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefil
         s[nb][r] = __builtin_amdgcn_exp2f(s[nb][r] - base);
         psum += s[nb][r];
       }
-    l = fmaf(l, alpha, psum);
+    l[ch] = fmaf(l[ch], alpha, psum);
 #pragma unroll
-    for (int db = 0; db < 4; ++db) o[db] *= alpha;
+    for (int db = 0; db < 4; ++db) o[ch][db] *= alpha;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -273,40 +267,80 @@ __global__ __launch_bounds__(64 * QW * KG, QW == 2 ? 2 : 4) void attn_f32_prefil
         const float ve[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int db = 0; db < 4; ++db)
-          o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[db], 0, 0, 0);
+          o[ch][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[ch][db], 0, 0, 0);
       }
+  };
+
+  constexpr int kStep = kKT * KG;
+  int ok_next = 0;
+  if (kstart + kKT * kg < kend) {
+    ok_next = key_ok(kstart + kKT * kg);
+    issue(kstart + kKT * kg, 0);
+  }
+  // every wave of the block makes the same number of turns, so the barriers match; a group whose
+  // tile would start past the end neither copies nor computes
+  int st = 0;
+  for (int t0 = kstart; t0 < kend; t0 += kStep * CH) {
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch) {
+      const int kt = t0 + kStep * ch + kKT * kg;
+      if (CH > 1 && kt >= kend) break;   // whole block (KG is 1)
+      // tile kt has landed for every wave, and every wave is done with the other stage (the builtin
+      // wait, so that the compiler counts its own loads, q and the mask bytes, as landed too)
+      __builtin_amdgcn_s_waitcnt(kWaitAll);
+      asm volatile("s_barrier" ::: "memory");
+      const uint32_t valid = static_cast<uint32_t>(__ballot(ok_next != 0));
+      const int cur = CH > 1 ? ch & 1 : st;   // the tile's stage
+      st ^= 1;
+      if (kt + kStep < kend) {
+        ok_next = key_ok(kt + kStep);
+        issue(kt + kStep, cur ^ 1);
+      }
+      // nothing past the end, nor a tile that lies wholly in this wave's future
+      if (kt < kend && !(p.causal && kt > wq0 + kQT - 1))
+        work(kt, valid, lds[kg][cur][0], lds[kg][cur][1], ch);
+    }
+  }
+  // chain j's state (m, l, o) into chain 0's, j = 1, 2, 3 in order, whatever holds it
+  auto merge = [&](float mj, float lj, auto oj) {
+    const float m_new = fmaxf(m[0], mj);
+    const float base = m_new == -INFINITY ? 0.f : m_new;
+    const float a = __builtin_amdgcn_exp2f(m[0] - base), aj = __builtin_amdgcn_exp2f(mj - base);
+    m[0] = m_new;
+    l[0] = fmaf(lj, aj, l[0] * a);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      o[0][i >> 2][i & 3] = fmaf(oj(i), aj, o[0][i >> 2][i & 3] * a);
+  };
+  if constexpr (CH > 1) {
+#pragma unroll
+    for (int j = 1; j < CH; ++j)
+      merge(m[j], l[j], [&](int i) { return o[j][i >> 2][i & 3]; });
   }
   if constexpr (KG > 1) {
-    // the other groups' states (m, l, o) through the ring's memory, one float per lane at a time
+    // the other groups' states through the ring's memory, one float per lane at a time
     __syncthreads();   // every wave is done with its tiles
     float* part = reinterpret_cast<float*>(lds);
     if (kg > 0) {
       float* w = part + ((kg - 1) * QW + wave) * 18 * kWave + lane;
-      w[0] = m;
-      w[kWave] = l;
+      w[0] = m[0];
+      w[kWave] = l[0];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) w[(2 + i) * kWave] = o[i >> 2][i & 3];
+      for (int i = 0; i < 16; ++i) w[(2 + i) * kWave] = o[0][i >> 2][i & 3];
     }
     __syncthreads();
     if (kg > 0) return;
 #pragma unroll
     for (int j = 0; j < KG - 1; ++j) {
       const float* w = part + (j * QW + wave) * 18 * kWave + lane;
-      const float mj = w[0];
-      const float m_new = fmaxf(m, mj);
-      const float base = m_new == -INFINITY ? 0.f : m_new;
-      const float a = __builtin_amdgcn_exp2f(m - base), aj = __builtin_amdgcn_exp2f(mj - base);
-      m = m_new;
-      l = fmaf(w[kWave], aj, l * a);
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        o[i >> 2][i & 3] = fmaf(w[(2 + i) * kWave], aj, o[i >> 2][i & 3] * a);
+      merge(w[0], w[kWave], [&](int i) { return w[(2 + i) * kWave]; });
     }
   }
   if (qi >= S) return;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  store_out(p, qrow, h, g, l, o);
+  float sum = l[0];
+  sum += __shfl_xor(sum, 16, kWave);
+  sum += __shfl_xor(sum, 32, kWave);
+  store_out(p, qrow, h, g, sum, o[0]);
 }
 
 __global__ __launch_bounds__(64 * kWavesF) void attn_f32_decode_kernel(const F32Args p) {
@@ -454,12 +488,12 @@ __global__ __launch_bounds__(256) void attn_f32_combine_kernel(const float* __re
 
 constexpr int kBlocksSplit32 = 256, kBlocksSplit64 = 512;   // 64-query blocks
 
-template <int QW, int KG>
+template <int QW, int KG, int CH>
 int launch_prefill_f32(F32Args p, hipStream_t st) {
   p.q_tiles = (p.seq + kQT * QW - 1) / (kQT * QW);
   const int64_t blocks = (p.items + 7) / 8 * 8 * p.q_tiles;
   if (blocks > 0x7fffffff) return MDL_ERR_SHAPE;
-  hipLaunchKernelGGL((attn_f32_prefill_kernel<QW, KG>), dim3(static_cast<unsigned>(blocks)),
+  hipLaunchKernelGGL((attn_f32_prefill_kernel<QW, KG, CH>), dim3(static_cast<unsigned>(blocks)),
                      dim3(64 * QW * KG), 0, st, p);
   return launch_status();
 }
@@ -503,16 +537,17 @@ extern "C" int mdl_attn_prefill_f32(const float* q, const float* k_cache, const 
   p.out = out; p.out_layout = out_layout;
   if (p.items == 0) return MDL_OK;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  // How the longest block's chain of key tiles is cut while 64-query blocks number one or two per
-  // CU: four groups of waves take the tiles in turn, on 32 queries at up to one block per CU (so
-  // that twice as many CUs work) and on 64 at up to two.  Causal, us as one group of 64 / here:
-  // 144 blocks 34.6 / 20.0, 336 98 / 67, 512 60 / 47; at 940 265 / 265, at 2,496 110 / 140.
-  // Without the causal limit every block is as long as the longest, and one group is as good or
-  // better (144: 37.5 / 39.2, 432: 47.6 / 49.7).
+  // How the longest block's key tiles are split while 64-query blocks number one or two per CU:
+  // four groups of waves take the tiles in turn, on 32 queries at up to one block per CU (so that
+  // twice as many CUs work) and on 64 at up to two.  Causal, us as one group of 64 / here: 60
+  // blocks 17.0 / 10.9, 144 34.7 / 20.3, 432 33.3 / 28.5, 512 60.1 / 49.4.  Past that as one group
+  // (here) / as four: 528 45.1 / 43.7, 600 44.5 / 47.9, 624 56.9 / 50.0, 936 67 / 74, 2,496 142 /
+  // 182.  Without the causal limit every block is as long as the longest, and one group is as good
+  // or better (144: 37.5 / 39.2, 432: 47.6 / 49.7).
   const int64_t blocks = p.items * ((seq + 63) / 64);
-  if (p.causal && blocks <= kBlocksSplit32) return launch_prefill_f32<2, 4>(p, st);
-  if (p.causal && blocks <= kBlocksSplit64) return launch_prefill_f32<4, 4>(p, st);
-  return launch_prefill_f32<4, 1>(p, st);
+  if (p.causal && blocks <= kBlocksSplit32) return launch_prefill_f32<2, 4, 1>(p, st);
+  if (p.causal && blocks <= kBlocksSplit64) return launch_prefill_f32<4, 4, 1>(p, st);
+  return p.causal ? launch_prefill_f32<4, 1, 4>(p, st) : launch_prefill_f32<4, 1, 1>(p, st);
 }
 
 extern "C" int mdl_attn_decode_f32(const float* q, const float* k_cache, const float* v_cache,

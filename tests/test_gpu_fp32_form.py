@@ -422,3 +422,41 @@ def test_attn_prefill_f32_block_shapes(S, blocks, packed):
         r0 = int(off[b]) if packed else b * S
         want = ref[i].transpose(0, 1)[lo:]                   # [S - lo, H, 64]
         _attn_close(got[r0:r0 + S - lo], want, f"row {b}")
+
+
+@pytest.mark.parametrize("S", [1, 33, 130, 300, 811])
+@pytest.mark.parametrize("packed", [False, True])
+def test_attn_prefill_f32_rows_do_not_depend_on_the_launch(S, packed):
+    """Four groups of waves (launches of up to 256 and 512 blocks) and one group with four chains
+    take a row's key tiles in the same order: causal rows alone give the same bits as the same rows
+    in a large launch, padded or packed."""
+    g = torch.Generator().manual_seed(S)
+    H, slots = 4, S + 2
+    kv = [0, S // 3, min(S - 1, 45)]
+    pm = torch.ones(3, S, dtype=torch.uint8)
+    for b in range(3):
+        pm[b, :kv[b]] = 0
+    pm[0, S // 2:S // 2 + 40] = 0                     # a hole of more than a tile
+    pm[0, 0] = 1
+    q = torch.randn(3, S, H * 64, generator=g) * 0.3
+    kc, vc = (torch.randn(3, H, slots, 64, generator=g) for _ in range(2))
+
+    def rows(idx):
+        B, kvi = len(idx), torch.tensor([kv[i] for i in idx], dtype=torch.int32)
+        qi, off = q[idx].reshape(-1, H * 64), None
+        if packed:
+            qi = torch.cat([q[i, kv[i]:] for i in idx])
+            off = (torch.cumsum(S - kvi, 0) - (S - kvi)).to(torch.int32).to(DEV)
+        out = torch.zeros(qi.shape[0], 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+        K().attn_prefill_f32(qi.contiguous().to(DEV), kc[idx].to(DEV), vc[idx].to(DEV), B, S, H,
+                             pm[idx].to(DEV), kvi.to(DEV), off, qi.shape[0], True, out)
+        o = out.cpu()
+        n = [S - kv[i] if packed else S for i in idx]
+        return [o[sum(n[:j]):sum(n[:j + 1])] for j in range(3)]
+
+    per = H * -(-S // 64)                             # 64-query blocks of a row
+    alone = rows([0, 1, 2])
+    for blocks in (255, 511, 700):
+        many = rows([j % 3 for j in range(max(3, blocks // per))])
+        for b in range(3):
+            assert torch.equal(many[b], alone[b]), (blocks, b)

@@ -259,7 +259,10 @@ attn_f32_prefill_kernel(const F32Args p) {
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[ch][db] *= alpha;
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int nb = 0; nb < 2; ++nb) {
+      // sixteen keys past the row or in this wave's future: their weights are zero, but zero times
+      // a value that is not finite is NaN
+      if (nb == 1 && (kt + 16 >= S || (p.causal && kt + 16 > wq0 + kQT - 1))) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * nb + 4 * g + r;
@@ -269,6 +272,7 @@ attn_f32_prefill_kernel(const F32Args p) {
         for (int db = 0; db < 4; ++db)
           o[ch][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(ve[db], s[nb][r], o[ch][db], 0, 0, 0);
       }
+    }
   };
 
   constexpr int kStep = kKT * KG;

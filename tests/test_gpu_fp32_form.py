@@ -460,3 +460,29 @@ def test_attn_prefill_f32_rows_do_not_depend_on_the_launch(S, packed):
         many = rows([j % 3 for j in range(max(3, blocks // per))])
         for b in range(3):
             assert torch.equal(many[b], alone[b]), (blocks, b)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("B", [1, 40])                # four groups of waves, one group
+def test_attn_prefill_f32_leaves_later_values_out(bad, B):
+    """A value that is not finite changes no query before its sixteen keys, and as the last key of a
+    row it reaches the queries that see it as itself."""
+    g = torch.Generator().manual_seed(5)
+    H, S = 4, 208
+    q = (torch.randn(B * S, H * 64, generator=g) * 0.3).to(DEV)
+    kc, vc = (torch.randn(B, H, S, 64, generator=g).to(DEV) for _ in range(2))
+
+    def run(causal):
+        out = torch.empty(B * S, 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+        K().attn_prefill_f32(q, kc, vc, B, S, H, None, None, None, B * S, causal, out)
+        return out.view(B, S, 2, H, 64)[:, :, 0].clone()
+
+    want = run(True)
+    vc[:, 1, 80, 3] = bad                             # keys 80 .. 95, the second half of a tile
+    vc[:, 2, 207, 3] = bad                            # the second half of the last tile has no key
+    got = run(True)
+    assert torch.equal(got[:, :80], want[:, :80])
+    assert torch.equal(got[:, :192, 2], want[:, :192, 2])
+    assert not bool(got[:, 80:, 1, 3].isfinite().any())
+    last = run(False)[:, :, 2, 3]
+    assert bool((last.isnan() if bad != bad else last == bad).all())

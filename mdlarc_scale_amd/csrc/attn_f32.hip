@@ -245,16 +245,35 @@ attn_f32_prefill_kernel(const F32Args p) {
       for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[nb][r]);
     const float m_new = fmaxf(m[ch], max_over_groups(tmax));
     const float base = m_new == -INFINITY ? 0.f : m_new;   // no visible key yet: weights 0
-    const float alpha = __builtin_amdgcn_exp2f(m[ch] - base);
+    const float alpha = exp2f(m[ch] - base);
     m[ch] = m_new;
-    float psum = 0.f;
+    // exp2f scales its argument to keep results below 2^-126, five instructions more than the bare
+    // one, which gives the same bits above: taken where a weight may lie there (2,496 blocks 142 us
+    // without it, 150 with it for every weight, 144 so)
+    float least = s[0][0];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        s[nb][r] = __builtin_amdgcn_exp2f(s[nb][r] - base);
-        psum += s[nb][r];
+        least = fminf(least, s[nb][r]);
+        s[nb][r] -= base;
       }
+    if (__any(least - base < -126.f)) {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[nb][r] = exp2f(s[nb][r]);
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[nb][r] = __builtin_amdgcn_exp2f(s[nb][r]);
+    }
+    float psum = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) psum += s[nb][r];
     l[ch] = fmaf(l[ch], alpha, psum);
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[ch][db] *= alpha;
@@ -309,7 +328,7 @@ attn_f32_prefill_kernel(const F32Args p) {
   auto merge = [&](float mj, float lj, auto oj) {
     const float m_new = fmaxf(m[0], mj);
     const float base = m_new == -INFINITY ? 0.f : m_new;
-    const float a = __builtin_amdgcn_exp2f(m[0] - base), aj = __builtin_amdgcn_exp2f(mj - base);
+    const float a = exp2f(m[0] - base), aj = exp2f(mj - base);
     m[0] = m_new;
     l[0] = fmaf(lj, aj, l[0] * a);
 #pragma unroll

@@ -486,3 +486,24 @@ def test_attn_prefill_f32_leaves_later_values_out(bad, B):
     assert not bool(got[:, 80:, 1, 3].isfinite().any())
     last = run(False)[:, :, 2, 3]
     assert bool((last.isnan() if bad != bad else last == bad).all())
+
+
+@pytest.mark.parametrize("B", [1, 60])                # four groups of waves, one group
+def test_attn_prefill_f32_keeps_weights_below_the_normal_range(B):
+    """A weight of 2^-130 is a denormal fp32 number, and counts: times a value of 2^127 it is 1/8."""
+    H, S = 4, 192
+    q = torch.zeros(B * S, H * 64, device=DEV)
+    q[:, ::64] = 1.0                                  # the score is the key's first channel
+    kc, vc = torch.zeros(2, B, H, S, 64, device=DEV).unbind()
+    kc[..., 0] = -130.0
+    heavy = torch.arange(4) * 32                      # in each of four tiles a key of weight 1
+    kc[:, :, heavy, 0] = 0.0
+    vc[..., 5] = 2.0 ** 127
+    vc[:, :, heavy, 5] = 0.0
+    out = torch.empty(B * S, 2 * H * 64, device=DEV, dtype=torch.bfloat16)
+    K().attn_prefill_f32(q, kc, vc, B, S, H, None, None, None, B * S, True, out)
+    got = unsplit(out.cpu()).view(B, S, H, 64)[..., 5]
+    seen = torch.arange(S) // 32 + 1
+    n = torch.minimum(seen, torch.tensor(4))          # heavy keys that a query sees
+    want = ((torch.arange(S) + 1 - n) / 8.0 / n)[:, None]
+    assert bool(((got - want).abs() <= 2 ** -15 * want).all())   # the split of the output

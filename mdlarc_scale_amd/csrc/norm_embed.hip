@@ -492,9 +492,13 @@ using namespace mdl;
 
 namespace mdl {
 
-// Rows from which the sixteen-row kernel is the faster one (fp32 tables: 2.7 us against 2.4 at 256
-// rows, 3.0 against 3.2 at 1,024; bf16: 2.25 against 1.9 at one row, 2.0 against 2.3 at 8)
-constexpr int kEmbTileRowsF32 = 1024, kEmbTileRowsBf16 = 8;
+// Rows from which the sixteen-row kernel is the faster one, us against the row kernel: bf16 tables
+// at d = 768 2.2 / 1.85 at one row, 1.97 / 2.26 at 8, 2.28 / 2.49 at 64, 2.6 / 3.2 at 1,024; fp32 ones
+// 2.84 / 2.6 at 256, 3.07 / 3.23 at 1,024.  A narrow row (d = 256) is one load of a wave: bf16 2.25 /
+// 2.06 at 64, 2.35 / 2.29 at 1,024, 2.50 / 2.62 at 2,048; fp32 2.78 / 2.46, 2.96 / 2.86 and at 4,096
+// 3.26 / 3.60.
+constexpr int kEmbTileRowsF32 = 1024, kEmbTileRowsBf16 = 8, kEmbTileRowsNarrow = 2048;
+constexpr int kEmbNarrow = 512;   // channels
 
 // x in the tile layout, the sixteen-row kernel; `pk` NULL: ids in row order
 template <typename TT>
@@ -567,7 +571,9 @@ extern "C" int mdl_embed_rmsnorm(const int64_t* ids, const int64_t* example_ids,
   const dim3 grid((rows + 3) / 4);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (layout == MDL_LAYOUT_TILES && !xs_out && !rstd_out &&   // x alone
-      rows >= (table_dtype == MDL_DTYPE_F32 ? kEmbTileRowsF32 : kEmbTileRowsBf16))
+      rows >= (d < kEmbNarrow                 ? kEmbTileRowsNarrow
+               : table_dtype == MDL_DTYPE_F32 ? kEmbTileRowsF32
+                                              : kEmbTileRowsBf16))
     return table_dtype == MDL_DTYPE_F32
                ? launch_embed_tiles<float>(ids, example_ids, tok_table, ex_table, vocab,
                                            n_examples, rows, row_len, d, x_out, nullptr, s)

@@ -1547,7 +1547,7 @@ def test_embed_x_alone_in_tiles(d, table_dtype, with_ex):
     tok = torch.randn(14, d, generator=g).to(table_dtype).to(DEV)
     ex = torch.randn(5, d, generator=g).to(table_dtype).to(DEV) if with_ex else None
     gamma = torch.ones(d, device=DEV)
-    for B, S in ((1, 1), (3, 5), (2, 16), (7, 33), (31, 34)):
+    for B, S in ((1, 1), (3, 5), (2, 16), (7, 33), (31, 34), (61, 34)):
         ids = torch.randint(-2, 17, (B, S), generator=g).to(DEV)      # clamped into the table
         exi = torch.randint(0, 5, (B,), generator=g).to(DEV) if with_ex else None
         pos = torch.randint(0, 30, (B, S, 3), generator=g).to(DEV)

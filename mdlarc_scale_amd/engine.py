@@ -460,8 +460,8 @@ class HipEngine:
         if nx:
             pos_p = torch.empty(pk.n_tokens, 3, dtype=pos.dtype, device=pos.device)
             K.embed_packed(ids.contiguous(), pos.contiguous(),
-                           ex_ids.reshape(-1) if use_ex else None, tok, ex if use_ex else None,
-                           pk.gather, pk.token_row, sc.x, pos_p)
+                           ex_ids.reshape(-1).contiguous() if use_ex else None, tok,
+                           ex if use_ex else None, pk.gather, pk.token_row, sc.x, pos_p)
         else:
             ids_p = ids.reshape(-1).index_select(0, pk.gather)
             pos_p = pos.reshape(-1, 3).index_select(0, pk.gather)

@@ -965,6 +965,34 @@ def test_packed_prefill_equals_padded(form, monkeypatch):
                 assert bool(((x - y).abs() <= tol * y.abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("form", FORMS)
+def test_packed_prompt_takes_an_expanded_example_id(form):
+    """One example id for all rows, as an expanded view: the packed prompt of the same ids written
+    out, bit for bit."""
+    from mdlarc_scale_amd import inference as inf
+    from mdlarc_scale_amd.engine import Scratch, pack_prompt
+
+    m, _ = _preset_model("tiny", form, seed=4, max_seq_len=512)
+    ids, pos, mask = _left_pad(_random_prompts(np.random.default_rng(3), 3, 1, 2, 5))
+    ids, pos, mask = ids.to(DEV), pos.to(DEV), mask.to(DEV)
+    B, S = ids.shape
+    one = torch.tensor([7], device=DEV)
+    res = []
+    for ex in (one.repeat(B), one.expand(B)):
+        gen = inf.Generator(m)
+        with torch.no_grad():
+            W = gen.eng.packed(ids.device)
+            st = gen.prepare(ids, pos, ex, mask, S + 4)
+            starts = torch.stack([st.kv_start, st.last_row]).cpu().numpy()
+            pk = pack_prompt(starts[0], starts[1], B, S, ids.device)
+            sc = Scratch.for_prompt(pk.n_tokens, m.config, ids.device, W.f32)
+            sc.x.zero_()
+            gen.eng.run_packed(W, ids, pos, ex, st.pmask, st.kv_start, pk, st.cache.layer, sc,
+                               row_holes=st.holes)
+        res.append(sc.x.clone())
+    assert torch.equal(*res)
+
+
 def test_decode_forms_agree(monkeypatch):
     """The decode step on K5 with the norms, SwiGLU and residual adds fused (five launches per
     layer, tiled x) against the separate-kernel form (hipBLASLt, add+RMSNorm, K3; row-major):

@@ -348,9 +348,12 @@ class HipEngine:
     def _signature(self) -> tuple:
         # every parameter outside the embedding tables, straight from the module tree:
         # named_parameters builds a name and a set entry for each (60 us for 43 of them, this 15)
-        sig, todo = [], [self.model]
+        sig, todo, seen = [], [self.model], set()
         while todo:
             m = todo.pop()
+            if id(m) in seen:   # a module reached by two ways, or one that holds its parent
+                continue
+            seen.add(id(m))
             for p in m._parameters.values():
                 if p is not None:
                     sig.append((p.data_ptr(), p._version, p.dtype, p.device))

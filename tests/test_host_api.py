@@ -234,3 +234,22 @@ def test_fp32_form_requires_k5_widths():
                       torch.device("cpu"))
     with pytest.raises(TypeError, match="float32 and bfloat16"):
         model_form(M.create_model(d_model=128, n_heads=2, n_layers=1, d_ff=64).half())
+
+
+def test_weights_signature_of_shared_and_cyclic_modules():
+    """The engine's record of the parameters ends, and has each once, where a module is held twice or
+    holds its parent; the embedding tables are not part of it, a changed weight is."""
+    from mdlarc_scale_amd.engine import HipEngine
+
+    m = M.create_model(d_model=128, n_heads=2, n_layers=2, d_ff=64)
+    plain = HipEngine(m)._signature()
+    m.also = m.blocks[0]
+    m.blocks[0].parent = m
+    signal = HipEngine(m)._signature()
+    assert sorted(map(str, signal)) == sorted(map(str, plain))
+    assert len(plain) == len(list(m.parameters())) - 2
+    with torch.no_grad():
+        m.token_embed.weight.add_(1)
+        assert HipEngine(m)._signature() == signal
+        m.blocks[1].ffn.fc_up.bias.add_(1)
+    assert HipEngine(m)._signature() != signal

@@ -643,7 +643,9 @@ int mdl_attn_decode_f32(const float* q, const float* k_cache, const float* v_cac
  *     mask is the key mask [batch, seq].
  *   mdl_decode_layers: per layer mdl_gemm_norm_qkv, mdl_attn_decode, mdl_gemm_split_residual,
  *     mdl_gemm_norm_swiglu, mdl_gemm_split_residual, with rows == batch; mask is the prompt mask
- *     [batch, seq], the token's slot is *slot_dev.
+ *     [batch, seq], the token's slot is *slot_dev (not NULL).
+ * Refused before the first launch: slots outside 1 .. INT_MAX, f32 with an absent *_lo, at decode
+ * rows != batch and a NULL slot_dev.
  * Replaces: the layer loops of _prefill / _decode_step (src/inference.py:397-415, :437-456) and
  *           TinyTransformer.forward (src/transformer.py:591-604).
  */

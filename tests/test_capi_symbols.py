@@ -163,3 +163,40 @@ def test_argument_errors_are_reported_before_any_launch():
                                    1, 64, None, None, None, fake, 3, None) == -3
     with pytest.raises(RuntimeError, match="head_dim"):
         _lib.check(-4, "probe")
+
+
+def _fake_stack(**kw):
+    """A two-layer mdl_stack of pointers that are never dereferenced, with ``kw`` changed: a name of
+    mdl_stack, or one of mdl_layer for the second layer."""
+    import ctypes
+
+    fake = 1 << 20
+    layers = (_lib.Layer * 2)()
+    for rec in layers:
+        for name, kind in _lib.Layer._fields_:
+            setattr(rec, name, 64 if name == "slots" else fake)
+    ints = dict(n_layers=2, f32=1, rows=4, batch=4, seq=1, n_heads=2, d_ff=64, max_x=32, max_y=32,
+                max_z=8, px=10, py=10, pz=12, split_len=64, ws_bytes=1 << 30)
+    ptrs = {n: fake for n, t in _lib.Stack._fields_ if t is ctypes.c_void_p}
+    stack = _lib.Stack(layers=layers, **ints, **ptrs)
+    for name, v in kw.items():
+        setattr(layers[1] if hasattr(layers[1], name) else stack, name, v)
+    return ctypes.byref(stack)
+
+
+def test_layer_stacks_refuse_what_their_entries_cannot_see():
+    """Checks of the whole stack, ahead of the first layer's launches."""
+    _require_lib()
+    L = _lib.lib()
+    for entry in (L.mdl_prompt_layers, L.mdl_decode_layers):
+        assert entry(None, None) == -1
+        assert entry(_fake_stack(layers=None), None) == -1
+        assert entry(_fake_stack(n_layers=-1), None) == -3
+        assert entry(_fake_stack(n_heads=0), None) == -3
+        for slots in (0, -1, 1 << 31, (1 << 32) + 64):
+            assert entry(_fake_stack(slots=slots), None) == -3, slots
+        for lo in ("qkv_lo", "out_lo", "gu_lo", "down_lo"):
+            assert entry(_fake_stack(**{lo: None}), None) == -1, lo
+    # K5 writes K / V of `rows` rows, the attention reads those of `batch`
+    assert L.mdl_decode_layers(_fake_stack(rows=5), None) == -3
+    assert L.mdl_decode_layers(_fake_stack(slot_dev=None), None) == -1

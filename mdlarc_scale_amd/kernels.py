@@ -926,8 +926,8 @@ def _stack(W, cfg, sc, kv_layers, rows: int, batch: int, seq: int, pos: torch.Te
             shape = c.shape
             if len(shape) != 4 or shape[0] != batch or shape[1] != H or shape[3] != HEAD_DIM:
                 raise ValueError(f"{name} must be [batch, n_heads, slots, 64]")
-        if vc.shape[2] < kc.shape[2]:
-            raise ValueError("v_cache has fewer slots than k_cache")
+        if vc.shape[2] != kc.shape[2]:   # one row stride serves both
+            raise ValueError("v_cache and k_cache differ in slots")
         rec.k_cache, rec.v_cache, rec.slots = kc.data_ptr(), vc.data_ptr(), kc.shape[2]
     p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     mx, my, mz, px, py, pz = W.rope_geom

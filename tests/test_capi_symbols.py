@@ -200,3 +200,28 @@ def test_layer_stacks_refuse_what_their_entries_cannot_see():
     # K5 writes K / V of `rows` rows, the attention reads those of `batch`
     assert L.mdl_decode_layers(_fake_stack(rows=5), None) == -3
     assert L.mdl_decode_layers(_fake_stack(slot_dev=None), None) == -1
+
+
+def test_layer_stack_wrapper_refuses_caches_of_different_slots(monkeypatch):
+    """K and V of a layer share one row stride, so a longer V is refused like a shorter one."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from mdlarc_scale_amd import kernels as K
+
+    monkeypatch.setattr(K, "_need", lambda *a, **k: None)
+    n = torch.empty(0)
+    W = SimpleNamespace(f32=False, rope_tab=n, rope_geom=(32, 32, 8, 10, 10, 12), eps=1e-5,
+                        layers=bytes((_lib.Layer * 1)()))
+    sc = SimpleNamespace(x=n, q=n, qkv=n, rstd=n, attn=n, h=n)
+    cfg = SimpleNamespace(n_heads=2, n_layers=1, d_ff=64)
+    for k_slots, v_slots in ((8, 8), (8, 9), (9, 8)):
+        caches = torch.empty(3, 2, k_slots, 64), torch.empty(3, 2, v_slots, 64)
+        stack = lambda: K._stack(W, cfg, sc, lambda li: caches, 3, 3, 5, n, 1.0, None,  # noqa: E731
+                                 None, None)
+        if k_slots == v_slots:
+            assert stack().layers[0].slots == k_slots
+        else:
+            with pytest.raises(ValueError, match="slots"):
+                stack()

@@ -441,9 +441,10 @@ int mdl_prefill_gemm_norm_qkv(const float* x, const float* gamma, float eps, con
                               const int32_t* token_row, const int32_t* token_slot, void* stream);
 /*
  * mdl_prefill_gemm_norm_qkv of an fp32 weight (w, w_lo) for an fp32 cache: fp32 q [m, d], K and V,
- * no lead rows.  Small row counts run as mdl_gemm_norm and mdl_qkv_rope_cache through the scratch
- * qkv [m, ldq >= 3 d] and rstd [m], which are otherwise not written.
+ * no lead rows.  Up to MDL_F32W_QKV_ROWS rows run as mdl_gemm_norm and mdl_qkv_rope_cache through the
+ * scratch qkv [m, ldq >= 3 d] and rstd [m]; with more rows both are not written (never NULL).
  */
+#define MDL_F32W_QKV_ROWS 448
 int mdl_prefill_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps,
                                    const uint16_t* w, const uint16_t* w_lo, int m, int n_heads,
                                    float* qkv, int64_t ldq, float* rstd, const int64_t* pos,

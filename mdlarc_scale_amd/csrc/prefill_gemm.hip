@@ -909,7 +909,7 @@ int launch_f32w(const Args& p, hipStream_t st) {
 // one launch.  Out, gate / up and down together, us on K5 / on K6: d = 768 at 384 rows 37 / 53, 768
 // 53 / 60, 896 60 / 63, 1,536 114 / 80; d = 1,280 at 768 rows 104 / 116, 896 150 / 120.  qkv: d = 768
 // at 384 rows 17.3 / 19.0, 512 24.5 / 22.4; d = 1,280 at 256 24.9 / 28.9, 384 35.0 / 32.2.
-constexpr int kK5Rows = 768, kK5RowsQkv = 448;
+constexpr int kK5Rows = 768, kK5RowsQkv = MDL_F32W_QKV_ROWS;   // 448
 
 // the split forms by A layout and parts: row-major activations, and the forms with the hi part
 // alone, are not on the prompt path and run on the large shape

@@ -224,30 +224,28 @@ class Scratch:
         (whole 16-row blocks); the RMSNorms run inside the K5 launches (``HipEngine._mlp``).
         ``fused``: the prompt form on K6 -- the same layouts; the RMSNorms run inside the K6
         launches.  ``f32``: the fp32 form (prompt or decode) -- the ``tiled`` layouts on K5,
-        q in fp32, qkv the fp32 projection output of every row."""
+        q in fp32, qkv the fp32 projection output of every row (``fused`` with ``f32``, a prompt on
+        K6: of the few rows that do not run in one launch)."""
         e = lambda *s, dt=torch.bfloat16: torch.empty(*s, dtype=dt, device=device)  # noqa: E731
         f = torch.float32
         tiled = tiled or f32
         split_gemm = not (tiled or fused)               # hipBLASLt path: xs, delta, gu
         sr = rows if split_gemm else K.tile_rows(rows)  # rows of the tiled activations
-        fused = fused and not f32
+        fused, fused_f32 = fused and not f32, fused and f32
+        qkv_rows = min(rows, K.F32W_QKV_ROWS) if fused_f32 else rows
         h_parts = PROMPT_DOWN_PARTS if fused else 2
         return Scratch(x=e(sr, d, dt=f), xs=e(sr if split_gemm else 0, 2 * d),
-                       rstd=e(rows, dt=f), qkv=e(rows, 3 * d, dt=f),
+                       rstd=e(rows, dt=f), qkv=e(qkv_rows, 3 * d, dt=f),
                        q=e(rows, d, dt=f if f32 else torch.bfloat16),
                        attn=e(sr, 2 * d), delta=e(rows if split_gemm else 0, d, dt=f),
                        gu=e(rows if split_gemm else 0, 2 * d_ff, dt=f), h=e(sr, h_parts * d_ff),
-                       rows=rows, tiled=tiled, fused=fused, f32=f32)
+                       rows=rows, tiled=tiled, fused=fused, f32=f32, fused_f32=fused_f32)
 
     @staticmethod
     def for_prompt(rows: int, cfg, device: torch.device, f32: bool) -> "Scratch":
-        """Scratch of a prompt pass: the fp32 form, or the bf16 form on K6 when the model's
-        shapes fit it (hipBLASLt otherwise)."""
-        if f32:
-            sc = Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device, f32=True)
-            sc.fused_f32 = prompt_gemms_fused(cfg.d_model, cfg.d_ff)
-            return sc
-        return Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device,
+        """Scratch of a prompt pass: on K6 when the model's shapes fit it (otherwise the fp32 form is on
+        K5, the bf16 form on hipBLASLt)."""
+        return Scratch.alloc(rows, cfg.d_model, cfg.d_ff, device, f32=f32,
                              fused=prompt_gemms_fused(cfg.d_model, cfg.d_ff))
 
 

@@ -476,6 +476,7 @@ def gemm_split_residual(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor,
 
 
 PREFILL_NORM_MAX_K = 2048   # K6 norm forms: gamma is staged in LDS (kMaxNormK)
+F32W_QKV_ROWS = 448         # MDL_F32W_QKV_ROWS: rows of fp32 qkv scratch on K6 with fp32 weights
 
 
 def _split_a(a: torch.Tensor, m: int, k: int, tiled: bool, parts: int = 2) -> tuple[int, int]:
@@ -655,16 +656,16 @@ def prefill_gemm_norm_qkv_f32w(x: torch.Tensor, gamma: torch.Tensor, eps: float,
                                token_row: torch.Tensor | None = None,
                                token_slot: torch.Tensor | None = None, seq: int = 0) -> None:
     """prefill_gemm_norm_qkv of an fp32 weight (w, w_lo) for an fp32 cache: fp32 q [rows, d], K and
-    V; qkv [rows, 3d] and rstd [rows] are scratch of small row counts."""
+    V; qkv [rows, 3d] and rstd [rows] are scratch of up to F32W_QKV_ROWS rows."""
     d = n_heads * HEAD_DIM
     _need(x, "x", F32, tile_rows(rows) * d)
     _need(gamma, "gamma", F32, d)
     _need(w, "w", BF16, tile_rows(3 * d) * d)
     _need(w_lo, "w_lo", BF16, tile_rows(3 * d) * d)
-    _need(qkv, "qkv", F32, rows * 3 * d)
+    _need(qkv, "qkv", F32, min(rows, F32W_QKV_ROWS) * 3 * d)
     if qkv.dim() != 2 or qkv.shape[1] != 3 * d:
         raise ValueError(f"qkv must be [rows, {3 * d}]")
-    _need(rstd, "rstd", F32, rows)
+    _need(rstd, "rstd", F32, min(rows, F32W_QKV_ROWS))
     _need(pos, "pos", I64, rows * 3)
     _need(rope_tab, "rope_tab", F32)
     _need(q_out, "q_out", F32, rows * d)
@@ -908,7 +909,7 @@ def _stack(W, cfg, sc, kv_layers, rows: int, batch: int, seq: int, pos: torch.Te
     dt = F32 if W.f32 else BF16
     _need(sc.x, "x", F32, tile_rows(rows) * d)
     _need(sc.q, "q", dt, rows * d)
-    _need(sc.qkv, "qkv", F32, rows * 3 * d)
+    _need(sc.qkv, "qkv", F32, (min(rows, F32W_QKV_ROWS) if W.f32 else rows) * 3 * d)
     _need(sc.rstd, "rstd", F32, rows)
     _need(sc.attn, "attn", BF16, split_numel(rows, d, True))
     _need(pos, "pos", I64, rows * 3)

@@ -202,6 +202,27 @@ def test_layer_stacks_refuse_what_their_entries_cannot_see():
     assert L.mdl_decode_layers(_fake_stack(slot_dev=None), None) == -1
 
 
+def test_fp32_prompt_scratch():
+    """The fp32 projection scratch of an fp32 model's prompt on K6 holds the rows that the header
+    names and no more; the other forms' holds every row."""
+    import re
+
+    import torch
+
+    from mdlarc_scale_amd import kernels as K
+    from mdlarc_scale_amd.engine import Scratch
+    from mdlarc_scale_amd.transformer import TransformerConfig as Config
+
+    src = open(_lib.HEADER).read()
+    rows = int(re.search(r"define MDL_F32W_QKV_ROWS (\d+)", src).group(1))
+    assert K.F32W_QKV_ROWS == rows
+    cpu = torch.device("cpu")
+    for d, n, f32, want in ((256, rows + 1, True, rows), (256, 5, True, 5),
+                            (256, rows + 1, False, rows + 1), (2304, rows + 1, True, rows + 1)):
+        cfg = Config(d_model=d, n_heads=d // 64, d_ff=64)
+        assert Scratch.for_prompt(n, cfg, cpu, f32).qkv.shape == (want, 3 * d)
+
+
 def test_layer_stack_wrapper_refuses_caches_of_different_slots(monkeypatch):
     """K and V of a layer share one row stride, so a longer V is refused like a shorter one."""
     from types import SimpleNamespace

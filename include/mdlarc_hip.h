@@ -454,6 +454,16 @@ int mdl_prefill_gemm_norm_qkv_f32w(const float* x, const float* gamma, float eps
                                    const int32_t* token_row, const int32_t* token_slot,
                                    void* stream);
 /*
+ * The block shape (0 .. mdl_prefill_gemm_shapes(form) - 1, smallest tile first) that K6 takes for an
+ * [m, k] x [n, k]^T product on the current device, a_parts 2 and tiled operands (host only).
+ */
+#define MDL_GEMM_NORM 0        /* activation: x * gamma through the RMSNorm prologue */
+#define MDL_GEMM_SPLIT 1       /* activation: tiled split */
+#define MDL_GEMM_NORM_F32W 2   /* the same with fp32 weights, past the row counts that run on K5 */
+#define MDL_GEMM_SPLIT_F32W 3
+int mdl_prefill_gemm_shapes(int form);
+int mdl_prefill_gemm_pick(int form, int m, int n, int k);
+/*
  * dst = src ([rows, cols] bf16, row stride ld) in MDL_LAYOUT_TILES, rows padded to a multiple
  * of 16 with zeros (dst holds ceil(rows / 16) * 16 * cols elements).  cols a multiple of 32.
  * Packs the decode weights once per model version (no reference counterpart: a layout step).

@@ -109,6 +109,8 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "mdl_prefill_gemm_norm_qkv_f32w": (c_int, [P, P, c_float, P, P, c_int, c_int, P, c_int64, P, P,
                                                P, c_int, c_int, c_int, c_int, c_int, c_int,
                                                c_float, P, P, P, c_int, c_int, c_int, P, P, P]),
+    "mdl_prefill_gemm_shapes": (c_int, [c_int]),
+    "mdl_prefill_gemm_pick": (c_int, [c_int, c_int, c_int, c_int]),
     "mdl_zero_tiled_rows": (c_int, [P, c_int, c_int, c_int, P]),
     "mdl_prompt_layers": (c_int, [STACK, P]),
     "mdl_decode_layers": (c_int, [STACK, P]),

@@ -845,10 +845,10 @@ int cheapest(const StepCost (&costs)[COUNT], bool norm, int m, int n, int k) {
 // Measured at d = 768, F = 2048, us per launch (qkv / out / gate-up / down), one block of 256 x 256
 // per CU (what every size ran on before these shapes) -> the shape taken here:
 //   256 rows    50 / 37 / 43 / 87      12 / 6 / 12 / 11     S0
-//   731 rows    53 / 38 / 45 / 88      17 / 7 / 21 / 13     S0
+//   731 rows    53 / 38 / 45 / 88      17 / 7 / 21 / 13     S0 / S0 / S1 / S0
 //   2,300 rows  55 / 38 / 48 / 88      30 / 10 / 40 / 22    S2 / S0 / S3 / S0
 //   4,096 rows  57 / 41 / 54 / 90      50 / 16 / 51 / 31    S3 / S1 / S3 / S1
-//   8,192 rows  106 / 42 / 99 / 92     77 / 28 / 92 / 55    S1 / S2 / S3 / S2
+//   8,192 rows  106 / 42 / 99 / 92     77 / 28 / 92 / 55    S2 / S2 / S3 / S2
 //   16,669      157 / 50 / 227 / 103   126 / 45 / 185 / 90  S3
 // Past five rounds the power limit sets in, and the paced copies of the norm forms' S4 win: 701
 // against 729 us for the gate / up projection of 65,536 rows.
@@ -1051,6 +1051,24 @@ extern "C" int mdl_prefill_gemm_norm_qkv(
   p.slots = cache_slots; p.seq = seq; p.batch = batch; p.lead = lead;
   p.M = m; p.N = 3 * d; p.K = d;
   return launch_norm<E_QKV>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdl_prefill_gemm_shapes(int form) {
+  switch (form) {
+    case MDL_GEMM_NORM: return 5;
+    case MDL_GEMM_SPLIT: return 4;
+    case MDL_GEMM_NORM_F32W:
+    case MDL_GEMM_SPLIT_F32W: return 3;
+    default: return MDL_ERR_SHAPE;
+  }
+}
+
+extern "C" int mdl_prefill_gemm_pick(int form, int m, int n, int k) {
+  if (form < MDL_GEMM_NORM || form > MDL_GEMM_SPLIT_F32W || m <= 0 || n <= 0 || k <= 0 || k % 32)
+    return MDL_ERR_SHAPE;
+  const bool norm = form == MDL_GEMM_NORM || form == MDL_GEMM_NORM_F32W;
+  if (norm && k > kMaxNormK) return MDL_ERR_SHAPE;
+  return form < MDL_GEMM_NORM_F32W ? pick_shape(norm, m, n, k) : pick_shape_f32(norm, m, n, k);
 }
 
 extern "C" int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, float eps,

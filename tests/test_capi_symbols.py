@@ -118,6 +118,13 @@ def test_argument_errors_are_reported_before_any_launch():
                                           32, None) == -3
     assert L.mdl_prefill_gemm_norm_swiglu(fake, fake, 1e-5, 1, fake, None, None, fake, 3, 4, 16,
                                           32, None) == -3
+    assert [L.mdl_prefill_gemm_shapes(f) for f in range(-1, 5)] == [-3, 5, 4, 3, 3, -3]
+    for form in range(4):
+        for m in (1, 700, 5000, 40_000, 2 ** 31 - 1):
+            assert 0 <= L.mdl_prefill_gemm_pick(form, m, 2304, 768) < L.mdl_prefill_gemm_shapes(form)
+        assert L.mdl_prefill_gemm_pick(form, 4, 16, 48) == -3
+        assert (L.mdl_prefill_gemm_pick(form, 4, 16, 2080) == -3) == (form % 2 == 0)
+    assert L.mdl_prefill_gemm_pick(4, 4, 16, 32) == -3
     assert L.mdl_gemm_split_tiles() >= 1
     assert 1 <= L.mdl_gemm_split_pick(256, 2304, 768) <= L.mdl_gemm_split_tiles()
     # packed prefill: the per-row starts / offsets and the per-token rows / slots are required

@@ -323,9 +323,28 @@ def test_split_gemm_at_config2_size_against_hipblaslt():
     assert float((out[rows].double() - sub).abs().max() / sub.abs().max()) < 2e-6
 
 
-# rows at the tiles' edges, and where d = 768, F = 2048 products change their block shape: the norm
-# forms run small / mid / wide / large, the split forms likewise, over these row counts
+# rows at the tiles' edges, and where products of d = 768 change their block shape
 ROUTE_ROWS = [1, 63, 65, 257, 731, 1025, 2047, 3000, 4097, 6030, 8193]
+MANY_ROWS = 20_600       # the shape of the largest gate / up products, from 20,481 rows on
+MANY_QKV_ROWS = 36_400   # the same of qkv, from 36,353
+F32W_ROWS = [1, 17, 250, 641, 768, 769, 1025, 1500, 3000, 4097, 8193]   # K5 up to 768
+F32W_QKV_ROWS = [1, 448, 449, 640, 641, 1100, 4097, 12345]              # K5 up to 448
+
+
+@pytest.mark.parametrize("form,n,k,rows", [
+    ("NORM", 4096, 768, ROUTE_ROWS + [MANY_ROWS]), ("SPLIT", 768, 768, ROUTE_ROWS + [MANY_ROWS]),
+    ("NORM", 2304, 768, ROUTE_ROWS + [MANY_QKV_ROWS]),
+    ("NORM_F32W", 1408, 768, [m for m in F32W_ROWS if m > 768]),
+    ("SPLIT_F32W", 768, 768, [m for m in F32W_ROWS if m > 768]),
+    ("NORM_F32W", 576, 192, [m for m in F32W_QKV_ROWS if m > 448])])
+def test_row_lists_take_each_block_shape(form, n, k, rows):
+    """The row counts of the tests below run every block shape of a form, in its store, SwiGLU,
+    residual and qkv epilogues."""
+    from mdlarc_scale_amd import _lib
+
+    code = ["NORM", "SPLIT", "NORM_F32W", "SPLIT_F32W"].index(form)
+    picks = {_lib.lib().mdl_prefill_gemm_pick(code, m, n, k) for m in rows}
+    assert picks == set(range(_lib.lib().mdl_prefill_gemm_shapes(code)))
 
 
 @pytest.mark.parametrize("k", [768, 1952, 1984])   # odd multiples of 32, past gamma's 1,920
@@ -333,7 +352,7 @@ def test_rows_do_not_depend_on_the_row_count(k):
     """Every block shape sums in the same order, so the first m rows of a product are the same bits
     whatever m is: each form at row counts that take each shape, against the rows of one large
     product (which the tests above pin to fp64)."""
-    f, total = 2048, 20_000
+    f, total = 2048, MANY_ROWS
     g = torch.Generator(DEV).manual_seed(k)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
     wgu = K().tile_matrix((0.05 * rnd(2 * f, k)).to(torch.bfloat16))
@@ -360,7 +379,7 @@ def test_rows_do_not_depend_on_the_row_count(k):
             assert torch.equal(got, want[:m]), f"{name} at {m} rows"
 
 
-@pytest.mark.parametrize("m", ROUTE_ROWS)
+@pytest.mark.parametrize("m", ROUTE_ROWS + [MANY_QKV_ROWS])
 def test_norm_qkv_at_each_block_shape(m):
     """The qkv epilogue of each shape against the E_STORE form and K2, bit for bit."""
     H, d = 12, 768
@@ -422,7 +441,7 @@ def test_fp32_weight_forms(k):
     ref = torch.nn.functional.silu(gate) * blocks[:, :, 1].reshape(total, f)
     h = d(whole[2])
     assert rel(h[:, :f] + h[:, f:], ref) < 2e-5          # as the bf16 form's: the split of h
-    for m in (1, 17, 250, 641, 768, 769, 1025, 1500, 3000, 4097, 8193):
+    for m in F32W_ROWS:
         for name, got, want in zip(("store", "rstd", "swiglu", "residual"), forms(m), whole):
             assert torch.equal(got, want[:m]), f"{name} at {m} rows"
 
@@ -438,7 +457,7 @@ def _f32w_qkv_inputs(m, H, seed):
 
 
 @pytest.mark.parametrize("H", [3, 4, 12])
-@pytest.mark.parametrize("m", [1, 448, 449, 640, 641, 1100, 4097, 12345])
+@pytest.mark.parametrize("m", F32W_QKV_ROWS)
 @pytest.mark.parametrize("packed", [False, True])
 def test_norm_qkv_of_fp32_weights(m, H, packed):
     """The fp32 qkv epilogue against the E_STORE form and K2, bit for bit; a packed list with

@@ -493,7 +493,6 @@ __global__ __launch_bounds__(512, 6) void attn_lead_kernel(
   // lane reads back what it wrote.
   float* pw = ps + 32 * wave * (wave + 1);   // the wave's 64-float blocks, one per 8 keys
   float* aw = as + 32 * wave * (wave + 1);
-#pragma unroll 2
   for (int t = 0; t <= wave; ++t) {
     float s[kLeadLanes];
 #pragma unroll

@@ -905,11 +905,18 @@ int launch_f32w(const Args& p, hipStream_t st) {
 }
 
 // fp32 weights: up to this many rows the projections run on K5, whose waves split K and need no
-// ring to fill, with the same bits; qkv up to the second, since past it K5 and K2 are slower than the
-// one launch.  Out, gate / up and down together, us on K5 / on K6: d = 768 at 384 rows 37 / 53, 768
-// 53 / 60, 896 60 / 63, 1,536 114 / 80; d = 1,280 at 768 rows 104 / 116, 896 150 / 120.  qkv: d = 768
-// at 384 rows 17.3 / 19.0, 512 24.5 / 22.4; d = 1,280 at 256 24.9 / 28.9, 384 35.0 / 32.2.
-constexpr int kK5Rows = 768, kK5RowsQkv = MDL_F32W_QKV_ROWS;   // 448
+// ring to fill, with the same bits; qkv up to the last, since past it K5 and K2 are slower than the
+// one launch.  Out, gate / up and down, us on K5 / on K6: d = 768 at 384 rows 37 / 53, 768 53 / 60,
+// 896 60 / 63, 1,536 114 / 80; d = 1,280 at 768 rows 104 / 116, 896 150 / 120.  At d = 256 a k-step's
+// share of the fold is larger: gate / up at 1,024 rows 10.1 / 10.6, 1,536 14.1 / 13.1; out and down at
+// 1,536 9.9 / 13.9, 2,304 14.0 / 14.6.  qkv: d = 768 at 384 rows 17.3 / 19.0, 512 24.5 / 22.4;
+// d = 1,280 at 256 24.9 / 28.9, 384 35.0 / 32.2.
+constexpr int kK5Rows = 768, kK5RowsNarrow = 1024, kK5RowsNarrowResidual = 2048;
+constexpr int kK5RowsQkv = MDL_F32W_QKV_ROWS;   // 448
+constexpr int kNarrow = 512;                    // channels
+
+bool on_k5_norm(int m, int k) { return m <= (k < kNarrow ? kK5RowsNarrow : kK5Rows); }
+bool on_k5_residual(int m, int n) { return m <= (n < kNarrow ? kK5RowsNarrowResidual : kK5Rows); }
 
 // the split forms by A layout and parts: row-major activations, and the forms with the hi part
 // alone, are not on the prompt path and run on the large shape
@@ -1082,7 +1089,7 @@ extern "C" int mdl_prefill_gemm_norm_f32w(const float* x, const float* gamma, fl
   if (!aligned16(w_lo) || !aligned16(x) || !aligned16(gamma) || !aligned16(out) || ldo % 4 != 0)
     return MDL_ERR_ALIGN;
   if (m == 0) return MDL_OK;
-  if (m <= kK5Rows)
+  if (on_k5_norm(m, k))
     return mdl_gemm_norm(x, gamma, eps, w, w_lo, out, ldo, rstd_out, m, n, k, 0, stream);
   Args p{};
   p.x = x; p.gamma = gamma; p.eps = eps; p.w = w; p.wl = w_lo; p.out = out; p.ldo = ldo;
@@ -1152,7 +1159,7 @@ extern "C" int mdl_prefill_gemm_norm_swiglu_f32w(const float* x, const float* ga
       (bias_gate && !aligned16(bias_gate)) || (bias_up && !aligned16(bias_up)))
     return MDL_ERR_ALIGN;
   if (m == 0) return MDL_OK;
-  if (m <= kK5Rows)
+  if (on_k5_norm(m, k))
     return mdl_gemm_norm_swiglu(x, gamma, eps, w_gu, w_gu_lo, bias_gate, bias_up, h_out, m, d_ff,
                                 k, 0, stream);
   Args p{};
@@ -1172,7 +1179,7 @@ extern "C" int mdl_prefill_gemm_split_residual_f32w(const uint16_t* a, const uin
   if (n % 32 != 0) return MDL_ERR_SHAPE;   // x in the fp32 tile layout: whole 32-column blocks
   if (!aligned16(w_lo) || !aligned16(x) || (bias && !aligned16(bias))) return MDL_ERR_ALIGN;
   if (m == 0) return MDL_OK;
-  if (m <= kK5Rows) return mdl_gemm_split_residual(a, w, w_lo, x, bias, m, n, k, 0, stream);
+  if (on_k5_residual(m, n)) return mdl_gemm_split_residual(a, w, w_lo, x, bias, m, n, k, 0, stream);
   Args p{};
   p.a = a; p.w = w; p.wl = w_lo; p.x_res = x; p.bias_a = bias; p.M = m; p.N = n; p.K = k;
   return launch_f32w<E_RESIDUAL>(p, static_cast<hipStream_t>(stream));

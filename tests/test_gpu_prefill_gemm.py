@@ -327,7 +327,7 @@ def test_split_gemm_at_config2_size_against_hipblaslt():
 ROUTE_ROWS = [1, 63, 65, 257, 731, 1025, 2047, 3000, 4097, 6030, 8193]
 MANY_ROWS = 20_600       # the shape of the largest gate / up products, from 20,481 rows on
 MANY_QKV_ROWS = 36_400   # the same of qkv, from 36,353
-F32W_ROWS = [1, 17, 250, 641, 768, 769, 1025, 1500, 3000, 4097, 8193]   # K5 up to 768
+F32W_ROWS = [1, 17, 250, 641, 768, 769, 1025, 1500, 2048, 2049, 3000, 4097, 8193]   # K5 up to 768
 F32W_QKV_ROWS = [1, 448, 449, 640, 641, 1100, 4097, 12345]              # K5 up to 448
 
 
@@ -403,12 +403,14 @@ def test_norm_qkv_at_each_block_shape(m):
         assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("k", [96, 224, 256, 768, 1952, 2048])   # under 8 k-steps, 8, and more
-def test_fp32_weight_forms(k):
+# under 8 k-steps, 8, and more; narrow outputs and inputs stay on K5 for up to 2,048 and 1,024 rows
+@pytest.mark.parametrize("k,n", [(96, 768), (224, 768), (256, 768), (704, 256), (768, 768),
+                                 (1952, 768), (2048, 768)])
+def test_fp32_weight_forms(k, n):
     """The fp32-weight forms: a large product against fp64 of the products they form, a_hi w +
-    a_lo w + a_hi w_lo (fp32 sums: 2e-6, as above), and every row count, on K5 (up to 768 rows)
+    a_lo w + a_hi w_lo (fp32 sums: 2e-6, as above), and every row count, on K5 (a few rows)
     and K6, at the edges of the tiles, the same bits as those rows of the large product."""
-    f, n, total = 704, 768, 20_000
+    f, total = 704, 20_000
     g = torch.Generator(DEV).manual_seed(k)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
     wg, wo = 0.05 * rnd(2 * f, k), 0.05 * rnd(n, k)
